@@ -4,13 +4,12 @@
 // bk_n3_v0), the Partial forms axhelm/kernel/VOLTA/axhelm.okl:158-290 and
 // the host oracle axhelm/axhelmReference.cpp:19-101.
 //
-// Mapping to gfx950: one workgroup per element with Nq*Nq lanes (one wave64
-// at N=7); lane (i,j) owns the node column k = 0..Nq-1 in registers.  Each
-// k-slab of q goes through LDS for the r and s derivatives; the t derivative
-// and the t-part of the transpose stay in the register column.  ggeo is
-// streamed plane by plane, coalesced (64 consecutive doubles per load per
-// factor at N=7).  The four D vectors a lane needs (row i, row j, column i,
-// column j) sit in registers; D[k][:] is read from LDS as a broadcast.
+// Mapping to gfx950: Nq*Nq lanes per element (one wave64 at N=7, several
+// elements per workgroup at small orders).  A lane owns a node column, an r
+// line and an s line of the element in turn; lines are exchanged through LDS,
+// the t direction stays in registers, and D's rows are scalar operands
+// (axhelm_lines).  ggeo is streamed plane by plane, coalesced (64 consecutive
+// doubles per load per factor at N=7).
 //
 // FP64 arithmetic order (identical to the CPU oracle, bit-exact):
 //   qr = fma chain over m of D[i][m] q(m,j,k), qs and qt alike
@@ -19,94 +18,6 @@
 #include "nbx_axhelm_impl.h"
 
 namespace nbx {
-
-// FP64 BK one-field operator at N = 7 with each element split over two
-// waves: wave w owns the slabs k = 4w .. 4w+3.  The element's q sits in LDS
-// (4 KB), so the t derivative reads the column from there and no wave keeps
-// a q column in registers; each wave walks four slabs (half the chain of
-// dependent load rounds), and eight waves per SIMD (64 VGPRs) keep a 16^3
-// mesh (8192 waves) in one round.  After the slab loop, Gt of every slab
-// replaces q in LDS and each output node takes the t transpose as the
-// one-wave column does, an fma chain over the slabs in increasing order:
-// the arithmetic is the one-wave kernel's, bit for bit.
-__global__ __launch_bounds__(128, 8) void k_axhelm_bk8_split(const int32_t Nelements,
-                                                             const double* ggeo,
-                                                             const double* __restrict__ D,
-                                                             const double* __restrict__ q, double* __restrict__ Aq,
-                                                             const int* __restrict__ skip)
-{
-  constexpr int NQ = 8, NQ2 = 64, NP = 512, H = 4;
-  if (skip && *skip) return;
-  __shared__ double s_D[NQ2], s_qt[NP], s_Gr[2][2][NQ2], s_Gs[2][2][NQ2];
-  // w is uniform in each wave: D's row and column k come from scalar loads
-  const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(threadIdx.y), i = t & 7, j = t >> 3;
-  const int64_t e = blockIdx.x;
-  if (w == 0) s_D[t] = D[t];
-  // uniform element bases, one 32-bit lane offset: the loads take a scalar
-  // base and a shared lane register rather than a 64-bit address each
-  const double* qe = q + e * NP;
-  const int o = H * w * NQ2 + t;
-#pragma unroll
-  for (int kk = 0; kk < H; ++kk) s_qt[o + kk * NQ2] = ldnt(&qe[o + kk * NQ2]);
-  const double* g = ggeo + e * (int64_t)(kNggeo * NP);
-  const double *g00 = g + kG00 * NP, *g01 = g + kG01 * NP, *g02 = g + kG02 * NP;
-  const double *g11 = g + kG11 * NP, *g12 = g + kG12 * NP, *g22 = g + kG22 * NP;
-  // the first slab's geometric factors are in flight across the barrier and
-  // its derivatives (few registers are live here; later slabs load theirs
-  // after the derivatives, inside the 64-register budget)
-  double G0[6];
-  G0[0] = ldnt(&g00[o]);
-  G0[1] = ldnt(&g01[o]);
-  G0[2] = ldnt(&g02[o]);
-  G0[3] = ldnt(&g11[o]);
-  G0[4] = ldnt(&g12[o]);
-  G0[5] = ldnt(&g22[o]);
-  __syncthreads();
-  double Gt[H], ars[H];
-#pragma unroll
-  for (int kk = 0; kk < H; ++kk) {
-    const int k = H * w + kk;
-    double qr = 0.0, qs = 0.0, qt = 0.0;
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) {
-      qr = __builtin_fma(s_D[i * NQ + m], s_qt[k * NQ2 + j * NQ + m], qr);
-      qs = __builtin_fma(s_D[j * NQ + m], s_qt[k * NQ2 + m * NQ + i], qs);
-      qt = __builtin_fma(D[k * NQ + m], s_qt[m * NQ2 + t], qt);
-      if (m % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // bounds the reads the scheduler batches
-    }
-    const int n = o + kk * NQ2;
-    const double G00 = kk == 0 ? G0[0] : ldnt(&g00[n]), G01 = kk == 0 ? G0[1] : ldnt(&g01[n]);
-    const double G02 = kk == 0 ? G0[2] : ldnt(&g02[n]), G11 = kk == 0 ? G0[3] : ldnt(&g11[n]);
-    const double G12 = kk == 0 ? G0[4] : ldnt(&g12[n]), G22 = kk == 0 ? G0[5] : ldnt(&g22[n]);
-    double* sr = s_Gr[w][kk & 1];
-    double* ss = s_Gs[w][kk & 1];
-    sr[t] = __builtin_fma(G02, qt, __builtin_fma(G01, qs, G00 * qr));
-    ss[t] = __builtin_fma(G12, qt, __builtin_fma(G11, qs, G01 * qr));
-    Gt[kk] = __builtin_fma(G22, qt, __builtin_fma(G12, qs, G02 * qr));
-    __syncthreads();
-    double ar = 0.0, as = 0.0;
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) {
-      ar = __builtin_fma(s_D[m * NQ + i], sr[j * NQ + m], ar);
-      as = __builtin_fma(s_D[m * NQ + j], ss[m * NQ + i], as);
-      if (m % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-    }
-    ars[kk] = ar + as;
-  }
-  // every q read of both waves precedes their last barrier above
-#pragma unroll
-  for (int kk = 0; kk < H; ++kk) s_qt[(H * w + kk) * NQ2 + t] = Gt[kk];
-  __syncthreads();
-  double* Ae = Aq + e * NP;
-#pragma unroll
-  for (int kk = 0; kk < H; ++kk) {
-    const int k = H * w + kk;
-    double at = 0.0;
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) at = __builtin_fma(D[m * NQ + k], s_qt[m * NQ2 + t], at);
-    stnt(ars[kk] + at, &Ae[o + kk * NQ2]);
-  }
-}
 
 int axhelm_dispatch_f64(int N, int Nf, int bk, bool partial, int32_t Nelements, int32_t offset,
                         const int32_t* elementList, const void* ggeo, const void* D, const void* lambda,

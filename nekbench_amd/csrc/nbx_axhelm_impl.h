@@ -47,308 +47,616 @@ __device__ __forceinline__ T ldgc(const G* p)
   }
 }
 
-// Elements per workgroup: one element (Nq*Nq lanes) from Nq = 8 up; small
-// orders pack several elements (threadIdx.y = slot) so that a workgroup
-// holds at least 128 lanes.
-template <int NQ>
-struct Epb {
-  static constexpr int value = NQ * NQ >= 64 ? 1 : 128 / (NQ * NQ);
-};
-
-// Per-workgroup state of the operator: LDS slabs and the lane's D vectors.
+// LDS places of node (i, j, k).  r array: i + j RS + k PS with RS odd, so a
+// lane per r line (address t RS) meets no bank conflict; s array: i + j NQ + k
+// QS with QS = NQ modulo the slots one LDS cycle serves (128 bytes), so lanes
+// over nodes and lanes over s lines both read consecutive slots.
 template <typename T, int NQ>
-struct AxLane {
-  T Di[NQ], Dj[NQ], DTi[NQ], DTj[NQ];
-  int t, i, j;
-  __device__ __forceinline__ void init(const T* s_D)
+struct LineLayout {
+  static constexpr int RS = NQ | 1, PS = NQ * RS, SZ = NQ * PS;
+  static constexpr int M = 128 / (int)sizeof(T);
+  static constexpr int QS = NQ * NQ + ((NQ - NQ * NQ) % M + M) % M, SS = NQ * QS;
+};
+
+// Row i of D through the constant address space: uniform addresses become
+// scalar loads and the row's values scalar operands of the products.  The
+// pointer is made opaque at every row, or the compiler keeps all of D in
+// scalar registers from the first use to the last and spills them.
+template <typename T>
+using ConstPtr = const T __attribute__((address_space(4)))*;
+template <typename T, int NQ>
+struct DRow {
+  T d[NQ];
+  __device__ __forceinline__ void load(ConstPtr<T> D, int row)
   {
-    t = threadIdx.x;
-    i = t % NQ;
-    j = t / NQ;
+    asm volatile("" : "+s"(D));
 #pragma unroll
-    for (int m = 0; m < NQ; ++m) {
-      Di[m] = s_D[i * NQ + m];
-      Dj[m] = s_D[j * NQ + m];
-      DTi[m] = s_D[m * NQ + i];
-      DTj[m] = s_D[m * NQ + j];
-    }
+    for (int m = 0; m < NQ; ++m) d[m] = D[row * NQ + m];
   }
 };
 
-// One field of one element: out[k] = (A q)(i,j,k) for the lane's column rq.
-// g, l0, l1 point at the lane's node (k = 0) of ggeo, lambda0, lambda1.
-// DL: read the lane's D vectors from LDS instead of registers (frees 4*NQ
-// registers; used where that buys a fourth wave per SIMD)
-// NTG: nontemporal loads of the geometric factors and lambda (false when
-// other thread groups of the workgroup read the same values)
-// EARLY: issue each slab's geometric-factor loads before the slab's
-// barriers, so they are in flight while the slab goes through LDS
-template <typename T, int NQ, bool BK, typename G = T, bool DL = false, bool NTG = true, bool EARLY = false>
-__device__ __forceinline__ void axhelm_column(const AxLane<T, NQ>& L, const T (&rq)[NQ], T (&out)[NQ],
-                                              const T* __restrict__ s_D, T* s_q, T* s_Gr, T* s_Gs,
-                                              const G* __restrict__ g, const G* __restrict__ l0,
-                                              const G* __restrict__ l1)
-{
-  constexpr int NQ2 = NQ * NQ;
-  constexpr int NP = NQ2 * NQ;
-  T rAt[NQ], rArs[NQ];
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) rAt[k] = T(0);
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
+// The geometric factors and lambda0 of the lane's column, one slab at a time,
+// fetched AHEAD slabs before their use.  NT: nontemporal loads (single use);
+// cached ones where other workgroups of the XCD read the same element.
+template <typename T, int NQ, bool BK, typename G, bool NT, int AHEAD, typename IDX>
+struct GeoStream {
+  static constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ;
+  const G *g, *l0, *l1;  // element bases (uniform in the workgroup)
+  IDX go, lo;            // the lane's node (k = 0) past them
+  T Gk[AHEAD][7];
+  __device__ __forceinline__ void fetch(int k)
+  {
     const int n = k * NQ2;
-    T Gk[6];
-    auto load_g = [&]() {
-      Gk[0] = ldgc<T, G, NTG>(&g[kG00 * NP + n]);
-      Gk[1] = ldgc<T, G, NTG>(&g[kG01 * NP + n]);
-      Gk[2] = ldgc<T, G, NTG>(&g[kG02 * NP + n]);
-      Gk[3] = ldgc<T, G, NTG>(&g[kG11 * NP + n]);
-      Gk[4] = ldgc<T, G, NTG>(&g[kG12 * NP + n]);
-      Gk[5] = ldgc<T, G, NTG>(&g[kG22 * NP + n]);
-    };
-    if (EARLY) load_g();
+    T(&u)[7] = Gk[k % AHEAD];
+    u[0] = ldgc<T, G, NT>(&(g + kG00 * NP)[go + n]);
+    u[1] = ldgc<T, G, NT>(&(g + kG01 * NP)[go + n]);
+    u[2] = ldgc<T, G, NT>(&(g + kG02 * NP)[go + n]);
+    u[3] = ldgc<T, G, NT>(&(g + kG11 * NP)[go + n]);
+    u[4] = ldgc<T, G, NT>(&(g + kG12 * NP)[go + n]);
+    u[5] = ldgc<T, G, NT>(&(g + kG22 * NP)[go + n]);
+    if (!BK) u[6] = ldgc<T, G, NT>(&l0[lo + n]);
+  }
+  __device__ __forceinline__ void begin()
+  {
+#pragma unroll
+    for (int k = 0; k < AHEAD && k < NQ; ++k) fetch(k);
+  }
+  __device__ __forceinline__ void next(int k)
+  {
+    if (k + AHEAD < NQ) fetch(k + AHEAD);
+  }
+  __device__ __forceinline__ T f(int k, int c) const { return Gk[k % AHEAD][c]; }
+  __device__ __forceinline__ T lam(int k) const { return Gk[k % AHEAD][6]; }
+  __device__ __forceinline__ T mass(int k) const
+  {
+    const int n = k * NQ2;
+    return ldgc<T, G, NT>(&(g + kGWJ * NP)[go + n]) * ldgc<T, G, NT>(&l1[lo + n]);
+  }
+};
+
+// The same for three fields of one element, read once: the factors of every
+// slab stay in registers, lambda0 and GWJ lambda1 in LDS (each lane its own
+// column, so without a barrier).
+template <typename T, int NQ, bool BK, typename G, typename IDX>
+struct GeoKept {
+  static constexpr int NQ2 = NQ * NQ;
+  GeoStream<T, NQ, true, G, true, NQ, IDX> s;
+  T *l, *w;
+  __device__ __forceinline__ void load()
+  {
+    s.begin();
+    if constexpr (!BK) {
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) {
+        l[k * NQ2] = ldg<T, G>(&s.l0[s.lo + k * NQ2]);
+        w[k * NQ2] = s.mass(k);
+      }
+    }
+  }
+  __device__ __forceinline__ void begin() {}
+  __device__ __forceinline__ void next(int) {}
+  __device__ __forceinline__ T f(int k, int c) const { return s.Gk[k][c]; }
+  __device__ __forceinline__ T lam(int k) const { return l[k * NQ2]; }
+  __device__ __forceinline__ T mass(int k) const { return w[k * NQ2]; }
+};
+
+// One field of one element in line form: a lane is the owner of a node column
+// (i, j) = (t % NQ, t / NQ), of an r line and of an s line in turn.  A
+// contraction reads its line once, forms all NQ outputs with D's rows as
+// scalar operands and writes them back in place, so every node moves through
+// LDS 15 times in all; with a lane per output, each derivative read NQ values
+// (4 NQ reads a node, and D), and from N = 4 up LDS and registers, not HBM,
+// were the bound.  12e6 nodes, one field, before -> now: FP64 BK N = 5
+// 335 -> 138 us, N = 7 142 -> 125, N = 12 208 -> 155, N = 15 303 -> 155;
+// non-BK N = 12 626 -> 204; FP32 non-BK N = 6 154 -> 101; three fields FP64
+// non-BK N = 7 501 -> 266, N = 9 723 -> 377, N = 12 1884 -> 389.  One field
+// moves 5.0 to 6.0 TB/s now, HBM-bound.  Each output is the fma chain over m
+// (or k) in increasing order, as the oracle has it.
+// rq: q of the lane's column on entry; after_forward() may replace it (the
+// next field's); q_again(mq) gives q once more for the mass term, before the
+// transposed contractions or, with LATE, after them.
+template <typename T, int NQ, bool BK, bool LATE = false, typename GEO, typename F1, typename F2>
+__device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[NQ], ConstPtr<T> D, T* s_r, T* s_s,
+                                             GEO& geo, F1&& after_forward, F2&& q_again)
+{
+  using LL = LineLayout<T, NQ>;
+  constexpr int RS = LL::RS, PS = LL::PS, QS = LL::QS;
+  const int a = t % NQ, b = t / NQ;
+  T* const nr = s_r + b * RS + a;  // node (a, b, k) at + k PS
+  T* const ns = s_s + t;           // the same node, at + k QS
+  T* const lr = s_r + t * RS;      // r line (j, k) = (a, b)
+  T* const ls = s_s + b * QS + a;  // s line (i, k) = (a, b), node j at + j NQ
+  const T* const lq = s_r + b * PS + a;  // the same line of q
+  T v[NQ];
+  {
+    T ql[NQ], qm[NQ];
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) nr[k * PS] = rq[k];
     __syncthreads();
-    s_q[L.t] = rq[k];
-    __syncthreads();
-    T qr = T(0), qs = T(0), qt = T(0);
 #pragma unroll
     for (int m = 0; m < NQ; ++m) {
-      qr = fmaT(DL ? s_D[L.i * NQ + m] : L.Di[m], s_q[L.j * NQ + m], qr);
-      qs = fmaT(DL ? s_D[L.j * NQ + m] : L.Dj[m], s_q[m * NQ + L.i], qs);
-      qt = fmaT(s_D[k * NQ + m], rq[m], qt);
+      ql[m] = lr[m];
+      qm[m] = lq[m * RS];
     }
-    if (!EARLY) load_g();
-    const T G00 = Gk[0], G01 = Gk[1], G02 = Gk[2], G11 = Gk[3], G12 = Gk[4], G22 = Gk[5];
-    T Gr = fmaT(G02, qt, fmaT(G01, qs, G00 * qr));
-    T Gs = fmaT(G12, qt, fmaT(G11, qs, G01 * qr));
-    T Gt = fmaT(G22, qt, fmaT(G12, qs, G02 * qr));
-    if (!BK) {
-      const T lam0 = ldgc<T, G, NTG>(&l0[n]);
-      Gr = lam0 * Gr;
-      Gs = lam0 * Gs;
-      Gt = lam0 * Gt;
-    }
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) rAt[m] = fmaT(s_D[k * NQ + m], Gt, rAt[m]);
-    s_Gr[L.t] = Gr;
-    s_Gs[L.t] = Gs;
     __syncthreads();
-    T ar = T(0), as = T(0);
+    DRow<T, NQ> R, Rn;
+    R.load(D, 0);
+    T qr, qs;
 #pragma unroll
-    for (int m = 0; m < NQ; ++m) {
-      ar = fmaT(DL ? s_D[m * NQ + L.i] : L.DTi[m], s_Gr[L.j * NQ + m], ar);
-      as = fmaT(DL ? s_D[m * NQ + L.j] : L.DTj[m], s_Gs[m * NQ + L.i], as);
+    for (int i = 0; i < NQ; ++i) {
+      // the first products wait for row i; then the previous row's results
+      // and the next row's loads are issued, in flight during the rest
+      T pr = qr, ps = qs;
+      qr = fmaT(R.d[0], ql[0], T(0));
+      qs = fmaT(R.d[0], qm[0], T(0));
+      T qt = fmaT(R.d[0], rq[0], T(0));
+      __builtin_amdgcn_sched_barrier(0);
+      if (i > 0) {
+        lr[i - 1] = pr;
+        ls[(i - 1) * NQ] = ps;
+      }
+      if (i + 1 < NQ) Rn.load(D, i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 1; m < NQ; ++m) {
+        qr = fmaT(R.d[m], ql[m], qr);
+        qs = fmaT(R.d[m], qm[m], qs);
+        qt = fmaT(R.d[m], rq[m], qt);
+      }
+      v[i] = qt;
+      R = Rn;
     }
-    rArs[k] = ar + as;
+    lr[NQ - 1] = qr;
+    ls[(NQ - 1) * NQ] = qs;
   }
 #pragma unroll
+  for (int k = 0; k < NQ; ++k) out[k] = T(0);
+  after_forward();
+  __syncthreads();
+  {
+    geo.begin();
+    DRow<T, NQ> R, Rn;
+    R.load(D, 0);
+    T qr = nr[0], qs = ns[0], qrn, qsn;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const T G01 = geo.f(k, 1), G02 = geo.f(k, 2), G12 = geo.f(k, 4), qt = v[k];
+      T Gr = fmaT(G02, qt, fmaT(G01, qs, geo.f(k, 0) * qr));
+      T Gs = fmaT(G12, qt, fmaT(geo.f(k, 3), qs, G01 * qr));
+      T Gt = fmaT(geo.f(k, 5), qt, fmaT(G12, qs, G02 * qr));
+      if (!BK) {
+        const T lam0 = geo.lam(k);
+        Gr = lam0 * Gr;
+        Gs = lam0 * Gs;
+        Gt = lam0 * Gt;
+      }
+      out[0] = fmaT(R.d[0], Gt, out[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      nr[k * PS] = Gr;
+      ns[k * QS] = Gs;
+      if (k + 1 < NQ) {
+        Rn.load(D, k + 1);
+        qrn = nr[(k + 1) * PS];
+        qsn = ns[(k + 1) * QS];
+      }
+      geo.next(k);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 1; m < NQ; ++m) out[m] = fmaT(R.d[m], Gt, out[m]);
+      R = Rn;
+      qr = qrn;
+      qs = qsn;
+    }
+  }
+  __syncthreads();
+  T mq[NQ];
+  if (!LATE) q_again(mq);
+  {
+    T ar[NQ], as[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) ar[i] = as[i] = T(0);
+    DRow<T, NQ> R, Rn;
+    R.load(D, 0);
+    T gr = lr[0], gs = ls[0], grn, gsn;
+#pragma unroll
+    for (int m = 0; m < NQ; ++m) {
+      ar[0] = fmaT(R.d[0], gr, ar[0]);
+      as[0] = fmaT(R.d[0], gs, as[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (m + 1 < NQ) {
+        Rn.load(D, m + 1);
+        grn = lr[m + 1];
+        gsn = ls[(m + 1) * NQ];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 1; i < NQ; ++i) {
+        ar[i] = fmaT(R.d[i], gr, ar[i]);
+        as[i] = fmaT(R.d[i], gs, as[i]);
+      }
+      R = Rn;
+      gr = grn;
+      gs = gsn;
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      lr[i] = ar[i];
+      ls[i * NQ] = as[i];
+    }
+  }
+  __syncthreads();
+  if (LATE) q_again(mq);
+#pragma unroll
   for (int k = 0; k < NQ; ++k) {
-    T res = rArs[k] + rAt[k];
+    T res = (nr[k * PS] + ns[k * QS]) + out[k];
     if (!BK) {
-      const int n = k * NQ2;
-      res = fmaT(ldgc<T, G, NTG>(&g[kGWJ * NP + n]) * ldgc<T, G, NTG>(&l1[n]), rq[k], res);
+      res = fmaT(geo.mass(k), mq[k], res);
     }
     out[k] = res;
   }
 }
 
-// the one-field BK kernel at N = 7 reads D from LDS and fits four waves per
-// SIMD (128 VGPRs): 4096 elements, the 16^3 mesh, fill the chip in one round
-template <int NQ, int NF, bool BK>
-struct AxDL {
-  static constexpr bool value = NQ == 8 && NF == 1 && BK;
+
+// ---- launch shapes ---------------------------------------------------------
+// Elements per workgroup (threadIdx.y = slot): enough to fill two to four
+// waves with few idle lanes, no more (a workgroup's waves wait for each other
+// at five barriers; N = 1 with 64 instead of 32 elements cost 8 % at 37500).
+// Slabs of factors in flight: four; two where FP64 would drop below three
+// waves per SIMD (N = 11 non-BK, 12e6 nodes: 195 against 219 us); all eight at
+// N = 7 BK (129 registers; 32768 elements 177 against 179 us).  N = 12 non-BK
+// is held to the 168 registers of three waves (204 against 213 us); at higher
+// orders that spills.
+template <typename T, int NQ, bool BK>
+struct AxShape {
+  static constexpr bool f64 = sizeof(T) == 8;
+  static constexpr int epb = NQ == 2 ? 32 : NQ == 3 ? 14 : NQ == 4 ? 8 : NQ == 5 ? 5 : NQ == 6 ? 3 : 1;
+  static constexpr int ahead = f64 && (NQ >= 12 || (NQ == 9 && !BK)) ? 2 : f64 && NQ == 8 && BK ? 8 : 4;
+  static constexpr int waves = f64 && NQ == 13 && !BK ? 3 : 1;
+};
+// Three fields: the element's factors kept in registers for all of them
+// (k_axhelm_kept) against one workgroup per field (k_axhelm), whose second
+// and third read of the factors come from L2 at about 9 TB/s at most.  12e6
+// nodes, kept against per field: FP64 N = 7 207 / 242 us (BK) and 266 / 315
+// (non-BK), N = 9 BK 287 / 300, FP32 N = 7 113 / 123 and N = 5 124 / 155; the
+// FP64 non-BK form at N = 9 would spill and is per field (377 / 442).  Three
+// times the workgroups are better while the chip is not full: 1e6 nodes, FP32
+// N = 7 14.3 / 11.2 us and FP64 N = 8 non-BK 45.8 / 40.4; FP64 gains from the
+// kept factors up to N = 7 at every size (21.8 / 25.2).
+template <typename T, int NQ, bool BK>
+struct AxKept {
+  static constexpr bool f64 = sizeof(T) == 8;
+  static constexpr bool value = f64 ? NQ <= 9 || (NQ == 10 && BK) : NQ <= 8;
+  static constexpr int epb = NQ == 2 ? 32 : NQ == 3 ? 14 : NQ == 4 ? 8 : NQ == 5 ? 5 : NQ == 6 ? 3 : 1;
+  static constexpr int waves = f64 && NQ >= 7 ? 2 : 1;
+  static bool when(int64_t Nelements)
+  {
+    const bool full = Nelements * (NQ * NQ) >= 64 * 8192;  // eight waves per SIMD
+    return f64 ? NQ <= 8 || BK || full : NQ >= 3 && full;
+  }
 };
 
-// Thread groups of NQ*NQ lanes per workgroup: Epb elements at small orders;
-// for the three-field Helmholtz (non-BK) operator with 8 <= Nq <= 12 and
-// FP64 or FP32 geometry, one group per field of one element, reading the
-// shared geometric factors and lambda with cached loads; each field's
-// arithmetic is the one-field column's.  Measured on 32^3 N = 7: 0.805 ->
-// 0.695 ms; the BK form and bf16 geometry are faster with the field loop and
-// keep it.
-template <int NQ, int NF, bool BK, typename G = double>
-struct AxGroups {
-  static constexpr bool fields = NF == 3 && !BK && Epb<NQ>::value == 1 && NQ <= 12 && sizeof(G) != 2;
-  static constexpr int value = fields ? NF : Epb<NQ>::value;
+// Three-field PCG form: one thread group per field of an element against the
+// fields in turn.  Its lane sums run over the fields, so the fields of an
+// element stay in one workgroup.  Groups are faster while the chip is not
+// full, and where the fields in turn leave one wave per SIMD (FP64 non-BK, us,
+// groups / in turn: N = 7 at 1e5 nodes 7.8 / 11.0, at 8e6 288 / 236; N = 9 at
+// 1e5 12.8 / 18.7, at 8e6 433 / 389; N = 11 at 8e6 399 / 752).  The line in
+// lanes (Nq^2 per element) lies between the measured sizes on each side.
+template <typename T, int NQ, bool BK, typename G>
+struct AxFieldGroups {
+  static constexpr bool fits = NQ >= 4 && 3 * (LineLayout<T, NQ>::SZ + LineLayout<T, NQ>::SS) * sizeof(T) < 150000;
+  static bool when(int64_t Nelements)
+  {
+    const int64_t lanes = Nelements * (NQ * NQ);
+    if (sizeof(T) == 8) return NQ == 9 || NQ >= 12 || (NQ == 11 && !BK) || lanes < 64 * (NQ == 11 ? 4096 : 1024);
+    if (sizeof(G) == 2 && (NQ == 10 || NQ == 11)) return lanes < 64 * 2048;
+    return NQ >= 9 || lanes < 64 * 16384;
+  }
 };
 
-// The FP64 field-group kernels read D from LDS as well (4 Nq fewer doubles
-// in registers) and keep three waves per SIMD up to Nq = 10 (168 VGPRs; left
-// alone they take 256 and run two); the one-field BK kernel at N = 7 keeps
-// four (128 VGPRs).  The FP32-arithmetic kernels keep D in registers: their
-// vectors take half the registers, and reading D from LDS made LDS the bound
-// (one-field BK at N = 7 on 32^3: bf16 geometry 80 -> 65 us, FP32 89 -> 84 us
-// with D in registers, the same bits).
-template <typename T, int NQ, int NF, bool BK>
-struct AxUseDL {
-  static constexpr bool value = sizeof(T) == 8 && (AxDL<NQ, NF, BK>::value || AxGroups<NQ, NF, BK>::fields);
-};
-// Early geometric-factor loads (axhelm_column's EARLY), measured on 32^3,
-// N = 7, one field: the FP64 BK PCG-form operator 230 -> 219 us (and no
-// spill where it had 12 bytes), the FP32 operator 83.7 -> 82.3 us; bf16
-// geometry got slower (63.2 -> 64.4 us), the stand-alone FP64 kernel spilled
-// 124 bytes and the FP64 non-BK PCG form grew from 168 to 256 VGPRs (two
-// waves per SIMD instead of three), so those keep the loads after the barriers.
-template <typename T, int NQ, int NF, bool BK, typename G, bool PCG>
-struct AxEarly {
-  static constexpr bool value = NQ == 8 && NF == 1 && sizeof(G) != 2 && (sizeof(T) == 4 || (PCG && BK));
-};
-template <typename T, int NQ, int NF, bool BK>
-struct AxMinWaves {
-  static constexpr int value =
-      AxDL<NQ, NF, BK>::value ? 4 : (AxGroups<NQ, NF, BK>::fields && sizeof(T) == 8 && NQ <= 10 ? 3 : 1);
-};
-
-template <typename T, int NQ, int NF, bool BK, bool PARTIAL, typename G = T>
-__global__ __launch_bounds__((NQ * NQ * AxGroups<NQ, NF, BK, G>::value), (AxMinWaves<T, NQ, NF, BK>::value)) void k_axhelm(const int32_t Nelements, const int32_t offset,
-                                                                  const int32_t* __restrict__ elementList,
-                                                                  const G* __restrict__ ggeo,
-                                                                  const T* __restrict__ D,
-                                                                  const G* __restrict__ lambda,
-                                                                  const T* __restrict__ q, T* __restrict__ Aq,
-                                                                  const int* __restrict__ skip)
-{
-  constexpr int NQ2 = NQ * NQ;
-  constexpr int NP = NQ2 * NQ;
-  constexpr int EPB = Epb<NQ>::value;
-  constexpr bool FG = AxGroups<NQ, NF, BK, G>::fields;
-  constexpr int GR = AxGroups<NQ, NF, BK, G>::value;
-  if (skip && *skip) return;
-  __shared__ T s_D[NQ2], s_q[GR][NQ2], s_Gr[GR][NQ2], s_Gs[GR][NQ2];
-  const int slot = GR > 1 ? (int)threadIdx.y : 0;  // element slot, or field when FG
-  const int32_t idx = FG ? (int32_t)blockIdx.x : (int32_t)blockIdx.x * EPB + slot;
-  const bool active = EPB == 1 || idx < Nelements;
-  // an idle slot works on the last element without storing: every lane
-  // reaches the workgroup barriers
-  const int32_t ie = EPB == 1 ? (int32_t)blockIdx.x : (active ? idx : Nelements - 1);
-  const int64_t e = PARTIAL ? (int64_t)elementList[ie] : (int64_t)ie;
-  if (slot == 0) s_D[threadIdx.x] = D[threadIdx.x];
-  __syncthreads();
-  AxLane<T, NQ> L;
-  L.init(s_D);
-  const G* g = ggeo + e * (int64_t)(kNggeo * NP) + L.t;
-  const G* l0 = lambda + e * NP + L.t;
-  const G* l1 = lambda + e * NP + offset + L.t;
-  auto field = [&](int f) {
-    const int64_t base = e * NP + (int64_t)f * offset + L.t;
-    T rq[NQ], out[NQ];
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) rq[k] = ldnt(&q[base + k * NQ2]);
-    axhelm_column<T, NQ, BK, G, AxUseDL<T, NQ, NF, BK>::value, !FG, AxEarly<T, NQ, NF, BK, G, false>::value>(L, rq, out, s_D, s_q[slot], s_Gr[slot],
-                                                                     s_Gs[slot], g, l0, l1);
-    if (active) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) stnt(out[k], &Aq[base + k * NQ2]);
+// The elements of a workgroup: a uniform base and a lane offset, so that the
+// loads take a scalar base and one 32-bit lane register; with an element list
+// and several slots the offset is 64 bits wide.  An idle slot of the last
+// workgroup works on its last element and stores nothing (every lane reaches
+// the barriers).
+template <bool PARTIAL, int EPB>
+struct ElemPlace {
+  using IDX = typename std::conditional<PARTIAL && (EPB > 1), int64_t, int32_t>::type;
+  int64_t base;
+  IDX rel;
+  bool active;
+  __device__ __forceinline__ ElemPlace(int32_t first, int32_t Nelements, const int32_t* elementList, int slot)
+  {
+    const int32_t s = EPB == 1 ? 0 : min(slot, Nelements - 1 - first);
+    active = EPB == 1 || s == slot;
+    if constexpr (PARTIAL && EPB > 1) {
+      base = 0;
+      rel = elementList[first + s];
+    } else if constexpr (PARTIAL) {
+      base = elementList[first];
+      rel = 0;
+    } else {
+      base = first;
+      rel = s;
     }
-  };
-  if constexpr (FG) {
-    field(slot);
-  } else {
+  }
+};
+
+// Aq = A q, one field per workgroup.  Three fields: workgroups of one element
+// follow each other on one XCD (workgroup b runs on XCD b % 8), so its L2
+// serves the factors to the second and third.
+template <typename T, int NQ, int NF, bool BK, bool PARTIAL, typename G>
+__global__ __launch_bounds__((NQ * NQ * AxShape<T, NQ, BK>::epb), (AxShape<T, NQ, BK>::waves)) void k_axhelm(
+    const int32_t Nelements, const int32_t offset, const int32_t* __restrict__ elementList,
+    const G* __restrict__ ggeo, const T* __restrict__ D, const G* __restrict__ lambda, const T* __restrict__ q,
+    T* __restrict__ Aq, const int* __restrict__ skip)
+{
+  using S = AxShape<T, NQ, BK>;
+  using LL = LineLayout<T, NQ>;
+  constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = S::epb;
+  if (skip && *skip) return;
+  __shared__ T s_r[EPB][LL::SZ], s_s[EPB][LL::SS];
+  const int t = threadIdx.x, slot = EPB > 1 ? (int)threadIdx.y : 0;
+  int32_t block = blockIdx.x, f = 0;
+  if constexpr (NF > 1) {
+    const int32_t local = block >> 3;
+    f = local % NF;
+    block = (local / NF) * 8 + (block & 7);
+    if ((int64_t)block * EPB >= Nelements) return;
+  }
+  const ElemPlace<PARTIAL, EPB> E(block * EPB, Nelements, elementList, slot);
+  using IDX = typename ElemPlace<PARTIAL, EPB>::IDX;
+  const IDX lo = E.rel * NP + t;
+  GeoStream<T, NQ, BK, G, NF == 1, S::ahead, IDX> geo{ggeo + E.base * (int64_t)(kNggeo * NP), lambda + E.base * NP,
+                                                      lambda + E.base * NP + offset, E.rel * (kNggeo * NP) + t, lo,
+                                                      {}};
+  const T* qf = q + E.base * NP + (int64_t)f * offset;
+  T* Af = Aq + E.base * NP + (int64_t)f * offset;
+  T rq[NQ], out[NQ];
 #pragma unroll
-    for (int f = 0; f < NF; ++f) field(f);
+  for (int k = 0; k < NQ; ++k) rq[k] = ldnt(&qf[lo + k * NQ2]);
+  axhelm_lines<T, NQ, BK>(
+      t, rq, out, (ConstPtr<T>)D, s_r[slot], s_s[slot], geo, []() {},
+      [&](T(&mq)[NQ]) {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) mq[k] = rq[k];
+      });
+  if (E.active) {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) stnt(out[k], &Af[lo + k * NQ2]);
   }
 }
 
-// FP64 BK one-field N = 7 operator, two waves per element (defined in nbx_axhelm.hip).
-__global__ __launch_bounds__(128, 8) void k_axhelm_bk8_split(const int32_t Nelements,
-                                                             const double* ggeo,
-                                                             const double* __restrict__ D,
-                                                             const double* __restrict__ q, double* __restrict__ Aq,
-                                                             const int* __restrict__ skip);
+// Three fields in turn, the element's factors read once (GeoKept); the next
+// field's q is loaded while the factors are applied to the current one.
+template <typename T, int NQ, bool BK, bool PARTIAL, typename G>
+__global__ __launch_bounds__((NQ * NQ * AxKept<T, NQ, BK>::epb), (AxKept<T, NQ, BK>::waves)) void k_axhelm_kept(
+    const int32_t Nelements, const int32_t offset, const int32_t* __restrict__ elementList,
+    const G* __restrict__ ggeo, const T* __restrict__ D, const G* __restrict__ lambda, const T* __restrict__ q,
+    T* __restrict__ Aq, const int* __restrict__ skip)
+{
+  using LL = LineLayout<T, NQ>;
+  constexpr int NF = 3, NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = AxKept<T, NQ, BK>::epb;
+  if (skip && *skip) return;
+  __shared__ T s_r[EPB][LL::SZ], s_s[EPB][LL::SS], s_l[BK ? 1 : EPB * NP], s_w[BK ? 1 : EPB * NP];
+  const int t = threadIdx.x, slot = EPB > 1 ? (int)threadIdx.y : 0;
+  const ElemPlace<PARTIAL, EPB> E((int32_t)blockIdx.x * EPB, Nelements, elementList, slot);
+  using IDX = typename ElemPlace<PARTIAL, EPB>::IDX;
+  const IDX lo = E.rel * NP + t;
+  const T* qf = q + E.base * NP;
+  T* Af = Aq + E.base * NP;
+  T rq[NQ], out[NQ];
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) rq[k] = ldnt(&qf[lo + k * NQ2]);
+  GeoKept<T, NQ, BK, G, IDX> geo{{ggeo + E.base * (int64_t)(kNggeo * NP), lambda + E.base * NP,
+                                  lambda + E.base * NP + offset, E.rel * (kNggeo * NP) + t, lo, {}},
+                                 s_l + (BK ? 0 : slot * NP + t),
+                                 s_w + (BK ? 0 : slot * NP + t)};
+  geo.load();
+#pragma unroll 1
+  for (int f = 0; f < NF; ++f) {
+    const T* qc = qf;
+    if (f + 1 < NF) qf += offset;
+    axhelm_lines<T, NQ, BK>(
+        t, rq, out, (ConstPtr<T>)D, s_r[slot], s_s[slot], geo,
+        [&]() {
+#pragma unroll
+          for (int k = 0; k < NQ; ++k) rq[k] = qf[lo + k * NQ2];
+        },
+        [&](T(&mq)[NQ]) {
+          if (!BK) {
+#pragma unroll
+            for (int k = 0; k < NQ; ++k) mq[k] = qc[lo + k * NQ2];
+          }
+        });
+    if (E.active) {
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) stnt(out[k], &Af[lo + k * NQ2]);
+    }
+    Af += offset;
+  }
+}
+
+// The three-field Helmholtz PCG form at 8 <= Nq <= 12 (FP64 and FP32
+// geometry) sums a lane's share of pAp per field, then (f0 + f1) + f2; every
+// other form runs one chain over fields then k.  The oracle states both.
+template <int NQ, int NF, bool BK, typename G>
+struct AxFieldSums {
+  static constexpr bool value = NF == 3 && !BK && NQ >= 8 && NQ <= 12 && sizeof(G) != 2;
+};
+
+template <int NQ2>
+constexpr int kTreeWidth = NQ2 <= 4 ? 4 : NQ2 <= 16 ? 16 : NQ2 <= 32 ? 32 : NQ2 <= 64 ? 64 : NQ2 <= 128 ? 128 : 256;
+
+// Sum of the NQ2 lane values of an element in the halving tree over the next
+// power of two (zero padded); valid in the slot's lane t = 0.  tid: the lane
+// in the workgroup, slot 0's lanes first; `on` is false in lanes that take no
+// part (every lane of the workgroup calls, for the barriers).
+template <int NQ2, int EPB>
+__device__ __forceinline__ double lane_tree(double v, double* s_red, const int slot, const int t, const int tid,
+                                            const bool on)
+{
+  constexpr int P2 = kTreeWidth<NQ2>;
+  if constexpr (P2 == NQ2 && P2 <= 64) {  // the slot's lanes are one aligned part of a wave
+#pragma unroll
+    for (int h = P2 / 2; h >= 1; h >>= 1) v += __shfl_xor(v, h, 64);
+    return v;
+  } else {
+    double* const red = s_red + slot * P2;
+    if (on) {
+      red[t] = v;
+      if (t + NQ2 < P2) red[t + NQ2] = 0.0;
+    }
+    if constexpr (P2 > 64) {
+      // the first wave of each slot (EPB = 1 here) sums 64 lanes from registers
+      static_assert(EPB == 1, "one element per workgroup from Nq = 9 up");
+      __syncthreads();
+      double x = 0.0;
+      if (tid < 64) {
+        x = P2 == 256 ? (red[tid] + red[tid + 128]) + (red[tid + 64] + red[tid + 192]) : red[tid] + red[tid + 64];
+        x = wave_sum(x);
+      }
+      return x;
+    } else {
+      for (int h = P2 / 2; h >= 1; h >>= 1) {
+        __syncthreads();
+        if (on && t < h) red[t] = red[t] + red[t + h];
+      }
+      return red[0];
+    }
+  }
+}
 
 // PCG form (FP64): p = z + beta p (BPScaledAdd, nekBone/solve.cpp:100), then
 // Ap_local = A p, and the element's share of pAp = sum_nodes p * Ap_local.
 // Because p is continuous and zero on the mask, sum_local p (A_L p) equals
 // <p, gs(A_L p)>_w exactly in real arithmetic (the weights 1/multiplicity
 // undo the gather-scatter); this value is what BPAxOperator's dot returns.
-// Lane (i,j) accumulates fma(p, Ap) over fields then k -- with one thread
-// group per field (three fields, non-BK, 8 <= Nq <= 12) each field's chain runs over k and
-// the lane takes (field0 + field1) + field2; the NQ*NQ lanes are summed by a
-// halving tree over the next power of two (zero padded); the element
-// partials go to partials[e].
-template <int NQ, int NF, bool BK, typename T, typename G>
-__global__ __launch_bounds__((NQ * NQ * AxGroups<NQ, NF, BK, G>::value), (AxMinWaves<T, NQ, NF, BK>::value)) void k_axhelm_pcg(const int32_t Nelements, const int32_t offset,
-                                                                      const G* __restrict__ ggeo,
-                                                                      const T* __restrict__ D,
-                                                                      const G* __restrict__ lambda,
-                                                                      const double* __restrict__ z,
-                                                                      double* __restrict__ p,
-                                                                      double* __restrict__ Ap,
-                                                                      double* __restrict__ partials,
-                                                                      const PcgFlags* __restrict__ S)
+// The lanes' shares are summed by lane_tree; the element partials go to
+// partials[e].
+// FG (three fields): one thread group of NQ2 lanes per field of an element
+// (threadIdx.y = field) instead of the fields in turn; the groups hand the
+// lane sums on through LDS in field order.
+template <int NQ, int NF, bool BK, typename T, typename G, bool FG>
+struct AxPcg {
+  static constexpr bool kept = NF == 3 && !FG && AxKept<T, NQ, BK>::value;
+  static constexpr int epb = FG ? 1 : kept ? AxKept<T, NQ, BK>::epb : AxShape<T, NQ, BK>::epb;
+  static constexpr int waves = kept ? AxKept<T, NQ, BK>::waves : NF == 1 ? AxShape<T, NQ, BK>::waves : 1;
+  // the next field's z and p in flight during the current one, where the registers allow it
+  static constexpr bool prefetch = kept && (sizeof(T) == 4 || NQ <= 8);
+  static constexpr bool late = NF == 3 && !FG && !prefetch;
+};
+
+template <int NQ, int NF, bool BK, typename T, typename G, bool FG>
+__global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FG>::epb * (FG ? NF : 1)), (AxPcg<NQ, NF, BK, T, G, FG>::waves)) void k_axhelm_pcg(
+    const int32_t Nelements, const int32_t offset, const G* __restrict__ ggeo, const T* __restrict__ D,
+    const G* __restrict__ lambda, const double* __restrict__ z, double* __restrict__ p, double* __restrict__ Ap,
+    double* __restrict__ partials, const PcgFlags* __restrict__ S)
 {
-  constexpr int NQ2 = NQ * NQ;
-  constexpr int NP = NQ2 * NQ;
-  constexpr int EPB = Epb<NQ>::value;
-  constexpr bool FG = AxGroups<NQ, NF, BK, G>::fields;
-  constexpr int GR = AxGroups<NQ, NF, BK, G>::value;
-  constexpr int P2 = NQ2 <= 1 ? 1 : (NQ2 <= 2 ? 2 : (NQ2 <= 4 ? 4 : (NQ2 <= 8 ? 8 : (NQ2 <= 16 ? 16 : (NQ2 <= 32 ? 32 : (NQ2 <= 64 ? 64 : (NQ2 <= 128 ? 128 : 256)))))));
+  using P = AxPcg<NQ, NF, BK, T, G, FG>;
+  using LL = LineLayout<T, NQ>;
+  constexpr bool SUMS = AxFieldSums<NQ, NF, BK, G>::value;
+  constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = P::epb, GR = EPB * (FG ? NF : 1), LOOP = FG ? 1 : NF;
   if (S->done) return;
   const double beta = S->beta;
-  __shared__ T s_D[NQ2], s_q[GR][NQ2], s_Gr[GR][NQ2], s_Gs[GR][NQ2];
-  __shared__ double s_red[GR][P2];
-  const int slot = GR > 1 ? (int)threadIdx.y : 0;  // element slot, or field when FG
-  const int32_t idx = FG ? (int32_t)blockIdx.x : (int32_t)blockIdx.x * EPB + slot;
-  const bool active = EPB == 1 || idx < Nelements;
-  // idle slots compute on the last element and store nothing
-  const int64_t e = EPB == 1 ? (int64_t)blockIdx.x : (active ? idx : Nelements - 1);
-  if (slot == 0) s_D[threadIdx.x] = D[threadIdx.x];
-  __syncthreads();
-  AxLane<T, NQ> L;
-  L.init(s_D);
-  const G* g = ggeo + e * (int64_t)(kNggeo * NP) + L.t;
-  const G* l0 = lambda + e * NP + L.t;
-  const G* l1 = lambda + e * NP + offset + L.t;
-  double acc = 0.0;
-  auto field = [&](int f) {
-    const int64_t base = e * NP + (int64_t)f * offset + L.t;
-    double pk[NQ];
-    T rq[NQ], out[NQ];
+  __shared__ T s_r[GR][LL::SZ], s_s[GR][LL::SS];
+  __shared__ T s_l[P::kept && !BK ? EPB * NP : 1], s_w[P::kept && !BK ? EPB * NP : 1];
+  __shared__ double s_red[EPB * kTreeWidth<NQ2>], s_acc[FG ? NF : 1][FG ? NQ2 : 1];
+  const int t = threadIdx.x, y = GR > 1 ? (int)threadIdx.y : 0, slot = FG ? 0 : y, field0 = FG ? y : 0;
+  const ElemPlace<false, EPB> E((int32_t)blockIdx.x * EPB, Nelements, nullptr, slot);
+  const int32_t lo = E.rel * NP + t;
+  const double* zf = z + E.base * NP + (int64_t)field0 * offset;
+  double* pf = p + E.base * NP + (int64_t)field0 * offset;
+  double* Af = Ap + E.base * NP + (int64_t)field0 * offset;
+  const G* const gb = ggeo + E.base * (int64_t)(kNggeo * NP);
+  const G* const lb = lambda + E.base * NP;
+  const int32_t go = E.rel * (kNggeo * NP) + t;
+  double zn[NQ], pn[NQ], acc = 0.0, fsum[NF];
+  auto load_zp = [&]() {
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-      pk[k] = __builtin_fma(beta, p[base + k * NQ2], ldnt(&z[base + k * NQ2]));
-      rq[k] = (T)pk[k];
-    }
-    if (EPB > 1) __syncthreads();  // all slots read p before any writes it (idle slots alias the last element)
-    if (active) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) p[base + k * NQ2] = pk[k];
-    }
-    axhelm_column<T, NQ, BK, G, AxUseDL<T, NQ, NF, BK>::value, !FG, AxEarly<T, NQ, NF, BK, G, true>::value>(L, rq, out, s_D, s_q[slot], s_Gr[slot],
-                                                                     s_Gs[slot], g, l0, l1);
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-      const double o = (double)out[k];
-      if (active) stnt(o, &Ap[base + k * NQ2]);
-      acc = __builtin_fma(pk[k], o, acc);
+      pn[k] = pf[lo + k * NQ2];
+      zn[k] = ldnt(&zf[lo + k * NQ2]);
     }
   };
-  if constexpr (FG) {
-    field(slot);
-    double* fa = s_red[slot];
-    fa[L.t] = acc;
-    __syncthreads();
-    acc = (s_red[0][L.t] + s_red[1][L.t]) + s_red[2][L.t];
-    __syncthreads();
-  } else {
+  if (P::prefetch) load_zp();
+  auto run = [&](auto& geo) {
+#pragma unroll 1
+    for (int f = 0; f < LOOP; ++f) {
+      T rq[NQ], out[NQ];
+      double pk[NQ];
+      if (!P::prefetch) load_zp();
 #pragma unroll
-    for (int f = 0; f < NF; ++f) field(f);
-  }
-  double sum;
-  if (NQ2 == 64) {
-    sum = wave_sum(acc);
-  } else {
-    double* red = s_red[slot];
-    red[L.t] = acc;
-    if (L.t + NQ2 < P2) red[L.t + NQ2] = 0.0;
-    for (int h = P2 / 2; h >= 1; h >>= 1) {
-      __syncthreads();
-      if (L.t < h) red[L.t] = red[L.t] + red[L.t + h];
+      for (int k = 0; k < NQ; ++k) {
+        const double v = __builtin_fma(beta, pn[k], zn[k]);
+        rq[k] = (T)v;
+        if (E.active) pf[lo + k * NQ2] = v;
+        if (LOOP == 1) pk[k] = v;
+      }
+      const double* const pc = pf;
+      if (f + 1 < LOOP) {
+        pf += offset;
+        zf += offset;
+      }
+      axhelm_lines<T, NQ, BK, P::late>(
+          t, rq, out, (ConstPtr<T>)D, s_r[y], s_s[y], geo,
+          [&]() {
+            if (P::prefetch) load_zp();  // the next field's (at the end the last field's again, unused)
+          },
+          [&](T(&mq)[NQ]) {
+#pragma unroll
+            for (int k = 0; k < NQ; ++k) {
+              if (LOOP > 1) pk[k] = pc[lo + k * NQ2];  // this lane's own store
+              mq[k] = (T)pk[k];
+            }
+          });
+      if (SUMS) acc = 0.0;
+      if (FG && !SUMS) {  // the chain over fields then k: each group continues the previous one's
+        for (int c = 0; c < NF; ++c) {
+          if (c == y) {
+            acc = c == 0 ? 0.0 : s_acc[c - 1][t];
+#pragma unroll
+            for (int k = 0; k < NQ; ++k) acc = __builtin_fma(pk[k], (double)out[k], acc);
+            s_acc[c][t] = acc;
+          }
+          __syncthreads();
+        }
+        acc = s_acc[NF - 1][t];
+      } else {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) acc = __builtin_fma(pk[k], (double)out[k], acc);
+      }
+      if (E.active) {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) stnt((double)out[k], &Af[lo + k * NQ2]);
+      }
+      Af += offset;
+      if (SUMS && !FG) {
+        if (f == 0) fsum[0] = acc;
+        else if (f == 1) fsum[NF > 1 ? 1 : 0] = acc;
+        else fsum[NF - 1] = acc;
+      }
     }
-    __syncthreads();
-    sum = red[0];
+  };
+  if constexpr (P::kept) {
+    GeoKept<T, NQ, BK, G, int32_t> geo{{gb, lb, lb + offset, go, lo, {}},
+                                       s_l + (BK ? 0 : slot * NP + t),
+                                       s_w + (BK ? 0 : slot * NP + t)};
+    geo.load();
+    run(geo);
+  } else {
+    GeoStream<T, NQ, BK, G, NF == 1, AxShape<T, NQ, BK>::ahead, int32_t> geo{gb, lb, lb + offset, go, lo, {}};
+    run(geo);
   }
-  if (L.t == 0 && active && (!FG || slot == 0)) partials[e] = sum;
+  if constexpr (SUMS && FG) {
+    s_acc[y][t] = acc;
+    __syncthreads();
+    acc = (s_acc[0][t] + s_acc[1][t]) + s_acc[2][t];
+  } else if constexpr (SUMS) {
+    acc = (fsum[0] + fsum[1]) + fsum[2];
+  }
+  const double sum = lane_tree<NQ2, EPB>(acc, s_red, slot, t, y * NQ2 + t, y == slot);
+  if (t == 0 && y == slot && E.active) partials[E.base + E.rel] = sum;
 }
 
 // Local Jacobi diagonal, nekBone/kernel/updateJacobi.okl:27-108, same
@@ -397,19 +705,22 @@ static int launch_axhelm_t(int32_t Nelements, int32_t offset, const int32_t* ele
                            const void* ggeo, const void* D, const void* lambda, const void* q, void* Aq,
                            const int* skip, hipStream_t s)
 {
-  if constexpr (std::is_same<T, double>::value && std::is_same<G, double>::value && NQ == 8 && NF == 1 && BK &&
-                !PARTIAL) {
-    if (Nelements <= 0) return NBX_SUCCESS;
-    hipLaunchKernelGGL(k_axhelm_bk8_split, dim3(Nelements), dim3(64, 2), 0, s, Nelements, (const double*)ggeo,
-                       (const double*)D, (const double*)q, (double*)Aq, skip);
-    NBX_HIP_LAUNCH();
-    return NBX_SUCCESS;
+  if (Nelements <= 0) return NBX_SUCCESS;
+  if constexpr (NF == 3 && AxKept<T, NQ, BK>::value) {
+    if (AxKept<T, NQ, BK>::when(Nelements)) {
+      constexpr int EPB = AxKept<T, NQ, BK>::epb;
+      hipLaunchKernelGGL((k_axhelm_kept<T, NQ, BK, PARTIAL, G>), dim3((Nelements + EPB - 1) / EPB),
+                         dim3(NQ * NQ, EPB), 0, s, Nelements, offset, elementList, (const G*)ggeo, (const T*)D,
+                         (const G*)lambda, (const T*)q, (T*)Aq, skip);
+      NBX_HIP_LAUNCH();
+      return NBX_SUCCESS;
+    }
   }
-  constexpr int EPB = Epb<NQ>::value;
-  constexpr int GR = AxGroups<NQ, NF, BK, G>::value;
-  hipLaunchKernelGGL((k_axhelm<T, NQ, NF, BK, PARTIAL, G>), dim3((Nelements + EPB - 1) / EPB), dim3(NQ * NQ, GR), 0,
-                     s, Nelements, offset, elementList, (const G*)ggeo, (const T*)D, (const G*)lambda,
-                     (const T*)q, (T*)Aq, skip);
+  constexpr int EPB = AxShape<T, NQ, BK>::epb;
+  const int32_t blocks = (Nelements + EPB - 1) / EPB;
+  const unsigned grid = NF == 1 ? (unsigned)blocks : (unsigned)((blocks + 7) / 8 * 8) * NF;
+  hipLaunchKernelGGL((k_axhelm<T, NQ, NF, BK, PARTIAL, G>), dim3(grid), dim3(NQ * NQ, EPB), 0, s, Nelements, offset,
+                     elementList, (const G*)ggeo, (const T*)D, (const G*)lambda, (const T*)q, (T*)Aq, skip);
   NBX_HIP_LAUNCH();
   return NBX_SUCCESS;
 }
@@ -471,30 +782,39 @@ static int dispatch_n(int N, int Nf, int bk, bool partial, int32_t Nelements, in
   }
 }
 
+template <int NQ, int NF, bool BK, typename T, typename G>
+static void axhelm_pcg_launch_k(int32_t Nelements, int32_t offset, const void* ggeo, const void* D,
+                                const void* lambda, const double* z, double* p, double* Ap, double* partials,
+                                const PcgFlags* S, hipStream_t s)
+{
+  if constexpr (NF == 3 && AxFieldGroups<T, NQ, BK, G>::fits) {
+    if (AxFieldGroups<T, NQ, BK, G>::when(Nelements)) {
+      hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, true>), dim3(Nelements), dim3(NQ * NQ, NF), 0, s, Nelements,
+                         offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap, partials, S);
+      return;
+    }
+  }
+  constexpr int EPB = AxPcg<NQ, NF, BK, T, G, false>::epb;
+  hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, false>), dim3((Nelements + EPB - 1) / EPB), dim3(NQ * NQ, EPB), 0,
+                     s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap, partials, S);
+}
+
 template <typename T, typename G>
 static int axhelm_pcg_launch_t(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                                const void* D, const void* lambda, const double* z, double* p, double* Ap,
                                double* partials, const PcgFlags* S, hipStream_t s)
 {
-#define NBX_AXP(NV)                                                                                          \
-  case NV:                                                                                                   \
-    if (Nelements < 1) break;                                                                                \
-    if (Nf == 1 && bk)                                                                                       \
-      hipLaunchKernelGGL((k_axhelm_pcg<NV + 1, 1, true, T, G>), dim3((Nelements + Epb<NV + 1>::value - 1) / Epb<NV + 1>::value), dim3((NV + 1) * (NV + 1), Epb<NV + 1>::value), 0, \
-                         s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap,       \
-                         partials, S);                                                                       \
-    else if (Nf == 1)                                                                                        \
-      hipLaunchKernelGGL((k_axhelm_pcg<NV + 1, 1, false, T, G>), dim3((Nelements + Epb<NV + 1>::value - 1) / Epb<NV + 1>::value), dim3((NV + 1) * (NV + 1), Epb<NV + 1>::value),   \
-                         0, s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap,    \
-                         partials, S);                                                                       \
-    else if (bk)                                                                                             \
-      hipLaunchKernelGGL((k_axhelm_pcg<NV + 1, 3, true, T, G>), dim3((Nelements + Epb<NV + 1>::value - 1) / Epb<NV + 1>::value), dim3((NV + 1) * (NV + 1), AxGroups<NV + 1, 3, true, G>::value), 0, \
-                         s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap,       \
-                         partials, S);                                                                       \
-    else                                                                                                     \
-      hipLaunchKernelGGL((k_axhelm_pcg<NV + 1, 3, false, T, G>), dim3((Nelements + Epb<NV + 1>::value - 1) / Epb<NV + 1>::value), dim3((NV + 1) * (NV + 1), AxGroups<NV + 1, 3, false, G>::value),   \
-                         0, s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap,    \
-                         partials, S);                                                                       \
+#define NBX_AXP(NV)                                                                                              \
+  case NV:                                                                                                       \
+    if (Nelements < 1) break;                                                                                    \
+    if (Nf == 1 && bk)                                                                                           \
+      axhelm_pcg_launch_k<NV + 1, 1, true, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);   \
+    else if (Nf == 1)                                                                                            \
+      axhelm_pcg_launch_k<NV + 1, 1, false, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);  \
+    else if (bk)                                                                                                 \
+      axhelm_pcg_launch_k<NV + 1, 3, true, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);   \
+    else                                                                                                         \
+      axhelm_pcg_launch_k<NV + 1, 3, false, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);  \
     break;
   if (Nf != 1 && Nf != 3) return fail(NBX_ERR_UNSUPPORTED, "axhelm_pcg: Nfields=%d", Nf);
   switch (N) {
