@@ -3,6 +3,7 @@
 // of a network to a BP handle.  The kernels are in nbx_net.hip.
 #include "nbx_bp_internal.h"
 #include "nbx_net.h"
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -17,8 +18,10 @@ struct nbx_net {
   float* v = nullptr;
   float* grad = nullptr;
   double* loss = nullptr;
-  float* partials = nullptr;
+  float* partials = nullptr;  // gradient sums of the chunks
   int partial_cap = 0;
+  float* grads = nullptr;     // gradients of up to kNetBatch samples
+  int grads_cap = 0;
   int2* samples = nullptr;
   int sample_cap = 0;
   int steps = 0;
@@ -88,7 +91,7 @@ void net_release(nbx_net* n)
   (void)hipDeviceSynchronize();
   for (nbx_bp* bp : n->attached) bp->net = nullptr;  // LEARNED solves now fail with an error
   for (void* p : {(void*)n->master, (void*)n->wbf, (void*)n->frag, (void*)n->m, (void*)n->v, (void*)n->grad, (void*)n->loss,
-                  (void*)n->partials, (void*)n->samples, (void*)n->R, (void*)n->Ev, (void*)n->invNorm,
+                  (void*)n->partials, (void*)n->grads, (void*)n->samples, (void*)n->R, (void*)n->Ev, (void*)n->invNorm,
                   (void*)n->work, (void*)n->invNormE})
     if (p) (void)hipFree(p);
   delete n;
@@ -585,6 +588,14 @@ static int ensure_work(nbx_net* n, int nsamples, int chunk)
     NBX_HIP(hipMalloc(&n->partials, sizeof(float) * kNetPartial * (size_t)nblocks));
     n->partial_cap = nblocks;
   }
+  const int held = std::min(nsamples, kNetBatch);
+  if (held > n->grads_cap) {
+    if (n->grads) (void)hipFree(n->grads);
+    n->grads = nullptr;
+    n->grads_cap = 0;
+    NBX_HIP(hipMalloc(&n->grads, sizeof(float) * kNetPartial * (size_t)held));
+    n->grads_cap = held;
+  }
   return NBX_SUCCESS;
 }
 
@@ -592,9 +603,11 @@ static int ensure_work(nbx_net* n, int nsamples, int chunk)
 static int run_gradient(nbx_net* n, nbx_bp* bp, int nsamples, int chunk, const double* G = nullptr)
 {
   const int nblocks = (nsamples + chunk - 1) / chunk;
-  int rc = net_train_launch(nsamples, chunk, n->samples, n->pairStride, n->R, n->Ev, n->invNorm, n->wbf, bp->feat,
-                            bp->invDiagA, G, n->partials, bp->stream);
-  if (rc) return rc;
+  for (int first = 0; first < nsamples; first += kNetBatch) {
+    int rc = net_train_launch(first, std::min(kNetBatch, nsamples - first), chunk, n->samples, n->pairStride, n->R,
+                              n->Ev, n->invNorm, n->wbf, bp->feat, bp->invDiagA, G, n->grads, n->partials, bp->stream);
+    if (rc) return rc;
+  }
   return net_grad_sum_launch(nblocks, n->partials, n->grad, n->loss, bp->stream);
 }
 

@@ -10,7 +10,8 @@ namespace nbx {
 constexpr int kOffWr = 0, kOffWg = 864, kOffB1 = 1088, kOffW2 = 1120, kOffB2 = 2144, kOffW3 = 2176, kOffB3 = 3040;
 constexpr int kNetParams = 3041;
 constexpr int kNetParamsPadded = 3042;  // loss (double) follows, 8-byte aligned
-constexpr int kNetPartial = 3044;       // floats per workgroup partial
+constexpr int kNetPartial = 3044;       // floats of a sample's or a chunk's gradient and loss
+constexpr int kNetBatch = 4096;         // samples whose gradients are held at once
 
 int net_apply_launch(int32_t E, const float* W, const float* feat, const double* r, const double* invDiag,
                      const double* w, double* zl, const int* fallback, const int* skip, hipStream_t s);
@@ -29,10 +30,9 @@ int net_apply_mma_launch(int32_t E, const void* frag, const float* W, const uint
 int net_apply_mma_resid_launch(int32_t E, const void* frag, const float* W, const uint16_t* feat16,
                                const float* res, const float* Ad, const double* invDiag, const double* w,
                                const uint8_t* deg, double* zl, const int* skip, hipStream_t s);
-size_t net_train_lds_bytes();
-int net_train_launch(int32_t nsamples, int32_t chunk, const int2* samples, int64_t pairStride, const float* R,
-                     const float* Ev, const double* invNorm, const float* W, const float* feat, const double* invDiag,
-                     const double* G, float* partials, hipStream_t s);
+int net_train_launch(int32_t first, int32_t count, int32_t chunk, const int2* samples, int64_t pairStride,
+                     const float* R, const float* Ev, const double* invNorm, const float* W, const float* feat,
+                     const double* invDiag, const double* G, float* grads, float* partials, hipStream_t s);
 int net_grad_sum_launch(int32_t nblocks, const float* partials, float* grad, double* loss, hipStream_t s);
 int net_adam_launch(float* master, float* m, float* v, const float* grad, float* wbf, float lr, int step,
                     hipStream_t s);

@@ -30,10 +30,19 @@
 namespace nbx {
 
 constexpr int kP = 512, kC = 32, kG = 7, kTaps = 27;
-// row stride of the [channel][node] LDS tiles of the training kernel: odd, so
-// the 32 lanes of a parameter gradient that read 32 channel rows at the same
-// node hit 32 different banks
-constexpr int kRow = kP + 1;
+constexpr int kPad = 10, kPadN = kPad * kPad * kPad;  // zero-padded tile of the training kernel
+constexpr int kFRow = 800;                            // a factor row: node (x, y, z) at 100 z + 10 y + x
+// 128 nodes of 96 channel rows; row stride 4 modulo the banks, so the 8 rows
+// that 8 lanes read 16 bytes of lie in different banks
+constexpr int kTrainRow = 132, kTrainRows = 96;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// place of the tap's neighbour in the padded tile, relative to the node's 100 z + 10 y + x
+__host__ __device__ constexpr int tap_place(int tap)
+{
+  return 111 + (tap / 9 - 1) * 100 + ((tap / 3) % 3 - 1) * 10 + (tap % 3 - 1);
+}
 
 __device__ __forceinline__ int tap_neighbor(int n, int tap)
 {
@@ -151,215 +160,351 @@ __global__ __launch_bounds__(512) void k_net_apply(const int32_t E, const float*
   zl[id] = wn * (di * (rn + s * (double)y));
 }
 
-// Training: each workgroup runs a chunk of (pair, element) samples through
-// forward and backward and accumulates the parameter gradient and the loss
-//   L = sum_samples inv_norm[pair] sum_n (z_n - e_n)^2
-// in lane-owned registers (parameter q is owned by lane q mod 512 of its
-// tensor); one partial per workgroup goes to partials[block][kNetParams+1].
-// With G non-null the loss is defined outside (energy norm of the assembled
-// error) and G[e*512+n] holds its derivative with respect to the unweighted
-// element output invDiag (r + s y) at local node n of element e; the kernel
-// then back-propagates dL/dy = G invDiag s and reports no loss.
-__global__ __launch_bounds__(512) void k_net_train(const int32_t nsamples, const int32_t chunk,
-                                                   const int2* __restrict__ samples, const int64_t pairStride,
-                                                   const float* __restrict__ R, const float* __restrict__ Ev,
-                                                   const double* __restrict__ invNorm, const float* __restrict__ W,
-                                                   const float* __restrict__ feat, const double* __restrict__ invDiag,
-                                                   const double* __restrict__ G, float* __restrict__ partials)
+// Training: one workgroup per (pair, element) sample, forward and backward;
+// the sample's parameter gradient goes to out[sample][kNetPartial], its loss
+//   L = inv_norm[pair] sum_n (z_n - e_n)^2
+// behind it.  With G non-null the loss is defined outside (energy norm of the
+// assembled error) and G[e*512+n] holds its derivative with respect to the
+// unweighted element output invDiag (r + s y) at local node n of element e;
+// the kernel then back-propagates dL/dy = G invDiag s and reports no loss.
+//
+// Lane n is node n for the forward pass and the data gradients (weights as
+// scalar operands, FP32 vector ALUs).  The parameter gradients are products
+// over the 512 nodes, dW[a][c] = sum_n A[a][n] B[n][c], an fma chain in
+// increasing n: they run on the matrix cores as 16x16x4 FP32 products, which
+// accumulate k in increasing order with one rounding a step -- the chain's
+// bits -- one 16x16 tile of one tensor a wave, 16 tiles over two phases:
+//   phase 1: W3 (taps x channels; dL/dT and h2), W2 (h1 and dL/dpre2)
+//   phase 2: Wr, Wg and b1 as 35 rows (r^ taps, factors, ones; dL/dpre1),
+//            b2 (ones; dL/dpre2), and b3 as a plain chain beside them.
+// The lanes hand their channels to the tiles through LDS 128 nodes at a time,
+// nodes ordered inside 16 so that a lane's four k values are one 16-byte
+// read; the tap operands are the zero-padded 10^3 tiles of r^ and dL/dy at a
+// fixed offset, the factors rows of the same layout.
+// Bound: FP32 vector issue (4864 fma a node, 130 us of 2048 samples on this
+// chip) beside 2048 matrix products of 32 cycles a sample (55 us); 80 KB of
+// LDS and 128 registers keep two workgroups a CU, so that one's products run
+// under the other's vector work.  2048 samples: 3836 -> 290 us against the
+// form that held one parameter a lane (two LDS reads an fma) and gave a
+// workgroup a whole chunk of samples (half the chip idle at 16 a chunk).
+struct TrainLds {
+  float rh[kPadN], dy[kPadN];      // zero-padded tiles
+  float g[kG * kFRow];             // factors, node (x, y, z) at 100 z + 10 y + x
+  float buf[kTrainRows * kTrainRow];  // T exchange, then 128 nodes of the channels
+  double red[kP / 64];
+};
+
+// Half a row of 32 weights in scalar registers (constant address space:
+// scalar loads); the pointer is made opaque at every half, or the compiler
+// loads weights long before their use and spills them.  for_rows runs
+// f(r, c, w[c % 16]) over the rows and channels in order; the next half's loads
+// are issued after the first product, which waits for this half's, and are in
+// flight during the others.
+typedef const float __attribute__((address_space(4)))* WeightPtr;
+struct WHalf {
+  float w[kC / 2];
+  __device__ __forceinline__ void load(WeightPtr p, int half)
+  {
+    asm volatile("" : "+s"(p));
+#pragma unroll
+    for (int c = 0; c < kC / 2; ++c) w[c] = p[half * (kC / 2) + c];
+  }
+};
+template <int ROWS, typename F>
+__device__ __forceinline__ void for_rows(const float* base, F&& f)
 {
-  extern __shared__ float lds[];
-  float* R1 = lds;                    // [32][kRow]: h2 -> h1 -> dpre1
-  float* R2 = R1 + kC * kRow;         // [32][kRow]: T / dT -> dpre2
-  float* s_rh = R2 + kC * kRow;       // [512]
-  float* s_g = s_rh + kP;             // [7][512]
-  float* s_dy = s_g + kG * kP;        // [512]
-  double* s_red = (double*)(s_dy + kP);  // [8]
-  const int n = threadIdx.x;
-  const float* W3 = W + kOffW3;
+  const WeightPtr p = (WeightPtr)base;
+  WHalf R, Rn;
+  R.load(p, 0);
+#pragma unroll
+  for (int h = 0; h < 2 * ROWS; ++h) {
+    const int c0 = (h & 1) * (kC / 2);
+    f(h >> 1, c0, R.w[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (h + 1 < 2 * ROWS) Rn.load(p, h + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 1; c < kC / 2; ++c) f(h >> 1, c0 + c, R.w[c]);
+    R = Rn;
+  }
+}
+// the value is formed here: without this the compiler moves whole products,
+// weights and all, into the later branch that stores their results
+__device__ __forceinline__ void keep_here(float& v) { asm volatile("" : "+v"(v)); }
+// acc[c] = fma(w[r][c], x(r), acc[c]) over the rows in order
+template <int ROWS, typename X>
+__device__ __forceinline__ void add_rows(const float* base, X&& x, float (&acc)[kC])
+{
+  float v;
+  for_rows<ROWS>(base, [&](int r, int c, float w) {
+    if (c == 0) v = x(r);
+    acc[c] = __builtin_fmaf(w, v, acc[c]);
+  });
+#pragma unroll
+  for (int c = 0; c < kC; ++c) keep_here(acc[c]);
+}
+// to(r, sum_c w[r][c] x[c]), the chain over c in order
+template <int ROWS, typename S>
+__device__ __forceinline__ void dot_rows(const float* base, const float (&x)[kC], S&& to)
+{
+  float t;
+  for_rows<ROWS>(base, [&](int r, int c, float w) {
+    t = __builtin_fmaf(w, x[c], c == 0 ? 0.f : t);
+    if (c == kC - 1) {
+      keep_here(t);
+      to(r, t);
+    }
+  });
+}
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
+{
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ samples, const int64_t pairStride,
+                                                      const float* __restrict__ R, const float* __restrict__ Ev,
+                                                      const double* __restrict__ invNorm, const float* __restrict__ W,
+                                                      const float* __restrict__ feat,
+                                                      const double* __restrict__ invDiag,
+                                                      const double* __restrict__ G, float* __restrict__ out)
+{
+  __shared__ TrainLds lds;
+  const int n = threadIdx.x, l = n & 63, wv = n >> 6, col = l & 15, kg = l >> 4;
+  const int i = n & 7, j = (n >> 3) & 7, k = n >> 6;
+  const int place = 100 * k + 10 * j + i;  // in the 10-strided layout; the tiles' interior starts at 111
+  const float* Wr = W + kOffWr;
+  const float* Wg = W + kOffWg;
   const float* W2 = W + kOffW2;
-  float gW3[2] = {0.f, 0.f}, gW2[2] = {0.f, 0.f}, gWr[2] = {0.f, 0.f}, gWg = 0.f, gb1 = 0.f, gb2 = 0.f, gb3 = 0.f;
-  double loss = 0.0;
-  const int32_t s0 = blockIdx.x * chunk, s1 = min(nsamples, s0 + chunk);
-  for (int32_t si = s0; si < s1; ++si) {
-    const int2 pe = samples[si];
-    const int64_t e = pe.y;
-    const int64_t off = (int64_t)pe.x * pairStride + e * kP + n;
-    const double rn = (double)R[off];
-    const double en = G ? 0.0 : (double)Ev[off];
-    const double di = invDiag[e * kP + n];
-    __syncthreads();  // previous sample done with LDS
-    const double s = element_scale(rn, s_red);
-    const double inv = s > 0.0 ? 1.0 / s : 0.0;
-    s_rh[n] = (float)(rn * inv);
-    float g[kG];
+  const float* W3 = W + kOffW3;
+  const int2 pe = samples[blockIdx.x];
+  const int64_t e = pe.y;
+  const int64_t off = (int64_t)pe.x * pairStride + e * kP + n;
+  const double rn = (double)R[off];
+  const double en = G ? 0.0 : (double)Ev[off];
+  const double di = invDiag[e * kP + n];
+  for (int q = n; q < kPadN; q += kP) lds.rh[q] = lds.dy[q] = 0.f;
+  float h1[kC], g[kG];
 #pragma unroll
-    for (int q = 0; q < kG; ++q) {
-      g[q] = feat[(e * kG + q) * kP + n];
-      s_g[q * kP + n] = g[q];
-    }
-    __syncthreads();
-    NetFwd a;
-    float T[kTaps];
-    net_forward_lane(W, n, s_rh, g, a, T);
+  for (int q = 0; q < kG; ++q) g[q] = feat[(e * kG + q) * kP + n];
 #pragma unroll
-    for (int tap = 0; tap < kTaps; ++tap) R2[tap * kRow + n] = T[tap];
-    __syncthreads();
-    float y = W[kOffB3];
+  for (int c = 0; c < kC; ++c) h1[c] = W[kOffB1 + c];
 #pragma unroll
-    for (int tap = 0; tap < kTaps; ++tap) {
-      const int nb = tap_neighbor(n, tap);
-      if (nb >= 0) y = y + R2[tap * kRow + nb];
-    }
-    const double z = di * (rn + s * (double)y);
-    const double res = z - en;
-    const double wn = G ? 0.0 : invNorm[pe.x];
-    // loss: lane values, fixed tree (per-wave halving, waves in order)
-    if (!G) {
-      double l = res * res * wn;
+  for (int q = 0; q < kG; ++q) lds.g[q * kFRow + place] = g[q];
+  add_rows<kG>(Wg, [&](int q) { return g[q]; }, h1);
+  const double s = element_scale(rn, lds.red);  // its barrier also ends the zero fill
+  const double inv = s > 0.0 ? 1.0 / s : 0.0;
+  lds.rh[111 + place] = (float)(rn * inv);
+  __syncthreads();
+  add_rows<kTaps>(Wr, [&](int tap) { return lds.rh[place + tap_place(tap)]; }, h1);
 #pragma unroll
-      for (int h = 32; h >= 1; h >>= 1) l += __shfl_xor(l, h, 64);
-      __syncthreads();
-      if ((n & 63) == 0) s_red[n >> 6] = l;
-      __syncthreads();
-      if (n == 0) {
-        double t = s_red[0];
-        for (int w = 1; w < kP / 64; ++w) t = t + s_red[w];
-        loss = loss + t;
-      }
-    }
-    const float dy = G ? (float)(G[e * kP + n] * di * s) : (float)(2.0 * res * wn * di * s);
-    s_dy[n] = dy;
-    __syncthreads();
-    // dT[tap] = dy at the output node m = n - tap
-    float dT[kTaps];
+  for (int c = 0; c < kC; ++c) h1[c] = h1[c] > 0.f ? h1[c] : 0.f;
+  float h2[kC];
 #pragma unroll
-    for (int tap = 0; tap < kTaps; ++tap) {
-      const int m = tap_neighbor(n, 26 - tap);  // n - delta(tap)
-      dT[tap] = m >= 0 ? s_dy[m] : 0.f;
-    }
-    float dpre2[kC];
+  for (int c = 0; c < kC; ++c) h2[c] = W[kOffB2 + c];
+  add_rows<kC>(W2, [&](int ci) { return h1[ci]; }, h2);
 #pragma unroll
-    for (int c = 0; c < kC; ++c) {
-      float acc = 0.f;
+  for (int c = 0; c < kC; ++c) h2[c] = h2[c] > 0.f ? h2[c] : 0.f;
+  // y = b3 + sum over the taps of T[tap] at node n + tap, nine taps (one dz)
+  // at a time through two halves of the buffer
+  const bool ox[3] = {i > 0, true, i < 7}, oy[3] = {j > 0, true, j < 7}, oz[3] = {k > 0, true, k < 7};
+  float y = W[kOffB3];
 #pragma unroll
-      for (int tap = 0; tap < kTaps; ++tap) acc = __builtin_fmaf(W3[tap * kC + c], dT[tap], acc);
-      dpre2[c] = a.h2[c] > 0.f ? acc : 0.f;
-    }
-    __syncthreads();  // everyone has read T from R2
-#pragma unroll
-    for (int c = 0; c < kC; ++c) R1[c * kRow + n] = a.h2[c];
-#pragma unroll
-    for (int tap = 0; tap < kTaps; ++tap) R2[tap * kRow + n] = dT[tap];
-    __syncthreads();
-    // dW3[tap][c] = sum_n h2[n][c] dT[n][tap]
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int q = n + u * kP;
-      if (q < kTaps * kC) {
-        const int tap = q / kC, c = q % kC;
-        float acc = 0.f;
-        for (int m = 0; m < kP; ++m) acc = __builtin_fmaf(R1[c * kRow + m], R2[tap * kRow + m], acc);
-        gW3[u] = gW3[u] + acc;
-      }
-    }
-    if (n == 0) {
-      float acc = 0.f;
-      for (int m = 0; m < kP; ++m) acc = acc + s_dy[m];
-      gb3 = gb3 + acc;
-    }
+  for (int z = 0; z < 3; ++z) {
+    float* const T = lds.buf + (z & 1) * 9 * kP;
+    dot_rows<9>(W3 + 9 * z * kC, h2, [&](int u, float t) { T[u * kP + n] = t; });
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < kC; ++c) {
-      R1[c * kRow + n] = a.h1[c];
-      R2[c * kRow + n] = dpre2[c];
-    }
-    __syncthreads();
-    // dW2[ci][c] = sum_n h1[n][ci] dpre2[n][c]; db2[c] = sum_n dpre2[n][c]
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int q = n + u * kP;
-      const int ci = q / kC, c = q % kC;
-      float acc = 0.f;
-      for (int m = 0; m < kP; ++m) acc = __builtin_fmaf(R1[ci * kRow + m], R2[c * kRow + m], acc);
-      gW2[u] = gW2[u] + acc;
-    }
-    if (n < kC) {
-      float acc = 0.f;
-      for (int m = 0; m < kP; ++m) acc = acc + R2[n * kRow + m];
-      gb2 = gb2 + acc;
-    }
-    // dpre1 = relu'(h1) (W2 dpre2)
-    float dpre1[kC];
-#pragma unroll
-    for (int ci = 0; ci < kC; ++ci) {
-      float acc = 0.f;
-#pragma unroll
-      for (int c = 0; c < kC; ++c) acc = __builtin_fmaf(W2[ci * kC + c], dpre2[c], acc);
-      dpre1[ci] = a.h1[ci] > 0.f ? acc : 0.f;
-    }
-    __syncthreads();  // R1 (h1) reads done
-#pragma unroll
-    for (int c = 0; c < kC; ++c) R1[c * kRow + n] = dpre1[c];
-    __syncthreads();
-    // dWr[tap][c] = sum_n dpre1[n][c] rh[n+tap]; dWg[q][c] = sum_n dpre1[n][c] g[n][q]; db1
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int q = n + u * kP;
-      if (q < kTaps * kC) {
-        const int tap = q / kC, c = q % kC;
-        float acc = 0.f;
-        for (int m = 0; m < kP; ++m) {
-          const int nb = tap_neighbor(m, tap);
-          if (nb >= 0) acc = __builtin_fmaf(R1[c * kRow + m], s_rh[nb], acc);
-        }
-        gWr[u] = gWr[u] + acc;
-      }
-    }
-    if (n < kG * kC) {
-      const int q = n / kC, c = n % kC;
-      float acc = 0.f;
-      for (int m = 0; m < kP; ++m) acc = __builtin_fmaf(R1[c * kRow + m], s_g[q * kP + m], acc);
-      gWg = gWg + acc;
-    }
-    if (n < kC) {
-      float acc = 0.f;
-      for (int m = 0; m < kP; ++m) acc = acc + R1[n * kRow + m];
-      gb1 = gb1 + acc;
+    for (int u = 0; u < 9; ++u) {
+      const int dx = u % 3, dyy = u / 3;
+      const bool in = ox[dx] && oy[dyy] && oz[z];
+      const int m = n + (dx - 1) + 8 * (dyy - 1) + 64 * (z - 1);
+      const float v = T[u * kP + (in ? m : n)];
+      y = y + (in ? v : 0.f);
     }
   }
-  float* out = partials + (int64_t)blockIdx.x * kNetPartial;
+  const double zz = di * (rn + s * (double)y);
+  const double res = zz - en;
+  const double wn = G ? 0.0 : invNorm[pe.x];
+  const float dy = G ? (float)(G[e * kP + n] * di * s) : (float)(2.0 * res * wn * di * s);
+  lds.dy[111 + place] = dy;
+  // loss: lane values, fixed tree (per-wave halving, waves in order)
+  if (!G) {
+    double v = res * res * wn;
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int q = n + u * kP;
-    if (q < kTaps * kC) {
-      out[kOffW3 + q] = gW3[u];
-      out[kOffWr + q] = gWr[u];
-    }
-    out[kOffW2 + q] = gW2[u];
+    for (int h = 32; h >= 1; h >>= 1) v += __shfl_xor(v, h, 64);
+    if (l == 0) lds.red[wv] = v;
   }
-  if (n < kG * kC) out[kOffWg + n] = gWg;
-  if (n < kC) {
-    out[kOffB1 + n] = gb1;
-    out[kOffB2 + n] = gb2;
-  }
+  __syncthreads();
+  float* const po = out + (int64_t)blockIdx.x * kNetPartial;
   if (n == 0) {
-    out[kOffB3] = gb3;
-    reinterpret_cast<double*>(out + kNetParamsPadded)[0] = loss;
+    double t = 0.0;
+    if (!G) {
+      t = lds.red[0];
+      for (int w = 1; w < kP / 64; ++w) t = t + lds.red[w];
+    }
+    reinterpret_cast<double*>(po + kNetParamsPadded)[0] = t;
+  }
+  // dL/dpre2 = relu'(h2) sum over the taps of W3[tap] dy(n - tap)
+  float d2[kC];
+#pragma unroll
+  for (int c = 0; c < kC; ++c) d2[c] = 0.f;
+  add_rows<kTaps>(W3, [&](int tap) { return lds.dy[place + tap_place(26 - tap)]; }, d2);
+#pragma unroll
+  for (int c = 0; c < kC; ++c) d2[c] = h2[c] > 0.f ? d2[c] : 0.f;
+
+  // the node's column in a 128-node buffer row: inside 16 nodes, 4 s + g is
+  // kept at 4 g + s, so k group g reads the nodes 4 s + g, s = 0..3, at once
+  const int cpos = (n & 0x70) | ((n & 3) << 2) | ((n >> 2) & 3);
+  const int rd = col * kTrainRow + 4 * kg;  // a lane's operand read: row col, group kg
+  // phase 1: waves 0..3 W3, waves 4..7 W2; one (row tile, channel tile) each
+  {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const int rt = (wv >> 1) & 1, ct = wv & 1;
+    const int tap = min(16 * rt + col, kTaps - 1);  // rows past the taps are not stored
+    const float* const ay = lds.dy + tap_place(26 - tap) + kg;
+    for (int h = 0; h < 4; ++h) {
+      __syncthreads();  // the buffer's last readers are done
+      if ((wv >> 1) == h) {
+#pragma unroll
+        for (int c = 0; c < kC; ++c) {
+          lds.buf[c * kTrainRow + cpos] = h2[c];
+          lds.buf[(kC + c) * kTrainRow + cpos] = h1[c];
+          lds.buf[(2 * kC + c) * kTrainRow + cpos] = d2[c];
+        }
+      }
+      __syncthreads();
+      if (wv < 4) {
+        const float* const b = lds.buf + 16 * ct * kTrainRow + rd;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const f32x4 bv = *reinterpret_cast<const f32x4*>(b + 16 * q);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            acc = mfma4(ay[200 * h + 100 * (q / 4) + 10 * ((2 * q + u / 2) % 8) + 4 * (u % 2)], bv[u], acc);
+        }
+      } else {
+        const float* const a = lds.buf + (kC + 16 * rt) * kTrainRow + rd;
+        const float* const b = lds.buf + (2 * kC + 16 * ct) * kTrainRow + rd;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const f32x4 av = *reinterpret_cast<const f32x4*>(a + 16 * q), bv = *reinterpret_cast<const f32x4*>(b + 16 * q);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc = mfma4(av[u], bv[u], acc);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int row = 16 * rt + 4 * kg + u;
+      if (wv >= 4) po[kOffW2 + row * kC + 16 * ct + col] = acc[u];
+      else if (row < kTaps) po[kOffW3 + row * kC + 16 * ct + col] = acc[u];
+    }
+  }
+  // dL/dpre1 = relu'(h1) W2 dL/dpre2, over h2's registers
+  dot_rows<kC>(W2, d2, [&](int ci, float a) { h2[ci] = h1[ci] > 0.f ? a : 0.f; });
+  // phase 2: waves 0..5 the 35 rows of Wr, Wg, b1 (three row tiles), waves 6, 7 b2
+  {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const int rt = wv >> 1, ct = wv & 1;
+    const int row0 = 16 * rt + col;  // this lane's A row
+    const bool one = rt == 3 || row0 >= kTaps + kG;
+    const float* const ax =
+        (row0 < kTaps ? lds.rh + tap_place(row0) : lds.g + (one ? 0 : row0 - kTaps) * kFRow) + kg;
+    float b3 = 0.f;
+    for (int h = 0; h < 4; ++h) {
+      __syncthreads();
+      if ((wv >> 1) == h) {
+#pragma unroll
+        for (int c = 0; c < kC; ++c) {
+          lds.buf[c * kTrainRow + cpos] = h2[c];
+          lds.buf[(kC + c) * kTrainRow + cpos] = d2[c];
+        }
+      }
+      __syncthreads();
+      const float* const b = lds.buf + ((rt == 3 ? kC : 0) + 16 * ct) * kTrainRow + rd;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const f32x4 bv = *reinterpret_cast<const f32x4*>(b + 16 * q);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int at = 200 * h + 100 * (q / 4) + 10 * ((2 * q + u / 2) % 8) + 4 * (u % 2);
+          const float a = one ? 1.f : ax[at];
+          acc = mfma4(a, bv[u], acc);
+          if (wv == 7) {  // b3: nodes in order, beside the products
+            const float* const d = lds.dy + 111 + at;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) b3 = b3 + d[x];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int row = 16 * rt + 4 * kg + u;
+      if (rt == 3) {
+        if (row == 48) po[kOffB2 + 16 * ct + col] = acc[u];
+      } else if (row < kTaps) {
+        po[kOffWr + row * kC + 16 * ct + col] = acc[u];
+      } else if (row < kTaps + kG) {
+        po[kOffWg + (row - kTaps) * kC + 16 * ct + col] = acc[u];
+      } else if (row == kTaps + kG) {
+        po[kOffB1 + 16 * ct + col] = acc[u];
+      }
+    }
+    if (n == kP - 1) po[kOffB3] = b3;
   }
 }
 
-// grad[q] = sum over workgroups (in order) of partials[b][q]; loss likewise
-__global__ __launch_bounds__(256) void k_net_grad_sum(const int32_t nblocks, const float* __restrict__ partials,
-                                                      float* __restrict__ grad, double* __restrict__ loss)
+// partials[b][q]: the sum over chunk b's samples, in order, of the sample
+// gradients (and losses); the samples of this launch are first .. first +
+// count - 1 of the batch, and a chunk begun in an earlier launch goes on from
+// its partial.
+__global__ __launch_bounds__(256) void k_net_chunk_sum(const int32_t first, const int32_t count, const int32_t chunk,
+                                                       const float* __restrict__ grads, float* __restrict__ partials)
+{
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  const int32_t b = first / chunk + (int32_t)blockIdx.y;
+  const int32_t s0 = max(first, (int32_t)((int64_t)b * chunk));
+  const int32_t s1 = (int32_t)min((int64_t)first + count, (int64_t)(b + 1) * chunk);
+  const bool goes_on = s0 != (int64_t)b * chunk;
+  float* const pb = partials + (int64_t)b * kNetPartial;
+  const float* const g = grads + (int64_t)(s0 - first) * kNetPartial;
+  if (q < kNetParams) {
+    float acc = goes_on ? pb[q] : 0.f;
+#pragma unroll 8
+    for (int32_t i = 0; i < s1 - s0; ++i) acc = acc + g[(int64_t)i * kNetPartial + q];
+    pb[q] = acc;
+  } else if (q == kNetParamsPadded) {
+    double acc = goes_on ? reinterpret_cast<const double*>(pb + kNetParamsPadded)[0] : 0.0;
+#pragma unroll 8
+    for (int32_t i = 0; i < s1 - s0; ++i)
+      acc = acc + reinterpret_cast<const double*>(g + (int64_t)i * kNetPartial + kNetParamsPadded)[0];
+    reinterpret_cast<double*>(pb + kNetParamsPadded)[0] = acc;
+  }
+}
+
+// grad[q] = sum over chunks (in order) of partials[b][q]; loss likewise
+// (a serial chain of loads: 32 in flight, 44 -> 12 us for 128 chunks)
+__global__ __launch_bounds__(64) void k_net_grad_sum(const int32_t nblocks, const float* __restrict__ partials,
+                                                     float* __restrict__ grad, double* __restrict__ loss)
 {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q < kNetParams) {
     float acc = 0.f;
-    for (int b = 0; b < nblocks; ++b) acc = acc + partials[(int64_t)b * kNetPartial + q];
+    int b = 0;
+    for (; b + 32 <= nblocks; b += 32) {
+      float t[32];
+#pragma unroll
+      for (int u = 0; u < 32; ++u) t[u] = partials[(int64_t)(b + u) * kNetPartial + q];
+#pragma unroll
+      for (int u = 0; u < 32; ++u) acc = acc + t[u];
+    }
+    for (; b < nblocks; ++b) acc = acc + partials[(int64_t)b * kNetPartial + q];
     grad[q] = acc;
-  }
-  if (q == 0) {
+  } else if (q == kNetParams) {
     double acc = 0.0;
+#pragma unroll 16
     for (int b = 0; b < nblocks; ++b)
       acc = acc + reinterpret_cast<const double*>(partials + (int64_t)b * kNetPartial + kNetParamsPadded)[0];
     *loss = acc;
@@ -406,31 +551,25 @@ int net_apply_launch(int32_t E, const float* W, const float* feat, const double*
   return NBX_SUCCESS;
 }
 
-size_t net_train_lds_bytes()
+// samples first .. first + count - 1 of a batch: their gradients into grads
+// (count rows of kNetPartial), summed into the chunks' partials
+int net_train_launch(int32_t first, int32_t count, int32_t chunk, const int2* samples, int64_t pairStride,
+                     const float* R, const float* Ev, const double* invNorm, const float* W, const float* feat,
+                     const double* invDiag, const double* G, float* grads, float* partials, hipStream_t s)
 {
-  return sizeof(float) * (2 * kC * kRow + kP + kG * kP + kP) + sizeof(double) * (kP / 64);
-}
-
-int net_train_launch(int32_t nsamples, int32_t chunk, const int2* samples, int64_t pairStride, const float* R,
-                     const float* Ev, const double* invNorm, const float* W, const float* feat, const double* invDiag,
-                     const double* G, float* partials, hipStream_t s)
-{
-  const int nblocks = (nsamples + chunk - 1) / chunk;
-  const size_t lds = net_train_lds_bytes();
-  static bool attr_set = false;
-  if (!attr_set) {
-    NBX_HIP(hipFuncSetAttribute((const void*)k_net_train, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr_set = true;
-  }
-  hipLaunchKernelGGL(k_net_train, dim3(nblocks), dim3(kP), lds, s, nsamples, chunk, samples, pairStride, R, Ev,
-                     invNorm, W, feat, invDiag, G, partials);
+  hipLaunchKernelGGL(k_net_train, dim3(count), dim3(kP), 0, s, samples + first, pairStride, R, Ev, invNorm, W, feat,
+                     invDiag, G, grads);
+  NBX_HIP_LAUNCH();
+  const int32_t chunks = (first + count - 1) / chunk - first / chunk + 1;
+  hipLaunchKernelGGL(k_net_chunk_sum, dim3((kNetPartial + 255) / 256, chunks), dim3(256), 0, s, first, count, chunk,
+                     grads, partials);
   NBX_HIP_LAUNCH();
   return NBX_SUCCESS;
 }
 
 int net_grad_sum_launch(int32_t nblocks, const float* partials, float* grad, double* loss, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_net_grad_sum, dim3((kNetParams + 255) / 256), dim3(256), 0, s, nblocks, partials, grad, loss);
+  hipLaunchKernelGGL(k_net_grad_sum, dim3((kNetParams + 1 + 63) / 64), dim3(64), 0, s, nblocks, partials, grad, loss);
   NBX_HIP_LAUNCH();
   return NBX_SUCCESS;
 }
