@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void k_pcg_update_precon_dots(
 // the loads of four nodes, all fields, before their stores, instead of one
 // value's three or four loads per round trip to memory.  The arithmetic and the
 // order of the sums (nodes, then fields) are those of the general loop.
-// 990 elements, N = 9: 40.6 -> 30 us a pass.
+// 990 elements, N = 9: 40.6 -> 31 us a pass.
 constexpr int kUpdateBatch3 = 4;
 
 template <bool JAC, bool FLEX, bool DEG>
