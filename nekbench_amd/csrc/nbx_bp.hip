@@ -310,17 +310,7 @@ __global__ __launch_bounds__(256) void k_pcg_finish_pap(const unsigned int nb, c
   __shared__ double s4[4];
   double v[1];
   combine_partials<1>(v, partials, nb, s4);
-  if (threadIdx.x == 0) {
-    S->pAp = v[0];
-    const double alpha = S->rdotz1 / v[0];  // solve.cpp:104
-    S->alpha = alpha;
-    hist_alpha[S->iter] = alpha;
-    if (!isfinite(alpha)) {
-      S->done = 1;
-      S->breakdown = 1;
-      S->iterations = S->iter - 1;
-    }
-  }
+  if (threadIdx.x == 0) pcg_after_pap(S, v[0], hist_alpha);
 }
 
 // x += alpha p; r -= alpha Ap of the previous iteration (BPUpdatePCG)
@@ -713,14 +703,10 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
                                bp->stream);
     if (rc) return rc;
     prof_mark(bp, kProfAx);  // p = z + beta p, A p and its pAp shares
-    rc = gs_add_mask_launch(bp->ogs, bp->Ap, bp->Nf, bp->fieldOffset, bp->Nmasked, bp->maskIds, &bp->S->done,
-                            bp->stream);
+    rc = gs_add_mask_pap_launch(bp->ogs, bp->Ap, bp->Nf, bp->fieldOffset, bp->Nmasked, bp->maskIds, (unsigned)bp->E,
+                                bp->elem_partials, bp->S, bp->hist_alpha, bp->stream);
     if (rc) return rc;
-    prof_mark(bp, kProfGs);
-    hipLaunchKernelGGL(k_pcg_finish_pap, dim3(1), dim3(256), 0, bp->stream, (unsigned)bp->E, bp->elem_partials, bp->S,
-                       bp->hist_alpha);
-    NBX_HIP_LAUNCH();
-    prof_mark(bp, kProfDot);
+    prof_mark(bp, kProfGs);  // with pAp's finish beside it
     return NBX_SUCCESS;
   }
   hipLaunchKernelGGL(k_pcg_pupdate, grid_for(bp->Nall), dim3(256), 0, bp->stream, bp->Nall, zsrc, bp->p, bp->S);

@@ -18,6 +18,26 @@ struct PcgScalars {
   int learned, fallback, stall_window, fallback_iter;  // learned preconditioner state
   double stall_ratio;
 };
+#ifdef __HIPCC__
+// alpha = rdotz / pAp (nekBone/solve.cpp:104), by the lane that holds the sum
+__device__ __forceinline__ void pcg_after_pap(PcgScalars* S, double pAp, double* hist_alpha)
+{
+  S->pAp = pAp;
+  const double alpha = S->rdotz1 / pAp;
+  S->alpha = alpha;
+  hist_alpha[S->iter] = alpha;
+  if (!isfinite(alpha)) {
+    S->done = 1;
+    S->breakdown = 1;
+    S->iterations = S->iter - 1;
+  }
+}
+#endif
+// gs_add_mask_launch (double, add) of a PCG iteration with pAp's nb partials
+// combined and alpha formed in the same launch; honours S->done
+int gs_add_mask_pap_launch(const nbx_ogs* o, double* v, int k, int32_t stride, int32_t Nmasked,
+                           const int32_t* maskIds, unsigned nb, const double* partials, PcgScalars* S,
+                           double* hist_alpha, hipStream_t s);
 static_assert(offsetof(PcgScalars, done) == offsetof(PcgFlags, done) &&
                   offsetof(PcgScalars, beta) == offsetof(PcgFlags, beta),
               "PcgScalars must start with PcgFlags");

@@ -12,7 +12,7 @@
 // Add/mul start from 0/1 and combine members in ascending order, min/max
 // start from the first member (gatherScatterMany.okl:58-86, 148-176, 300-330,
 // 455-485), so every result is bit-identical to the reference kernel's.
-#include "nbx_internal.h"
+#include "nbx_bp_internal.h"
 #include <hipcub/hipcub.hpp>
 #include <algorithm>
 #include <cmath>
@@ -189,11 +189,10 @@ __device__ __forceinline__ void gs_group_sum(const int32_t* __restrict__ ids, co
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_gs_add_mask(const GsClasses C, const int k, const int32_t stride,
-                                                     T* __restrict__ q, const int* __restrict__ skip)
+__device__ __forceinline__ void gs_add_mask_block(const int32_t block, const GsClasses& C, const int k,
+                                                  const int32_t stride, T* __restrict__ q)
 {
-  if (skip && *skip) return;
-  const int32_t xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int32_t xcd = block & 7, local = block >> 3;
   const int32_t slice = local / C.bstart[5], lb = local - slice * C.bstart[5];
   int c = 0;
   while (c < 5 && lb >= C.bstart[c + 1]) ++c;
@@ -220,6 +219,38 @@ __global__ __launch_bounds__(256) void k_gs_add_mask(const GsClasses C, const in
   if (c == 0) gs_group_sum<T, 2>(C.ids[0], item, k, stride, q);
   else if (c == 1) gs_group_sum<T, 4>(C.ids[1], item, k, stride, q);
   else gs_group_sum<T, 8>(C.ids[2], item, k, stride, q);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_gs_add_mask(const GsClasses C, const int k, const int32_t stride,
+                                                     T* __restrict__ q, const int* __restrict__ skip)
+{
+  if (skip && *skip) return;
+  gs_add_mask_block<T>((int32_t)blockIdx.x, C, k, stride, q);
+}
+
+// The gather-scatter of a PCG iteration with the finish of pAp beside it:
+// the element shares are complete before this launch and alpha is read after
+// it, so one workgroup of it combines them (the tile-partial order) while the
+// others assemble, instead of a one-workgroup kernel of its own (7.2 us of a
+// 487 us iteration at 32768 elements, 4.7 us and a launch at 990).  Workgroups
+// 0..7 are set apart so that the others keep their XCD.
+__global__ __launch_bounds__(256) void k_gs_add_mask_pap(const GsClasses C, const int k, const int32_t stride,
+                                                         double* __restrict__ q, const unsigned nb,
+                                                         const double* __restrict__ partials, PcgScalars* S,
+                                                         double* __restrict__ hist_alpha)
+{
+  if (blockIdx.x == 0) {
+    if (S->done) return;
+    __shared__ double s4[4];
+    double v[1];
+    combine_partials<1, 16>(v, partials, nb, s4);
+    if (threadIdx.x == 0) pcg_after_pap(S, v[0], hist_alpha);
+    return;
+  }
+  // (a breakdown set by workgroup 0 may stop some of the others: nothing reads q then)
+  if (blockIdx.x < 8 || S->done) return;
+  gs_add_mask_block<double>((int32_t)blockIdx.x - 8, C, k, stride, q);
 }
 
 __global__ __launch_bounds__(256) void k_mask(const int32_t Nmasked, const int32_t* __restrict__ maskIds,
@@ -277,13 +308,12 @@ int gs_launch(const nbx_ogs* o, void* v, int k, int32_t stride, nbx_type type, n
   }
 }
 
-template <typename T>
-static int gs_add_mask_launch_t(const nbx_ogs* o, T* v, int k, int32_t stride, int32_t Nmasked,
-                                const int32_t* maskIds, const int* skip, hipStream_t s)
+// the classes' chunks and slices; returns the number of workgroups (0: nothing to do)
+static int64_t gs_classes(const nbx_ogs* o, int32_t Nmasked, const int32_t* maskIds, GsClasses& C)
 {
-  GsClasses C{};
   const int32_t n[5] = {o->Nfix[0], o->Nfix[1], o->Nfix[2], o->Ngen, Nmasked};
   const int32_t* ids[5] = {o->d_fix[0], o->d_fix[1], o->d_fix[2], o->d_ids, maskIds};
+  C.off = o->d_offsets;
   int32_t items = 0;
   for (int c = 0; c < 5; ++c) {
     C.n[c] = n[c];
@@ -291,7 +321,7 @@ static int gs_add_mask_launch_t(const nbx_ogs* o, T* v, int k, int32_t stride, i
     C.ids[c] = ids[c];
     items += C.per[c];
   }
-  if (items == 0) return NBX_SUCCESS;
+  if (items == 0) return 0;
   // slices of about kGsSliceItems items of an XCD's chunk: with pairs of
   // one-field N = 7 elements about 128 elements, whose 512 KB of values the
   // XCD's 4 MB L2 holds while the slice's blocks run
@@ -302,8 +332,29 @@ static int gs_add_mask_launch_t(const nbx_ogs* o, T* v, int k, int32_t stride, i
     C.ps[c] = (C.per[c] + C.nslice - 1) / C.nslice;
     C.bstart[c + 1] = C.bstart[c] + (C.ps[c] + 255) / 256;
   }
-  const int64_t blocks = 8 * (int64_t)C.nslice * C.bstart[5];
+  return 8 * (int64_t)C.nslice * C.bstart[5];
+}
+
+template <typename T>
+static int gs_add_mask_launch_t(const nbx_ogs* o, T* v, int k, int32_t stride, int32_t Nmasked,
+                                const int32_t* maskIds, const int* skip, hipStream_t s)
+{
+  GsClasses C{};
+  const int64_t blocks = gs_classes(o, Nmasked, maskIds, C);
+  if (blocks == 0) return NBX_SUCCESS;
   hipLaunchKernelGGL(k_gs_add_mask<T>, dim3((unsigned)blocks), dim3(256), 0, s, C, k, stride, v, skip);
+  NBX_HIP_LAUNCH();
+  return NBX_SUCCESS;
+}
+
+int gs_add_mask_pap_launch(const nbx_ogs* o, double* v, int k, int32_t stride, int32_t Nmasked,
+                           const int32_t* maskIds, unsigned nb, const double* partials, PcgScalars* S,
+                           double* hist_alpha, hipStream_t s)
+{
+  GsClasses C{};
+  const int64_t blocks = gs_classes(o, Nmasked, maskIds, C);
+  hipLaunchKernelGGL(k_gs_add_mask_pap, dim3((unsigned)(8 + blocks)), dim3(256), 0, s, C, k, stride, v, nb, partials,
+                     S, hist_alpha);
   NBX_HIP_LAUNCH();
   return NBX_SUCCESS;
 }

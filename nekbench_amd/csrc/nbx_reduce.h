@@ -43,7 +43,7 @@ __device__ __forceinline__ void block_sum256(double (&v)[NV], double* s4)
 
 // Second phase: one 256-lane block combines the nb partials of each of the
 // NV values (partials[c*nb + b]) in fixed order; totals end in lane 0 of v.
-template <int NV>
+template <int NV, int kBatch = 32>
 __device__ __forceinline__ void combine_partials(double (&v)[NV], const double* __restrict__ partials,
                                                  unsigned int nb, double* s4)
 {
@@ -51,7 +51,6 @@ __device__ __forceinline__ void combine_partials(double (&v)[NV], const double* 
   for (int c = 0; c < NV; ++c) {
     // loads batched kBatch deep (a single block is latency-bound: 32 deep
     // takes a quarter of the round trips of 8); additions stay in i order
-    constexpr int kBatch = 32;
     double acc = 0.0;
     const double* pc = partials + (size_t)c * nb;
     unsigned int i = threadIdx.x;
