@@ -70,70 +70,12 @@ struct GsOp<T, NBX_MAX> {
   __device__ static T comb(T acc, T b) { return (b > acc) ? b : acc; }
 };
 
+// All classes of a gather-scatter, and the Dirichlet mask of an add, in one
+// launch (three or four launches, each over all the vector's lines, before:
+// smallest label of every node, 20677 elements of N = 7, 57 -> 46 us; a sum over
+// 512 elements of N = 7, three fields, 22 -> 5.7 us).
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own
-// L2.  Renumbering so that XCD x runs the x-th contiguous eighth of the
-// groups keeps neighbouring groups (which share cache lines of the same
-// element faces) in one L2.  The grid is a multiple of 8 blocks.
-__device__ __forceinline__ int32_t xcd_block(int32_t nblocks8)
-{
-  const int32_t per = nblocks8 >> 3;
-  return (int32_t)(blockIdx.x & 7) * per + (int32_t)(blockIdx.x >> 3);
-}
-
-template <typename T, int OP>
-__global__ __launch_bounds__(256) void k_gs_many(const int32_t Ngroups, const int k, const int32_t stride,
-                                                 const int32_t* __restrict__ offsets,
-                                                 const int32_t* __restrict__ ids, T* __restrict__ q,
-                                                 const int* __restrict__ skip)
-{
-  using O = GsOp<T, OP>;
-  const int32_t g = xcd_block(gridDim.x) * blockDim.x + threadIdx.x;
-  if (g >= Ngroups || (skip && *skip)) return;
-  const int32_t s = offsets[g], e = offsets[g + 1];
-  for (int f = 0; f < k; ++f) {
-    T* qf = q + (int64_t)f * stride;
-    T acc = O::first ? qf[ids[s]] : O::init();
-    for (int32_t n = s + (O::first ? 1 : 0); n < e; ++n) acc = O::comb(acc, qf[ids[n]]);
-    for (int32_t n = s; n < e; ++n) qf[ids[n]] = acc;
-  }
-}
-
-// groups of exactly DEG members, members stored contiguously (vector loads)
-template <typename T, int OP, int DEG>
-__global__ __launch_bounds__(256) void k_gs_fixed(const int32_t Ngroups, const int k, const int32_t stride,
-                                                  const int32_t* __restrict__ ids, T* __restrict__ q,
-                                                  const int* __restrict__ skip)
-{
-  using O = GsOp<T, OP>;
-  const int32_t g = xcd_block(gridDim.x) * blockDim.x + threadIdx.x;
-  if (g >= Ngroups || (skip && *skip)) return;
-  int32_t m[DEG];
-  if (DEG == 2) {
-    const int2 v = *reinterpret_cast<const int2*>(ids + (int64_t)g * 2);
-    m[0] = v.x;
-    m[1] = v.y;
-  } else {
-#pragma unroll
-    for (int c = 0; c < DEG / 4; ++c) {
-      const int4 v = *reinterpret_cast<const int4*>(ids + (int64_t)g * DEG + 4 * c);
-      m[4 * c + 0] = v.x;
-      m[4 * c + 1] = v.y;
-      m[4 * c + 2] = v.z;
-      m[4 * c + 3] = v.w;
-    }
-  }
-  for (int f = 0; f < k; ++f) {
-    T* qf = q + (int64_t)f * stride;
-    T acc = O::first ? qf[m[0]] : O::init();
-#pragma unroll
-    for (int n = O::first ? 1 : 0; n < DEG; ++n) acc = O::comb(acc, qf[m[n]]);
-#pragma unroll
-    for (int n = 0; n < DEG; ++n) qf[m[n]] = acc;
-  }
-}
-
-// All classes of a double-add gather-scatter and the Dirichlet mask in one
-// launch.  Every class list (pairs, quads, octets, CSR groups, masked nodes)
+// L2.  Every class list (pairs, quads, octets, CSR groups, masked nodes)
 // is cut into 8 equal chunks, chunk x of every class runs on XCD x (blocks
 // b with b % 8 == x), so one L2 sees the same element range for every class.
 // Each chunk is cut again into S equal slices, and an XCD runs slice s of
@@ -152,14 +94,16 @@ struct GsClasses {
   const int32_t* off;    // CSR offsets
 };
 
-// one group of DEG members (ids[item*DEG ..]): the sum in ascending member
-// order from zero, written back to every member.  DEG is a compile-time
-// constant so that a lane issues the loads of all members before the first
-// use (a run-time count compiled to one load per round trip to memory).
-template <typename T, int DEG>
-__device__ __forceinline__ void gs_group_sum(const int32_t* __restrict__ ids, const int32_t item, const int k,
-                                             const int32_t stride, T* __restrict__ q)
+// one group of DEG members (ids[item*DEG ..]): combined in ascending member
+// order (from the op's identity, or the first member), written back to every
+// member; fields f0, f0 + fs, ...  DEG is a compile-time constant so that a
+// lane issues the loads of all members before the first use (a run-time count
+// compiled to one load per round trip to memory).
+template <typename T, int OP, int DEG>
+__device__ __forceinline__ void gs_group(const int32_t* __restrict__ ids, const int32_t item, const int f0,
+                                         const int fs, const int k, const int32_t stride, T* __restrict__ q)
 {
+  using O = GsOp<T, OP>;
   int32_t m[DEG];
   if (DEG == 2) {
     const int2 v = *reinterpret_cast<const int2*>(ids + (int64_t)item * 2);
@@ -175,23 +119,26 @@ __device__ __forceinline__ void gs_group_sum(const int32_t* __restrict__ ids, co
       m[4 * h + 3] = v.w;
     }
   }
-  for (int f = 0; f < k; ++f) {
+  for (int f = f0; f < k; f += fs) {
     T* qf = q + (int64_t)f * stride;
     T v[DEG];
 #pragma unroll
     for (int n = 0; n < DEG; ++n) v[n] = qf[m[n]];
-    T acc = T(0);
+    T acc = O::first ? v[0] : O::init();
 #pragma unroll
-    for (int n = 0; n < DEG; ++n) acc = acc + v[n];
+    for (int n = O::first ? 1 : 0; n < DEG; ++n) acc = O::comb(acc, v[n]);
 #pragma unroll
     for (int n = 0; n < DEG; ++n) qf[m[n]] = acc;
   }
 }
 
-template <typename T>
-__device__ __forceinline__ void gs_add_mask_block(const int32_t block, const GsClasses& C, const int k,
-                                                  const int32_t stride, T* __restrict__ q)
+// fields blockIdx.y, blockIdx.y + gridDim.y, ...
+template <typename T, int OP>
+__device__ __forceinline__ void gs_block(const int32_t block, const GsClasses& C, const int k, const int32_t stride,
+                                         T* __restrict__ q)
 {
+  using O = GsOp<T, OP>;
+  const int f0 = blockIdx.y, fs = gridDim.y;
   const int32_t xcd = block & 7, local = block >> 3;
   const int32_t slice = local / C.bstart[5], lb = local - slice * C.bstart[5];
   int c = 0;
@@ -202,31 +149,31 @@ __device__ __forceinline__ void gs_add_mask_block(const int32_t block, const GsC
   if (item >= min(C.n[c], xcd * C.per[c] + min(C.per[c], s0 + C.ps[c]))) return;
   if (c == 4) {
     const int32_t id = C.ids[4][item];
-    for (int f = 0; f < k; ++f) q[id + (int64_t)f * stride] = T(0);
+    for (int f = f0; f < k; f += fs) q[id + (int64_t)f * stride] = T(0);
     return;
   }
   if (c == 3) {
     const int32_t s0 = C.off[item], e0 = C.off[item + 1];
     const int32_t* idg = C.ids[3];
-    for (int f = 0; f < k; ++f) {
+    for (int f = f0; f < k; f += fs) {
       T* qf = q + (int64_t)f * stride;
-      T acc = T(0);
-      for (int32_t n = s0; n < e0; ++n) acc = acc + qf[idg[n]];
+      T acc = O::first ? qf[idg[s0]] : O::init();
+      for (int32_t n = s0 + (O::first ? 1 : 0); n < e0; ++n) acc = O::comb(acc, qf[idg[n]]);
       for (int32_t n = s0; n < e0; ++n) qf[idg[n]] = acc;
     }
     return;
   }
-  if (c == 0) gs_group_sum<T, 2>(C.ids[0], item, k, stride, q);
-  else if (c == 1) gs_group_sum<T, 4>(C.ids[1], item, k, stride, q);
-  else gs_group_sum<T, 8>(C.ids[2], item, k, stride, q);
+  if (c == 0) gs_group<T, OP, 2>(C.ids[0], item, f0, fs, k, stride, q);
+  else if (c == 1) gs_group<T, OP, 4>(C.ids[1], item, f0, fs, k, stride, q);
+  else gs_group<T, OP, 8>(C.ids[2], item, f0, fs, k, stride, q);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_gs_add_mask(const GsClasses C, const int k, const int32_t stride,
-                                                     T* __restrict__ q, const int* __restrict__ skip)
+template <typename T, int OP>
+__global__ __launch_bounds__(256) void k_gs(const GsClasses C, const int k, const int32_t stride, T* __restrict__ q,
+                                            const int* __restrict__ skip)
 {
   if (skip && *skip) return;
-  gs_add_mask_block<T>((int32_t)blockIdx.x, C, k, stride, q);
+  gs_block<T, OP>((int32_t)blockIdx.x, C, k, stride, q);
 }
 
 // The gather-scatter of a PCG iteration with the finish of pAp beside it:
@@ -235,13 +182,13 @@ __global__ __launch_bounds__(256) void k_gs_add_mask(const GsClasses C, const in
 // others assemble, instead of a one-workgroup kernel of its own (7.2 us of a
 // 487 us iteration at 32768 elements, 4.7 us and a launch at 990).  Workgroups
 // 0..7 are set apart so that the others keep their XCD.
-__global__ __launch_bounds__(256) void k_gs_add_mask_pap(const GsClasses C, const int k, const int32_t stride,
+__global__ __launch_bounds__(256) void k_gs_pap(const GsClasses C, const int k, const int32_t stride,
                                                          double* __restrict__ q, const unsigned nb,
                                                          const double* __restrict__ partials, PcgScalars* S,
                                                          double* __restrict__ hist_alpha)
 {
   if (blockIdx.x == 0) {
-    if (S->done) return;
+    if (blockIdx.y != 0 || S->done) return;
     __shared__ double s4[4];
     double v[1];
     combine_partials<1, 16>(v, partials, nb, s4);
@@ -250,7 +197,7 @@ __global__ __launch_bounds__(256) void k_gs_add_mask_pap(const GsClasses C, cons
   }
   // (a breakdown set by workgroup 0 may stop some of the others: nothing reads q then)
   if (blockIdx.x < 8 || S->done) return;
-  gs_add_mask_block<double>((int32_t)blockIdx.x - 8, C, k, stride, q);
+  gs_block<double, NBX_ADD>((int32_t)blockIdx.x - 8, C, k, stride, q);
 }
 
 __global__ __launch_bounds__(256) void k_mask(const int32_t Nmasked, const int32_t* __restrict__ maskIds,
@@ -259,53 +206,6 @@ __global__ __launch_bounds__(256) void k_mask(const int32_t Nmasked, const int32
   const int32_t n = blockIdx.x * blockDim.x + threadIdx.x;
   if (skip && *skip) return;
   if (n < Nmasked) q[maskIds[n]] = 0.0;
-}
-
-inline dim3 grid8(int32_t n) { return dim3((unsigned)(((n + 255) / 256 + 7) / 8 * 8)); }
-
-template <typename T, int OP>
-static void gs_launch_op(const nbx_ogs* o, T* v, int k, int32_t stride, const int* skip, hipStream_t s)
-{
-  if (o->Nfix[0])
-    hipLaunchKernelGGL((k_gs_fixed<T, OP, 2>), grid8(o->Nfix[0]), dim3(256), 0, s, o->Nfix[0], k, stride, o->d_fix[0],
-                       v, skip);
-  if (o->Nfix[1])
-    hipLaunchKernelGGL((k_gs_fixed<T, OP, 4>), grid8(o->Nfix[1]), dim3(256), 0, s, o->Nfix[1], k, stride, o->d_fix[1],
-                       v, skip);
-  if (o->Nfix[2])
-    hipLaunchKernelGGL((k_gs_fixed<T, OP, 8>), grid8(o->Nfix[2]), dim3(256), 0, s, o->Nfix[2], k, stride, o->d_fix[2],
-                       v, skip);
-  if (o->Ngen)
-    hipLaunchKernelGGL((k_gs_many<T, OP>), grid8(o->Ngen), dim3(256), 0, s, o->Ngen, k, stride, o->d_offsets, o->d_ids,
-                       v, skip);
-}
-
-template <typename T>
-static int gs_launch_t(const nbx_ogs* o, void* v, int k, int32_t stride, nbx_op op, const int* skip,
-                       hipStream_t s)
-{
-  switch (op) {
-    case NBX_ADD: gs_launch_op<T, NBX_ADD>(o, (T*)v, k, stride, skip, s); break;
-    case NBX_MUL: gs_launch_op<T, NBX_MUL>(o, (T*)v, k, stride, skip, s); break;
-    case NBX_MIN: gs_launch_op<T, NBX_MIN>(o, (T*)v, k, stride, skip, s); break;
-    case NBX_MAX: gs_launch_op<T, NBX_MAX>(o, (T*)v, k, stride, skip, s); break;
-    default: return fail(NBX_ERR_INVALID, "gs: unknown op %d", (int)op);
-  }
-  NBX_HIP_LAUNCH();
-  return NBX_SUCCESS;
-}
-
-int gs_launch(const nbx_ogs* o, void* v, int k, int32_t stride, nbx_type type, nbx_op op, const int* skip,
-              hipStream_t s)
-{
-  if (o->NsharedGather == 0) return NBX_SUCCESS;
-  switch (type) {
-    case NBX_DOUBLE: return gs_launch_t<double>(o, v, k, stride, op, skip, s);
-    case NBX_FLOAT: return gs_launch_t<float>(o, v, k, stride, op, skip, s);
-    case NBX_INT: return gs_launch_t<int32_t>(o, v, k, stride, op, skip, s);
-    case NBX_LONG: return gs_launch_t<long long>(o, v, k, stride, op, skip, s);
-    default: return fail(NBX_ERR_INVALID, "gs: unknown type %d", (int)type);
-  }
 }
 
 // the classes' chunks and slices; returns the number of workgroups (0: nothing to do)
@@ -335,14 +235,58 @@ static int64_t gs_classes(const nbx_ogs* o, int32_t Nmasked, const int32_t* mask
   return 8 * (int64_t)C.nslice * C.bstart[5];
 }
 
+// rows of the grid (fields at a time): the fields in turn by the same lanes,
+// which read the members once, unless that leaves the chip's 2048 lanes a CU
+// unfilled
+static unsigned gs_field_rows(int64_t blocks, int k)
+{
+  return blocks * 256 < 256 * 2048 ? (unsigned)std::max(1, std::min(k, 65535)) : 1u;
+}
+
+template <typename T, int OP>
+static void gs_launch_op(const nbx_ogs* o, T* v, int k, int32_t stride, int32_t Nmasked, const int32_t* maskIds,
+                         const int* skip, hipStream_t s)
+{
+  GsClasses C{};
+  const int64_t blocks = gs_classes(o, Nmasked, maskIds, C);
+  if (blocks == 0) return;
+  hipLaunchKernelGGL((k_gs<T, OP>), dim3((unsigned)blocks, gs_field_rows(blocks, k)), dim3(256), 0, s, C, k, stride, v,
+                     skip);
+}
+
+template <typename T>
+static int gs_launch_t(const nbx_ogs* o, void* v, int k, int32_t stride, nbx_op op, const int* skip,
+                       hipStream_t s)
+{
+  switch (op) {
+    case NBX_ADD: gs_launch_op<T, NBX_ADD>(o, (T*)v, k, stride, 0, nullptr, skip, s); break;
+    case NBX_MUL: gs_launch_op<T, NBX_MUL>(o, (T*)v, k, stride, 0, nullptr, skip, s); break;
+    case NBX_MIN: gs_launch_op<T, NBX_MIN>(o, (T*)v, k, stride, 0, nullptr, skip, s); break;
+    case NBX_MAX: gs_launch_op<T, NBX_MAX>(o, (T*)v, k, stride, 0, nullptr, skip, s); break;
+    default: return fail(NBX_ERR_INVALID, "gs: unknown op %d", (int)op);
+  }
+  NBX_HIP_LAUNCH();
+  return NBX_SUCCESS;
+}
+
+int gs_launch(const nbx_ogs* o, void* v, int k, int32_t stride, nbx_type type, nbx_op op, const int* skip,
+              hipStream_t s)
+{
+  if (o->NsharedGather == 0) return NBX_SUCCESS;
+  switch (type) {
+    case NBX_DOUBLE: return gs_launch_t<double>(o, v, k, stride, op, skip, s);
+    case NBX_FLOAT: return gs_launch_t<float>(o, v, k, stride, op, skip, s);
+    case NBX_INT: return gs_launch_t<int32_t>(o, v, k, stride, op, skip, s);
+    case NBX_LONG: return gs_launch_t<long long>(o, v, k, stride, op, skip, s);
+    default: return fail(NBX_ERR_INVALID, "gs: unknown type %d", (int)type);
+  }
+}
+
 template <typename T>
 static int gs_add_mask_launch_t(const nbx_ogs* o, T* v, int k, int32_t stride, int32_t Nmasked,
                                 const int32_t* maskIds, const int* skip, hipStream_t s)
 {
-  GsClasses C{};
-  const int64_t blocks = gs_classes(o, Nmasked, maskIds, C);
-  if (blocks == 0) return NBX_SUCCESS;
-  hipLaunchKernelGGL(k_gs_add_mask<T>, dim3((unsigned)blocks), dim3(256), 0, s, C, k, stride, v, skip);
+  gs_launch_op<T, NBX_ADD>(o, v, k, stride, Nmasked, maskIds, skip, s);
   NBX_HIP_LAUNCH();
   return NBX_SUCCESS;
 }
@@ -353,8 +297,8 @@ int gs_add_mask_pap_launch(const nbx_ogs* o, double* v, int k, int32_t stride, i
 {
   GsClasses C{};
   const int64_t blocks = gs_classes(o, Nmasked, maskIds, C);
-  hipLaunchKernelGGL(k_gs_add_mask_pap, dim3((unsigned)(8 + blocks)), dim3(256), 0, s, C, k, stride, v, nb, partials,
-                     S, hist_alpha);
+  hipLaunchKernelGGL(k_gs_pap, dim3((unsigned)(8 + blocks), gs_field_rows(blocks, k)), dim3(256), 0, s, C, k, stride,
+                     v, nb, partials, S, hist_alpha);
   NBX_HIP_LAUNCH();
   return NBX_SUCCESS;
 }
