@@ -17,6 +17,9 @@
 //   3. Ap = axhelm(p)                          (BPAxOperator: kernel)
 //   4. Ap = gs(Ap), Ap[mask] = 0               (BPAxOperator: oogs::start/finish; mask)
 //   5. pAp = <p,Ap>_w, one-block finish: alpha = rdotz/pAp (BPWeightedInnerProduct)
+// With the fused operator the shares of pAp come from pass 3 and the finish of
+// 5 runs beside 4.  Multigrid and learned preconditioners: the update, <r,r>_w
+// and the stopping test, then z = M r, then the other dots.
 // Moving the update into the next iteration's first pass changes no value:
 // every element-wise operation is the same single fma in the same order.
 // The dots use the fixed reduction tree of nbx_reduce.h.  The CPU oracle
@@ -35,20 +38,18 @@ namespace nbx {
 
 
 
-__device__ __forceinline__ void pcg_after_dots(PcgScalars* S, double rdotz, double rdotr, double zdotAp,
-                                               double* hist_rdotr)
+// First half of an iteration's scalars: |r|^2 of the updated residual, TOL and
+// the stopping test.  Returns false where the solve ends here.
+__device__ __forceinline__ bool pcg_after_rr(PcgScalars* S, double rdotr, double* hist_rdotr)
 {
   const int it = S->iter + 1;
   S->iter = it;
   if (it > S->maxit) {  // loop end (solve.cpp:76); the last update has been applied
     S->done = 1;
     S->iterations = S->maxit;
-    return;
+    return false;
   }
-  S->rdotz2 = S->rdotz1;
-  S->rdotz1 = rdotz;
   S->rdotr = rdotr;
-  S->zdotAp = zdotAp;
   hist_rdotr[it] = rdotr;
   if (it == 1) {
     S->rdotr0 = rdotr;
@@ -58,19 +59,29 @@ __device__ __forceinline__ void pcg_after_dots(PcgScalars* S, double rdotz, doub
     S->done = 1;
     S->breakdown = 1;
     S->iterations = it - 1;
-    return;
+    return false;
   }
   if (rdotr <= S->TOL && !S->fixed) {  // solve.cpp:90
     S->done = 1;
     S->converged = 1;
     S->iterations = it - 1;
-    return;
+    return false;
   }
+  return true;
+}
+
+// Second half: beta from <r,z> (and <z,Ap>)
+__device__ __forceinline__ void pcg_after_rz(PcgScalars* S, double rdotz, double zdotAp, const double* hist_rdotr)
+{
+  const int it = S->iter;
+  S->rdotz2 = S->rdotz1;
+  S->rdotz1 = rdotz;
+  S->zdotAp = zdotAp;
   // learned preconditioner: Jacobi from the next iteration on when the
   // residual has not fallen below stall_ratio of its value stall_window
   // iterations ago (plain Jacobi PCG is the fallback)
   if (S->learned && !S->fallback && it > S->stall_window &&
-      !(rdotr <= S->stall_ratio * hist_rdotr[it - S->stall_window])) {
+      !(S->rdotr <= S->stall_ratio * hist_rdotr[it - S->stall_window])) {
     S->fallback = 1;
     S->fallback_iter = it;
   }
@@ -78,6 +89,12 @@ __device__ __forceinline__ void pcg_after_dots(PcgScalars* S, double rdotz, doub
     S->beta = -S->alpha * S->zdotAp / S->rdotz2;  // solve.cpp:92-95
   else
     S->beta = (it == 1) ? 0.0 : S->rdotz1 / S->rdotz2;  // solve.cpp:97
+}
+
+__device__ __forceinline__ void pcg_after_dots(PcgScalars* S, double rdotz, double rdotr, double zdotAp,
+                                               double* hist_rdotr)
+{
+  if (pcg_after_rr(S, rdotr, hist_rdotr)) pcg_after_rz(S, rdotz, zdotAp, hist_rdotr);
 }
 
 // nodes per lane whose loads the update pass issues together
@@ -313,21 +330,89 @@ __global__ __launch_bounds__(256) void k_pcg_finish_pap(const unsigned int nb, c
   if (threadIdx.x == 0) pcg_after_pap(S, v[0], hist_alpha);
 }
 
-// x += alpha p; r -= alpha Ap of the previous iteration (BPUpdatePCG)
-__global__ __launch_bounds__(256) void k_pcg_update(const int64_t Nall, const double* __restrict__ p,
-                                                    const double* __restrict__ Ap, double* __restrict__ x,
-                                                    double* __restrict__ r, const PcgScalars* S)
+// Multigrid and learned preconditioners: x += alpha p, r -= alpha Ap of the
+// previous iteration (BPUpdatePCG) and the tile partials of <r,r>_w, so that
+// the stopping test comes before the preconditioner: the cycle of the
+// iteration that has converged is not run (one of ten at 32768 elements,
+// 1e-8).  Each lane issues the loads of four nodes and a field together.
+template <bool DEG>
+__global__ __launch_bounds__(256) void k_pcg_update_rr(const int32_t N, const int32_t offset, const int Nf,
+                                                       const double* __restrict__ w, const uint8_t* __restrict__ deg,
+                                                       const double* __restrict__ p, const double* __restrict__ Ap,
+                                                       double* __restrict__ x, double* __restrict__ r,
+                                                       double* __restrict__ partials, const PcgScalars* S)
 {
-  if (S->done || S->iter == 0) return;
+  if (S->done) return;
+  const bool update = S->iter > 0;
   const double alpha = S->alpha;
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n < Nall) {
-    x[n] = __builtin_fma(alpha, ldnt(&p[n]), ldnt(&x[n]));
-    r[n] = __builtin_fma(-alpha, ldnt(&Ap[n]), ldnt(&r[n]));
+  constexpr int kB = 4;
+  __shared__ double s4[4];
+  double v[1] = {0.0};
+  const int32_t b0 = (int32_t)blockIdx.x * kRedTile + (int32_t)threadIdx.x;
+#pragma unroll 1
+  for (int h = 0; h < kRedPerLane; h += kB) {
+    double wi[kB], rn[kB][3];
+#pragma unroll
+    for (int u = 0; u < kB; ++u) {
+      const int32_t id = b0 + (h + u) * kRedLanes;
+      const int32_t at = id < N ? id : 0;
+      wi[u] = DEG ? (double)deg[at] : ldnt(&w[at]);
+    }
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      if (f >= Nf) break;
+      const int64_t o = (int64_t)f * offset;
+      double rr[kB], ap[kB], pp[kB], xx[kB];
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const int32_t id = b0 + (h + u) * kRedLanes;
+        const int64_t at = o + (id < N ? id : 0);  // a lane past the end neither stores nor adds
+        rr[u] = ldnt(&r[at]);
+        ap[u] = ldnt(&Ap[at]);
+        pp[u] = ldnt(&p[at]);
+        xx[u] = ldnt(&x[at]);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the loads above are issued before the first store
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const int32_t id = b0 + (h + u) * kRedLanes;
+        rn[u][f] = update ? __builtin_fma(-alpha, ap[u], rr[u]) : rr[u];
+        if (update && id < N) {
+          stnt(__builtin_fma(alpha, pp[u], xx[u]), &x[o + id]);
+          r[o + id] = rn[u][f];  // read again by the preconditioner
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kB; ++u) {
+      if (b0 + (h + u) * kRedLanes >= N) continue;
+      if (DEG) wi[u] = 1.0 / wi[u];  // weight<true>: the same IEEE division
+#pragma unroll
+      for (int f = 0; f < 3; ++f)
+        if (f < Nf) v[0] = __builtin_fma(wi[u] * rn[u][f], rn[u][f], v[0]);
+    }
+  }
+  block_sum256<1>(v, s4);
+  store_partials<1>(v, partials);
+}
+
+// |r|^2, TOL and the stopping test; `host` (pinned) receives the done flag
+__global__ __launch_bounds__(256) void k_pcg_finish_rr(const unsigned int nb, const double* __restrict__ partials,
+                                                       PcgScalars* S, double* __restrict__ hist_rdotr, int* host)
+{
+  __shared__ double s4[4];
+  if (!S->done) {
+    double v[1];
+    combine_partials<1>(v, partials, nb, s4);
+    if (threadIdx.x == 0) (void)pcg_after_rr(S, v[0], hist_rdotr);
+  }
+  if (threadIdx.x == 0) {
+    *host = S->done;
+    __threadfence_system();
   }
 }
 
-// tile partials of <r,z>_w, <r,r>_w, <z,Ap>_w for a given (assembled) z
+// tile partials of <r,z>_w and <z,Ap>_w for a given (assembled) z
 template <bool DEG>
 __global__ __launch_bounds__(256) void k_pcg_dots_z(const int32_t N, const int32_t offset, const int Nf,
                                                     const double* __restrict__ w, const uint8_t* __restrict__ deg,
@@ -336,8 +421,8 @@ __global__ __launch_bounds__(256) void k_pcg_dots_z(const int32_t N, const int32
                                                     const PcgScalars* S)
 {
   if (S->done) return;
-  __shared__ double s4[3 * 4];
-  double v[3] = {0.0, 0.0, 0.0};
+  __shared__ double s4[2 * 4];
+  double v[2] = {0.0, 0.0};
   const int64_t b0 = (int64_t)blockIdx.x * kRedTile + threadIdx.x;
 #pragma unroll
   for (int u = 0; u < kRedPerLane; ++u) {
@@ -349,13 +434,22 @@ __global__ __launch_bounds__(256) void k_pcg_dots_z(const int32_t N, const int32
         const double rf = ldnt(&r[iid]);
         const double zf = ldnt(&z[iid]);
         v[0] = __builtin_fma(wid * rf, zf, v[0]);
-        v[1] = __builtin_fma(wid * rf, rf, v[1]);
-        v[2] = __builtin_fma(wid * zf, ldnt(&Ap[iid]), v[2]);
+        v[1] = __builtin_fma(wid * zf, ldnt(&Ap[iid]), v[1]);
       }
     }
   }
-  block_sum256<3>(v, s4);
-  store_partials<3>(v, partials);
+  block_sum256<2>(v, s4);
+  store_partials<2>(v, partials);
+}
+
+__global__ __launch_bounds__(256) void k_pcg_finish_rz(const unsigned int nb, const double* __restrict__ partials,
+                                                       PcgScalars* S, const double* __restrict__ hist_rdotr)
+{
+  if (S->done) return;
+  __shared__ double s4[2 * 4];
+  double v[2];
+  combine_partials<2>(v, partials, nb, s4);
+  if (threadIdx.x == 0) pcg_after_rz(S, v[0], v[1], hist_rdotr);
 }
 
 // vecInv (nekBone/kernel/utils.okl:605-613)
@@ -406,6 +500,7 @@ static void bp_release(nbx_bp* bp)
   if (bp->hist_rdotr) (void)hipFree(bp->hist_rdotr);
   if (bp->hist_alpha) (void)hipFree(bp->hist_alpha);
   for (hipEvent_t ev : bp->prof_ev) (void)hipEventDestroy(ev);
+  if (bp->ev_test) (void)hipEventDestroy(bp->ev_test);
   if (bp->ev0) (void)hipEventDestroy(bp->ev0);
   if (bp->ev1) (void)hipEventDestroy(bp->ev1);
   bp->red.release();
@@ -526,6 +621,7 @@ static int bp_setup_impl(nbx_bp* bp)
   if ((rc = bp->red.init(bp->Nlocal, 3))) return rc;
   NBX_HIP(hipMalloc(&bp->S, sizeof(PcgScalars)));
   NBX_HIP(hipHostMalloc((void**)&bp->hS, sizeof(PcgScalars), hipHostMallocDefault));
+  NBX_HIP(hipEventCreateWithFlags(&bp->ev_test, hipEventDisableTiming));
   NBX_HIP(hipEventCreate(&bp->ev0));
   NBX_HIP(hipEventCreate(&bp->ev1));
   NBX_HIP(hipStreamSynchronize(bp->stream));
@@ -631,11 +727,20 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
   const uint8_t* deg = ogs_degree(bp->ogs);
   const double* zsrc = jac ? bp->z : r;
   if (o.precon == NBX_PRECON_LEARNED || o.precon == NBX_PRECON_MG) {
-    // update; z = M r (learned: gs(w invDiag (r + s f(r))), Jacobi after a
-    // stall; multigrid: one V-cycle); dots; finish
-    hipLaunchKernelGGL(k_pcg_update, grid_for(bp->Nall), dim3(256), 0, bp->stream, bp->Nall, bp->p, bp->Ap, x, r,
-                       bp->S);
+    // update and stopping test; z = M r (learned: gs(w invDiag (r + s f(r))),
+    // Jacobi after a stall; multigrid: one V-cycle); dots; finish
+    if (deg)
+      hipLaunchKernelGGL(k_pcg_update_rr<true>, dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, bp->fieldOffset,
+                         bp->Nf, w, deg, bp->p, bp->Ap, x, r, bp->red.partials, bp->S);
+    else
+      hipLaunchKernelGGL(k_pcg_update_rr<false>, dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, bp->fieldOffset,
+                         bp->Nf, w, deg, bp->p, bp->Ap, x, r, bp->red.partials, bp->S);
     prof_mark(bp, kProfUpdate);
+    hipLaunchKernelGGL(k_pcg_finish_rr, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
+                       bp->hist_rdotr, &bp->hS->done);
+    NBX_HIP_LAUNCH();
+    prof_mark(bp, kProfDot);
+    NBX_HIP(hipEventRecord(bp->ev_test, bp->stream));
     int rc;
     if (o.precon == NBX_PRECON_MG) {
       if ((rc = mg_apply(bp, r, bp->z, &bp->S->done))) return rc;
@@ -652,7 +757,7 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
     else
       hipLaunchKernelGGL(k_pcg_dots_z<false>, dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, bp->fieldOffset,
                          bp->Nf, w, deg, r, bp->z, bp->Ap, bp->red.partials, bp->S);
-    hipLaunchKernelGGL(k_pcg_finish_dots<3>, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
+    hipLaunchKernelGGL(k_pcg_finish_rz, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
                        bp->hist_rdotr);
     NBX_HIP_LAUNCH();
     prof_mark(bp, kProfDot);
@@ -789,15 +894,22 @@ static int bp_pcg_core(nbx_bp* bp, const double* lambda, double* r, double* x, d
     return rc;  // solve.cpp:72
   prof_mark(bp, kProfPreco);  // updateJacobi is timed as "preco" (solve.cpp:71-73)
   // iterations in chunks; the device flag ends the work, the host only polls
-  // each poll is a host wait; a multigrid iteration is long, so it is polled
-  // more often (the kernels of iterations past convergence exit at once)
-  const int chunk = bp->opt.precon == NBX_PRECON_MG ? 4 : 16;
+  // (each poll is a host wait).  A multigrid iteration is long and tests for
+  // the end before its cycle: the host enqueues one, waits for its test and
+  // enqueues the next while the cycle runs, so the kernels past the end (which
+  // exit at once, 0.4 ms a cycle of 32768 elements) are one cycle's.
+  const bool early = bp->opt.precon == NBX_PRECON_MG;
+  const int chunk = early ? 1 : 16;
   int enqueued = 0;
   for (;;) {
     const int n = std::min(chunk, maxit + 1 - enqueued);
     for (int c = 0; c < n; ++c)
       if ((rc = bp_enqueue_iteration(bp, lambda, r, x))) return rc;
     enqueued += n;
+    if (early && enqueued <= maxit) {
+      NBX_HIP(hipEventSynchronize(bp->ev_test));
+      if (!*(volatile int*)&bp->hS->done) continue;
+    }
     NBX_HIP(hipMemcpyAsync(bp->hS, bp->S, sizeof(PcgScalars), hipMemcpyDeviceToHost, bp->stream));
     NBX_HIP(hipStreamSynchronize(bp->stream));
     if ((rc = prof_collect(bp))) return rc;
