@@ -41,9 +41,14 @@
 #include "nbx_bp_internal.h"
 #include "nbx_axhelm_impl.h"
 #include "nbx_blas.h"
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
+
+namespace nbx {
+constexpr int kMgHeld = 8;  // smoothing directions a level holds before its solution takes them up
+}
 
 struct nbx_mg_level {
   nbx_bp* bp = nullptr;  // level 0: the solver's handle (not owned)
@@ -53,7 +58,8 @@ struct nbx_mg_level {
   std::vector<double> c1, c2;  // Chebyshev step coefficients
   // vectors of the cycle's precision (double or float); the last level's r
   // and x are double (its PCG); level 0 reads r and writes x of the solver
-  void *r = nullptr, *x = nullptr, *res = nullptr, *d = nullptr, *Ad = nullptr;
+  void *r = nullptr, *x = nullptr, *res = nullptr, *Ad = nullptr;
+  void* d[nbx::kMgHeld + 1] = {};  // directions (those held and the one being formed)
   double* J = nullptr;  // [Nq][Nq of level l+1]: interpolation from the next coarser level
   float* J32 = nullptr;
   float* invD32 = nullptr;  // FP32 Jacobi diagonal (FP32 / bf16 cycles)
@@ -99,18 +105,31 @@ __device__ __forceinline__ double fmaV<double>(double a, double b, double c) { r
 template <>
 __device__ __forceinline__ float fmaV<float>(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
+// Directions of a cycle that its solution has not taken up yet, in order.
+// x is not read and written at every smoothing step: each step leaves its
+// direction in a buffer of its own, and the last one (or one that would exceed
+// kHeld buffers) adds them all, x = ((x + d_1) + d_2) + ... as the steps would
+// have.  Per node and FP32 cycle of degree 3 with an FP64 x: 104 bytes of x and
+// 8 of the last residual and direction become 32.
+constexpr int kHeld = kMgHeld;
+template <typename V>
+struct Held {
+  const V* d[kHeld];
+  int n;
+  int started;  // x holds earlier directions
+};
+
 // Chebyshev-Jacobi step (n local nodes per field, fields at stride offset,
-// blockIdx.y = field, one Jacobi diagonal for all fields), arithmetic in V; the
-// level's right-hand side is R, its solution X (level 0: the solver's FP64
-// residual and correction):
-//   MODE 0 (first pre-smoothing step, x = 0):  res = (V)r; d = c2 D^-1 res; x = d
-//   MODE 1 (general step):  res -= Ad; d = c1 d + c2 D^-1 res; x += d
-//   MODE 2 (first post-smoothing step):  res -= Ad; d = c2 D^-1 res; x += d
-template <int MODE, typename V, typename R, typename X>
+// blockIdx.y = field, one Jacobi diagonal for all fields), arithmetic in V;
+// dp is the previous direction, d the new one:
+//   MODE 0 (first pre-smoothing step, x = 0):  res = (V)r; d = c2 D^-1 res
+//   MODE 1 (general step):  res -= Ad; d = c1 dp + c2 D^-1 res
+//   MODE 2 (first post-smoothing step):  res -= Ad; d = c2 D^-1 res
+template <int MODE, typename V, typename R>
 __global__ __launch_bounds__(256) void k_cheb(const int32_t n, const int32_t offset, const V c1, const V c2,
                                               const V* __restrict__ invD, const R* __restrict__ r,
-                                              V* __restrict__ res, const V* __restrict__ Ad, V* __restrict__ d,
-                                              X* __restrict__ x, const int* __restrict__ skip)
+                                              V* __restrict__ res, const V* __restrict__ Ad, const V* dp, V* d,
+                                              const int* __restrict__ skip)
 {
   if (skip && *skip) return;
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;  // node; blockIdx.y = field
@@ -121,9 +140,38 @@ __global__ __launch_bounds__(256) void k_cheb(const int32_t n, const int32_t off
   else ri = res[id] - Ad[id];
   res[id] = ri;
   const V t = c2 * (invD[i] * ri);
-  const V di = (MODE == 1) ? fmaV<V>(c1, d[id], t) : t;
-  d[id] = di;
-  x[id] = (MODE == 0) ? (X)di : x[id] + (X)di;
+  d[id] = (MODE == 1) ? fmaV<V>(c1, dp[id], t) : t;
+}
+
+// The same step (MODE 1 or 2), its direction and the held ones added to the
+// level's solution; res and d are stored where KEEP (a step follows).
+template <int MODE, typename V, typename X, bool KEEP>
+__global__ __launch_bounds__(256) void k_cheb_sum(const int32_t n, const int32_t offset, const V c1, const V c2,
+                                                  const V* __restrict__ invD, V* __restrict__ res,
+                                                  const V* __restrict__ Ad, const V* dp, V* d, const Held<V> H,
+                                                  X* __restrict__ x, const int* __restrict__ skip)
+{
+  if (skip && *skip) return;
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t id = (int64_t)blockIdx.y * offset + i;
+  const V rv = res[id], av = Ad[id], iv = invD[i], pv = MODE == 1 ? dp[id] : V(0);
+  V h[kHeld];
+#pragma unroll
+  for (int q = 0; q < kHeld; ++q)
+    if (q < H.n) h[q] = H.d[q][id];
+  X xv = H.started ? x[id] : X(0);
+  const V ri = rv - av;
+  const V t = c2 * (iv * ri);
+  const V di = (MODE == 1) ? fmaV<V>(c1, pv, t) : t;
+#pragma unroll
+  for (int q = 0; q < kHeld; ++q)
+    if (q < H.n) xv = (q == 0 && !H.started) ? (X)h[q] : xv + (X)h[q];
+  x[id] = (H.n == 0 && !H.started) ? (X)di : xv + (X)di;
+  if (KEEP) {
+    res[id] = ri;
+    d[id] = di;
+  }
 }
 
 // Restriction of one element: res -= Ad (stored), u = w res, then
@@ -182,12 +230,12 @@ __global__ __launch_bounds__(256) void k_mg_restrict(const int nqf, const int nq
 }
 
 // Prolongation of one element: v[i,j,k] = sum_c J[k][c] sum_b J[j][b] sum_a J[i][a] xc[a,b,c];
-// d = v, x += v.
-template <typename V, typename I, typename X, int NQF = 0, int NQC = 0>
+// d = v (x takes it up with the held directions).
+template <typename V, typename I, int NQF = 0, int NQC = 0>
 __global__ __launch_bounds__(256) void k_mg_prolong(const int nqf, const int nqc, const int32_t offf,
                                                     const int32_t offc, const V* __restrict__ J,
                                                     const I* __restrict__ xc, V* __restrict__ d,
-                                                    X* __restrict__ x, const int* __restrict__ skip)
+                                                    const int* __restrict__ skip)
 {
   if (skip && *skip) return;
   __shared__ V s_u[12 * 12 * 12];
@@ -221,9 +269,7 @@ __global__ __launch_bounds__(256) void k_mg_prolong(const int nqf, const int nqc
     const int ij = q % (Nqf * Nqf), k = q / (Nqf * Nqf);
     V acc = V(0);
     for (int c = 0; c < Nqc; ++c) acc = fmaV<V>(s_J[k * Nqc + c], s_u[ij + Nqf * Nqf * c], acc);
-    const int64_t id = fo + e * Npf + q;
-    d[id] = acc;
-    x[id] = x[id] + (X)acc;
+    d[fo + e * Npf + q] = acc;
   }
 }
 
@@ -736,17 +782,60 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
   const dim3 ge((unsigned)bp->E, (unsigned)bp->Nf);
   const int k = mg->degree;
   V* res = static_cast<V*>(L.res);
-  V* d = static_cast<V*>(L.d);
   V* Ad = static_cast<V*>(L.Ad);
   const V* invD = level_invD<V>(L);
   int rc;
+  // the direction last formed; `next` forms the following one in a free buffer
+  Held<V> H{};
+  V* d = static_cast<V*>(L.d[0]);
+  int used = 0;
+  auto hold = [&](V* dn) {
+    d = dn;
+    H.d[H.n++] = dn;
+  };
+  auto free_buffer = [&]() { return static_cast<V*>(L.d[used++]); };
+  // one smoothing step after level_apply of d; `last`: nothing reads res and d
+  // after it (the learned step does)
+  auto smooth = [&](int s, bool post, bool last) {
+    const bool first_post = post && s == 0;
+    const V c1 = first_post ? V(0) : (V)L.c1[s], c2 = (V)L.c2[s];
+    if (last || H.n >= (post ? kHeld : kHeld - 1)) {  // before the coarse correction one stays free for it
+#define NBX_SUM(MODE, KEEP)                                                                                         \
+  hipLaunchKernelGGL((k_cheb_sum<MODE, V, X, KEEP>), g, b, 0, bp->stream, n, off, c1, c2, invD, res, Ad, d, d, H, x, \
+                     skip)
+      const bool keep = !last || (l == 0 && mg->learned);
+      if (first_post) {
+        if (keep) NBX_SUM(2, true);
+        else NBX_SUM(2, false);
+      } else {
+        if (keep) NBX_SUM(1, true);
+        else NBX_SUM(1, false);
+      }
+#undef NBX_SUM
+      H.n = 0;
+      H.started = 1;
+      // the held buffers are free again, all but the one d sits in
+      std::swap(L.d[0], *std::find(L.d, L.d + kHeld + 1, static_cast<void*>(d)));
+      used = 1;
+      return;
+    }
+    V* dn = free_buffer();
+    if (first_post)
+      hipLaunchKernelGGL((k_cheb<2, V, R>), g, b, 0, bp->stream, n, off, c1, c2, invD, (const R*)nullptr, res, Ad, d, dn,
+                         skip);
+    else
+      hipLaunchKernelGGL((k_cheb<1, V, R>), g, b, 0, bp->stream, n, off, c1, c2, invD, (const R*)nullptr, res, Ad, d, dn,
+                         skip);
+    hold(dn);
+  };
   // pre-smoothing from x = 0
-  hipLaunchKernelGGL((k_cheb<0, V, R, X>), g, b, 0, bp->stream, n, off, V(0), (V)L.c2[0], invD, r, res,
-                     (const V*)nullptr, d, x, skip);
+  V* d0 = free_buffer();
+  hipLaunchKernelGGL((k_cheb<0, V, R>), g, b, 0, bp->stream, n, off, V(0), (V)L.c2[0], invD, r, res, (const V*)nullptr,
+                     (const V*)nullptr, d0, skip);
+  hold(d0);
   for (int s = 1; s < k; ++s) {
     if ((rc = level_apply(mg, L, d, Ad, skip))) return rc;
-    hipLaunchKernelGGL((k_cheb<1, V, R, X>), g, b, 0, bp->stream, n, off, (V)L.c1[s], (V)L.c2[s], invD,
-                       (const R*)nullptr, res, Ad, d, x, skip);
+    smooth(s, false, false);
   }
   if ((rc = level_apply(mg, L, d, Ad, skip))) return rc;
   // restriction of the smoothed residual
@@ -769,9 +858,10 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
     return rc;
   if ((rc = vcycle<V>(mg, l + 1, C.r, C.x, skip))) return rc;
   // coarse correction
+  V* v = free_buffer();
 #define NBX_PROLONG(F, C_)                                                                                 \
-  hipLaunchKernelGGL((k_mg_prolong<V, CV, X, F, C_>), ge, b, 0, bp->stream, L.Nq, C.Nq, off, C.bp->fieldOffset, \
-                     level_J<V>(L), static_cast<const CV*>(C.x), d, x, skip)
+  hipLaunchKernelGGL((k_mg_prolong<V, CV, F, C_>), ge, b, 0, bp->stream, L.Nq, C.Nq, off, C.bp->fieldOffset, \
+                     level_J<V>(L), static_cast<const CV*>(C.x), v, skip)
   if (L.Nq == 8 && C.Nq == 4) NBX_PROLONG(8, 4);
   else if (L.Nq == 4 && C.Nq == 2) NBX_PROLONG(4, 2);
   else if (L.Nq == 10 && C.Nq == 5) NBX_PROLONG(10, 5);
@@ -779,14 +869,11 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
   else NBX_PROLONG(0, 0);
 #undef NBX_PROLONG
   NBX_HIP_LAUNCH();
-  if ((rc = level_apply(mg, L, d, Ad, skip))) return rc;
+  hold(v);
   // post-smoothing
-  hipLaunchKernelGGL((k_cheb<2, V, R, X>), g, b, 0, bp->stream, n, off, V(0), (V)L.c2[0], invD, (const R*)nullptr, res,
-                     Ad, d, x, skip);
-  for (int s = 1; s < k; ++s) {
+  for (int s = 0; s < k; ++s) {
     if ((rc = level_apply(mg, L, d, Ad, skip))) return rc;
-    hipLaunchKernelGGL((k_cheb<1, V, R, X>), g, b, 0, bp->stream, n, off, (V)L.c1[s], (V)L.c2[s], invD,
-                       (const R*)nullptr, res, Ad, d, x, skip);
+    smooth(s, true, s + 1 == k);
   }
   NBX_HIP_LAUNCH();
   if constexpr (std::is_same<X, double>::value) {  // the fine level (its correction is FP64)
@@ -979,9 +1066,11 @@ extern "C" int nbx_bp_mg_setup(nbx_bp* bp, int nlevels, const int* orders, int d
     nbx_bp* b = L.bp;
     if ((rc = bp_update_jacobi(b, b->lambda))) break;
     const bool last = l + 1 == nlevels;
-    if (!last && ((rc = mg_alloc(mg, &L.res, b->Nall, es)) || (rc = mg_alloc(mg, &L.d, b->Nall, es)) ||
-                  (rc = mg_alloc(mg, &L.Ad, b->Nall, es))))
-      break;
+    if (!last && ((rc = mg_alloc(mg, &L.res, b->Nall, es)) || (rc = mg_alloc(mg, &L.Ad, b->Nall, es)))) break;
+    // a cycle's directions before the last: 2 degree, or kMgHeld and the one being formed
+    for (int q = 0; !last && q < std::min(2 * degree, kMgHeld + 1) && rc == NBX_SUCCESS; ++q)
+      rc = mg_alloc(mg, &L.d[q], b->Nall, es);
+    if (rc) break;
     if (l > 0 && ((rc = mg_alloc(mg, &L.r, b->Nall, last ? sizeof(double) : es)) ||
                   (rc = mg_alloc(mg, &L.x, b->Nall, last ? sizeof(double) : es))))
       break;
