@@ -28,9 +28,10 @@ int axhelm_dispatch_f64(int N, int Nf, int bk, bool partial, int32_t Nelements, 
 
 int axhelm_pcg_dispatch_f64(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                             const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                            double* partials, const PcgFlags* S, hipStream_t s)
+                            double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s)
 {
-  return axhelm_pcg_launch_t<double, double>(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);
+  return axhelm_pcg_launch_t<double, double>(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,
+                                            lane_sums, S, s);
 }
 
 int axhelm_launch(int N, int Nf, int bk, nbx_prec prec, int32_t Nelements, int32_t offset,
@@ -59,20 +60,26 @@ int axhelm_launch(int N, int Nf, int bk, nbx_prec prec, int32_t Nelements, int32
   }
 }
 
+// AxFieldBlocks, the union over the types
+int64_t axhelm_pcg_lane_sums(int N, int Nf, int bk)
+{
+  return Nf == 3 && !bk && N >= 9 && N <= 11 ? 3 * (N + 1) * (N + 1) : 0;
+}
+
 int axhelm_pcg_launch(int N, int Nf, int bk, nbx_prec prec, int32_t Nelements, int32_t offset, const void* ggeo,
                       const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                      double* partials, const PcgFlags* S, hipStream_t s)
+                      double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s)
 {
   switch (prec) {
     case NBX_F64:
       return axhelm_pcg_dispatch_f64(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,
-                                                 S, s);
+                                                 lane_sums, S, s);
     case NBX_F32:
       return axhelm_pcg_dispatch_f32(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,
-                                               S, s);
+                                               lane_sums, S, s);
     case NBX_BF16:
       return axhelm_pcg_dispatch_bf16(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap,
-                                                  partials, S, s);
+                                                  partials, lane_sums, S, s);
     default:
       return fail(NBX_ERR_UNSUPPORTED, "axhelm_pcg: precision %d", (int)prec);
   }

@@ -13,9 +13,10 @@ int axhelm_dispatch_bf16(int N, int Nf, int bk, bool partial, int32_t Nelements,
 
 int axhelm_pcg_dispatch_bf16(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                             const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                            double* partials, const PcgFlags* S, hipStream_t s)
+                            double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s)
 {
-  return axhelm_pcg_launch_t<float, uint16_t>(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);
+  return axhelm_pcg_launch_t<float, uint16_t>(N, Nf, bk, Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,
+                                             lane_sums, S, s);
 }
 
 }  // namespace nbx

@@ -336,19 +336,18 @@ struct AxKept {
 };
 
 // Three-field PCG form: one thread group per field of an element against the
-// fields in turn.  Its lane sums run over the fields, so the fields of an
-// element stay in one workgroup.  Groups are faster while the chip is not
-// full, and where the fields in turn leave one wave per SIMD (FP64 non-BK, us,
-// groups / in turn: N = 7 at 1e5 nodes 7.8 / 11.0, at 8e6 288 / 236; N = 9 at
-// 1e5 12.8 / 18.7, at 8e6 433 / 389; N = 11 at 8e6 399 / 752).  The line in
-// lanes (Nq^2 per element) lies between the measured sizes on each side.
+// fields in turn.  Groups are faster while the chip is not full, and where the
+// fields in turn leave one wave per SIMD (FP64 non-BK, us, groups / in turn:
+// N = 7 at 1e5 nodes 7.8 / 11.0, at 8e6 288 / 236; N = 11 at 8e6 399 / 752).
+// The line in lanes (Nq^2 per element) lies between the measured sizes on each
+// side.
 template <typename T, int NQ, bool BK, typename G>
 struct AxFieldGroups {
   static constexpr bool fits = NQ >= 4 && 3 * (LineLayout<T, NQ>::SZ + LineLayout<T, NQ>::SS) * sizeof(T) < 150000;
   static bool when(int64_t Nelements)
   {
     const int64_t lanes = Nelements * (NQ * NQ);
-    if (sizeof(T) == 8) return NQ == 9 || NQ >= 12 || (NQ == 11 && !BK) || lanes < 64 * (NQ == 11 ? 4096 : 1024);
+    if (sizeof(T) == 8) return NQ == 9 || NQ >= 12 || lanes < 64 * (NQ == 11 ? 4096 : 1024);
     if (sizeof(G) == 2 && (NQ == 10 || NQ == 11)) return lanes < 64 * 2048;
     return NQ >= 9 || lanes < 64 * 16384;
   }
@@ -485,6 +484,28 @@ struct AxFieldSums {
   static constexpr bool value = NF == 3 && !BK && NQ >= 8 && NQ <= 12 && sizeof(G) != 2;
 };
 
+// Where the lane sums run per field, the fields can have a workgroup each and
+// hand them on through memory (one value per line and field, 1 / Nq of a
+// field, and a small kernel).  Small workgroups of two or three waves then
+// take the place of one that holds three fields' lines in LDS or one field's
+// registers on one wave per SIMD, and G and lambda of the fields after the
+// first come from the XCD's L2.  us, the better other form / this one:
+//            3e5 nodes      1e6            8e6
+//   N = 9    24.6 / 17.4    52.2 / 40.0    395 / 333   FP64 (1e5: 12.6 / 12.4)
+//   N = 10   17.8 / 17.9    51.0 / 40.7    415 / 320   FP64 (1e5: 15.2 / 11.9)
+//   N = 11   20.1 / 22.4    58.0 / 46.7    400 / 363   FP64 (6e5: 38.6 / 33.9)
+//   N = 9    13.1 / 12.4    35.7 / 30.9    251 / 231   FP32 (1e5: 9.1 / 10.0)
+//   N = 10   12.2 / 13.0    37.6 / 30.9    297 / 231   FP32 (6e5: 24.5 / 19.0)
+//   N = 11   13.7 / 16.1    40.2 / 33.2    265 / 239   FP32 (6e5: 26.3 / 26.2)
+// N = 7 and 8 lose (FP64 at 8e6 237 / 289 and 314 / 377).  Below one element a
+// CU only FP64 N = 9 and 10 gain.
+template <int NQ, int NF, bool BK, typename T, typename G>
+struct AxFieldBlocks {
+  static constexpr bool value = AxFieldSums<NQ, NF, BK, G>::value && NQ >= 10;
+  static constexpr bool always = value && sizeof(T) == 8 && NQ <= 11;
+  static bool when(int64_t Nelements) { return always || Nelements >= 256; }
+};
+
 template <int NQ2>
 constexpr int kTreeWidth = NQ2 <= 4 ? 4 : NQ2 <= 16 ? 16 : NQ2 <= 32 ? 32 : NQ2 <= 64 ? 64 : NQ2 <= 128 ? 128 : 256;
 
@@ -534,36 +555,46 @@ __device__ __forceinline__ double lane_tree(double v, double* s_red, const int s
 // undo the gather-scatter); this value is what BPAxOperator's dot returns.
 // The lanes' shares are summed by lane_tree; the element partials go to
 // partials[e].
-// FG (three fields): one thread group of NQ2 lanes per field of an element
-// (threadIdx.y = field) instead of the fields in turn; the groups hand the
-// lane sums on through LDS in field order.
-template <int NQ, int NF, bool BK, typename T, typename G, bool FG>
+// Three fields: in turn, one thread group of NQ2 lanes per field of an element
+// (threadIdx.y = field; the groups hand the lane sums on through LDS in field
+// order), or one workgroup per field (its lane sums go to memory; k_field_sums).
+enum PcgFields { kInTurn, kGroups, kBlocks };
+template <int NQ, int NF, bool BK, typename T, typename G, int FORM>
 struct AxPcg {
-  static constexpr bool kept = NF == 3 && !FG && AxKept<T, NQ, BK>::value;
-  static constexpr int epb = FG ? 1 : kept ? AxKept<T, NQ, BK>::epb : AxShape<T, NQ, BK>::epb;
+  static constexpr bool kept = NF == 3 && FORM == kInTurn && AxKept<T, NQ, BK>::value;
+  static constexpr int epb = FORM != kInTurn ? 1 : kept ? AxKept<T, NQ, BK>::epb : AxShape<T, NQ, BK>::epb;
   static constexpr int waves = kept ? AxKept<T, NQ, BK>::waves : NF == 1 ? AxShape<T, NQ, BK>::waves : 1;
   // the next field's z and p in flight during the current one, where the registers allow it
   static constexpr bool prefetch = kept && (sizeof(T) == 4 || NQ <= 8);
-  static constexpr bool late = NF == 3 && !FG && !prefetch;
+  static constexpr bool late = NF == 3 && FORM == kInTurn && !prefetch;
 };
 
-template <int NQ, int NF, bool BK, typename T, typename G, bool FG>
-__global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FG>::epb * (FG ? NF : 1)), (AxPcg<NQ, NF, BK, T, G, FG>::waves)) void k_axhelm_pcg(
+template <int NQ, int NF, bool BK, typename T, typename G, int FORM>
+__global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FORM>::epb * (FORM == kGroups ? NF : 1)), (AxPcg<NQ, NF, BK, T, G, FORM>::waves)) void k_axhelm_pcg(
     const int32_t Nelements, const int32_t offset, const G* __restrict__ ggeo, const T* __restrict__ D,
     const G* __restrict__ lambda, const double* __restrict__ z, double* __restrict__ p, double* __restrict__ Ap,
-    double* __restrict__ partials, const PcgFlags* __restrict__ S)
+    double* __restrict__ partials, double* __restrict__ lane_sums, const PcgFlags* __restrict__ S)
 {
-  using P = AxPcg<NQ, NF, BK, T, G, FG>;
+  using P = AxPcg<NQ, NF, BK, T, G, FORM>;
+  constexpr bool FG = FORM == kGroups, FB = FORM == kBlocks;
   using LL = LineLayout<T, NQ>;
   constexpr bool SUMS = AxFieldSums<NQ, NF, BK, G>::value;
-  constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = P::epb, GR = EPB * (FG ? NF : 1), LOOP = FG ? 1 : NF;
+  constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = P::epb, GR = EPB * (FG ? NF : 1), LOOP = FORM == kInTurn ? NF : 1;
   if (S->done) return;
   const double beta = S->beta;
   __shared__ T s_r[GR][LL::SZ], s_s[GR][LL::SS];
   __shared__ T s_l[P::kept && !BK ? EPB * NP : 1], s_w[P::kept && !BK ? EPB * NP : 1];
   __shared__ double s_red[EPB * kTreeWidth<NQ2>], s_acc[FG ? NF : 1][FG ? NQ2 : 1];
-  const int t = threadIdx.x, y = GR > 1 ? (int)threadIdx.y : 0, slot = FG ? 0 : y, field0 = FG ? y : 0;
-  const ElemPlace<false, EPB> E((int32_t)blockIdx.x * EPB, Nelements, nullptr, slot);
+  const int t = threadIdx.x, y = GR > 1 ? (int)threadIdx.y : 0, slot = FG ? 0 : y;
+  int32_t block = blockIdx.x;
+  int field0 = FG ? y : 0;
+  if constexpr (FB) {  // as k_axhelm: an element's fields follow each other on one XCD
+    const int32_t local = block >> 3;
+    field0 = local % NF;
+    block = (local / NF) * 8 + (block & 7);
+    if (block >= Nelements) return;
+  }
+  const ElemPlace<false, EPB> E(block * EPB, Nelements, nullptr, slot);
   const int32_t lo = E.rel * NP + t;
   const double* zf = z + E.base * NP + (int64_t)field0 * offset;
   double* pf = p + E.base * NP + (int64_t)field0 * offset;
@@ -631,7 +662,7 @@ __global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FG>::epb * (FG ?
         for (int k = 0; k < NQ; ++k) stnt((double)out[k], &Af[lo + k * NQ2]);
       }
       Af += offset;
-      if (SUMS && !FG) {
+      if (SUMS && FORM == kInTurn) {
         if (f == 0) fsum[0] = acc;
         else if (f == 1) fsum[NF > 1 ? 1 : 0] = acc;
         else fsum[NF - 1] = acc;
@@ -648,15 +679,43 @@ __global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FG>::epb * (FG ?
     GeoStream<T, NQ, BK, G, NF == 1, AxShape<T, NQ, BK>::ahead, int32_t> geo{gb, lb, lb + offset, go, lo, {}};
     run(geo);
   }
+  if constexpr (FB) {
+    lane_sums[(E.base * NF + field0) * NQ2 + t] = acc;
+    return;
+  }
   if constexpr (SUMS && FG) {
     s_acc[y][t] = acc;
     __syncthreads();
     acc = (s_acc[0][t] + s_acc[1][t]) + s_acc[2][t];
-  } else if constexpr (SUMS) {
+  } else if constexpr (SUMS && FORM == kInTurn) {
     acc = (fsum[0] + fsum[1]) + fsum[2];
   }
   const double sum = lane_tree<NQ2, EPB>(acc, s_red, slot, t, y * NQ2 + t, y == slot);
   if (t == 0 && y == slot && E.active) partials[E.base + E.rel] = sum;
+}
+
+// partials[e] of the one-workgroup-per-field form: (f0 + f1) + f2 per lane,
+// then lane_tree's order; a wave per element.  Launch-bound (about 2.5 us at
+// 1e6 nodes).
+template <int NQ2>
+__global__ __launch_bounds__(256) void k_field_sums(const int32_t Nelements, const double* __restrict__ lane_sums,
+                                                    double* __restrict__ partials, const PcgFlags* __restrict__ S)
+{
+  constexpr int P2 = kTreeWidth<NQ2>;
+  static_assert(P2 == 128 || P2 == 256, "two or four values a lane");
+  if (S->done) return;
+  const int l = threadIdx.x & 63;
+  const int64_t e = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (e >= Nelements) return;
+  const double* const a = lane_sums + e * 3 * NQ2;
+  double v[P2 / 64];
+#pragma unroll
+  for (int u = 0; u < P2 / 64; ++u) {
+    const int t = l + 64 * u;
+    v[u] = t < NQ2 ? (a[t] + a[NQ2 + t]) + a[2 * NQ2 + t] : 0.0;
+  }
+  const double x = wave_sum(P2 == 256 ? (v[0] + v[P2 / 128]) + (v[1] + v[P2 / 64 - 1]) : v[0] + v[1]);
+  if (l == 0) partials[e] = x;
 }
 
 // Local Jacobi diagonal, nekBone/kernel/updateJacobi.okl:27-108, same
@@ -796,36 +855,54 @@ static int dispatch_n(int N, int Nf, int bk, bool partial, int32_t Nelements, in
 template <int NQ, int NF, bool BK, typename T, typename G>
 static void axhelm_pcg_launch_k(int32_t Nelements, int32_t offset, const void* ggeo, const void* D,
                                 const void* lambda, const double* z, double* p, double* Ap, double* partials,
-                                const PcgFlags* S, hipStream_t s)
+                                double* lane_sums, const PcgFlags* S, hipStream_t s)
 {
-  if constexpr (NF == 3 && AxFieldGroups<T, NQ, BK, G>::fits) {
-    if (AxFieldGroups<T, NQ, BK, G>::when(Nelements)) {
-      hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, true>), dim3(Nelements), dim3(NQ * NQ, NF), 0, s, Nelements,
-                         offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap, partials, S);
+  if constexpr (AxFieldBlocks<NQ, NF, BK, T, G>::value) {
+    if (AxFieldBlocks<NQ, NF, BK, T, G>::when(Nelements)) {
+      hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, kBlocks>), dim3((unsigned)((Nelements + 7) / 8 * 8) * NF),
+                         dim3(NQ * NQ), 0, s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p,
+                         Ap, partials, lane_sums, S);
+      hipLaunchKernelGGL(k_field_sums<NQ * NQ>, dim3((Nelements + 3) / 4), dim3(256), 0, s, Nelements, lane_sums,
+                         partials, S);
       return;
     }
   }
-  constexpr int EPB = AxPcg<NQ, NF, BK, T, G, false>::epb;
-  hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, false>), dim3((Nelements + EPB - 1) / EPB), dim3(NQ * NQ, EPB), 0,
-                     s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap, partials, S);
+  if constexpr (NF == 3 && AxFieldGroups<T, NQ, BK, G>::fits && !AxFieldBlocks<NQ, NF, BK, T, G>::always) {
+    if (AxFieldGroups<T, NQ, BK, G>::when(Nelements)) {
+      hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, kGroups>), dim3(Nelements), dim3(NQ * NQ, NF), 0, s,
+                         Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z, p, Ap, partials,
+                         lane_sums, S);
+      return;
+    }
+  }
+  if constexpr (!AxFieldBlocks<NQ, NF, BK, T, G>::always) {
+    constexpr int EPB = AxPcg<NQ, NF, BK, T, G, kInTurn>::epb;
+    hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, kInTurn>), dim3((Nelements + EPB - 1) / EPB),
+                       dim3(NQ * NQ, EPB), 0, s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z,
+                       p, Ap, partials, lane_sums, S);
+  }
 }
 
 template <typename T, typename G>
 static int axhelm_pcg_launch_t(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                                const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                               double* partials, const PcgFlags* S, hipStream_t s)
+                               double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s)
 {
 #define NBX_AXP(NV)                                                                                              \
   case NV:                                                                                                       \
     if (Nelements < 1) break;                                                                                    \
     if (Nf == 1 && bk)                                                                                           \
-      axhelm_pcg_launch_k<NV + 1, 1, true, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);   \
+      axhelm_pcg_launch_k<NV + 1, 1, true, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,           \
+                                                   lane_sums, S, s);                                            \
     else if (Nf == 1)                                                                                            \
-      axhelm_pcg_launch_k<NV + 1, 1, false, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);  \
+      axhelm_pcg_launch_k<NV + 1, 1, false, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,           \
+                                                   lane_sums, S, s);                                            \
     else if (bk)                                                                                                 \
-      axhelm_pcg_launch_k<NV + 1, 3, true, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);   \
+      axhelm_pcg_launch_k<NV + 1, 3, true, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,           \
+                                                   lane_sums, S, s);                                            \
     else                                                                                                         \
-      axhelm_pcg_launch_k<NV + 1, 3, false, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials, S, s);  \
+      axhelm_pcg_launch_k<NV + 1, 3, false, T, G>(Nelements, offset, ggeo, D, lambda, z, p, Ap, partials,           \
+                                                   lane_sums, S, s);                                            \
     break;
   if (Nf != 1 && Nf != 3) return fail(NBX_ERR_UNSUPPORTED, "axhelm_pcg: Nfields=%d", Nf);
   switch (N) {
@@ -865,12 +942,12 @@ int axhelm_dispatch_bf16(int N, int Nf, int bk, bool partial, int32_t Nelements,
                          const void* q, void* Aq, const int* skip, hipStream_t s);
 int axhelm_pcg_dispatch_f64(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                             const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                            double* partials, const PcgFlags* S, hipStream_t s);
+                            double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s);
 int axhelm_pcg_dispatch_f32(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                             const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                            double* partials, const PcgFlags* S, hipStream_t s);
+                            double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s);
 int axhelm_pcg_dispatch_bf16(int N, int Nf, int bk, int32_t Nelements, int32_t offset, const void* ggeo,
                              const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                             double* partials, const PcgFlags* S, hipStream_t s);
+                             double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s);
 
 }  // namespace nbx

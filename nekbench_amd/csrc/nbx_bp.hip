@@ -556,6 +556,8 @@ static int bp_setup_impl(nbx_bp* bp)
       (rc = bp->alloc(&bp->elem_partials, E)) || (rc = bp->alloc(&bp->b, bp->Nall)) ||
       (rc = bp->alloc(&bp->d, bp->Nall)))
     return rc;
+  if (const int64_t n = E * axhelm_pcg_lane_sums(bp->N, bp->Nf, o.bpmode ? 1 : 0))
+    if ((rc = bp->alloc(&bp->lane_sums, n))) return rc;
   NBX_HIP(hipMemcpy(bp->D, D.data(), sizeof(double) * D.size(), hipMemcpyHostToDevice));
   // lambda0 = 1, lambda1 per node (setup.cpp:104-108)
   hipLaunchKernelGGL(k_fill_lambda, grid_for(bp->fieldOffset), dim3(256), 0, bp->stream, (int64_t)bp->fieldOffset,
@@ -804,8 +806,8 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
       lam = bp->lambda16;
     }
     int rc = axhelm_pcg_launch(bp->N, bp->Nf, o.bpmode ? 1 : 0, bp->op_prec, bp->E, bp->fieldOffset, g, Dm, lam,
-                               zsrc, bp->p, bp->Ap, bp->elem_partials, reinterpret_cast<const PcgFlags*>(bp->S),
-                               bp->stream);
+                               zsrc, bp->p, bp->Ap, bp->elem_partials, bp->lane_sums,
+                               reinterpret_cast<const PcgFlags*>(bp->S), bp->stream);
     if (rc) return rc;
     prof_mark(bp, kProfAx);  // p = z + beta p, A p and its pAp shares
     rc = gs_add_mask_pap_launch(bp->ogs, bp->Ap, bp->Nf, bp->fieldOffset, bp->Nmasked, bp->maskIds, (unsigned)bp->E,

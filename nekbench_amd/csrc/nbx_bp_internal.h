@@ -56,6 +56,7 @@ struct nbx_bp {
   double *D = nullptr, *ggeo = nullptr, *lambda = nullptr, *invDiagA = nullptr, *rhs = nullptr;
   double *p = nullptr, *z = nullptr, *Ap = nullptr, *Ax = nullptr;
   double* elem_partials = nullptr;  // per-element shares of pAp (fused schedule)
+  double* lane_sums = nullptr;      // their lanes' sums (axhelm_pcg_lane_sums)
   // low-precision operator operands (built on first use)
   float* ggeo32 = nullptr;
   float* D32 = nullptr;

@@ -99,7 +99,9 @@ int mask_list_from_ids(int32_t N, const int64_t* ids, int32_t** maskIds, int32_t
 // float arithmetic); partials[e] = element share of pAp (FP64)
 int axhelm_pcg_launch(int N, int Nf, int bk, nbx_prec prec, int32_t Nelements, int32_t offset, const void* ggeo,
                       const void* D, const void* lambda, const double* z, double* p, double* Ap,
-                      double* partials, const PcgFlags* S, hipStream_t s);
+                      double* partials, double* lane_sums, const PcgFlags* S, hipStream_t s);
+// the doubles per element that it takes in lane_sums (0: none, lane_sums unused)
+int64_t axhelm_pcg_lane_sums(int N, int Nf, int bk);
 // double add gather-scatter of every field plus the Dirichlet mask, one launch
 int gs_add_mask_launch(const nbx_ogs* o, double* v, int k, int32_t stride, int32_t Nmasked,
                        const int32_t* maskIds, const int* skip, hipStream_t s);

@@ -87,3 +87,26 @@ def test_three_field_pcg_matches_oracle(nbx, nbo, dev, N, dims, bpmode):
     ob.pcg(rr, xr, 0.0, 5, jacobi=True)
     assert np.array_equal(x.cpu().numpy(), xr)
     assert np.array_equal(r.cpu().numpy(), rr)
+
+
+# one workgroup per field: element counts on each side of its line, and not a
+# multiple of eight (the XCD order pads the grid)
+@pytest.mark.parametrize("N,dims", [(9, (5, 17, 3)), (9, (1, 257, 1)), (10, (1, 255, 1)), (10, (16, 16, 1)),
+                                    (11, (1, 255, 1)), (11, (1, 257, 1))])
+def test_three_field_pcg_per_field_workgroups_match_oracle(nbx, nbo, dev, N, dims):
+    import torch
+    kw = dict(perturb=0.1, seed=60 + N)
+    bp = nbx.BP(nbx.Box.make(N, *dims, **kw), Nfields=3, bpmode=False, lambda1=0.3, precon=nbx.PRECON_JACOBI)
+    ob = nbo.OracleBP(nbo.Box.make(N, *dims, **kw), Nf=3, bpmode=False, lambda1=0.3)
+    for prec in (nbx.NBX_F64, nbx.NBX_F32):
+        r = torch.from_numpy(ob.rhs.copy()).to(dev)
+        x = torch.zeros_like(r)
+        rr, xr = ob.rhs.copy(), np.zeros_like(ob.rhs)
+        if prec == nbx.NBX_F64:
+            bp.pcg(r, x, 0.0, 3)
+            ob.pcg(rr, xr, 0.0, 3, jacobi=True)
+            assert np.array_equal(r.cpu().numpy(), rr)
+        else:
+            bp.pcg_mixed(r, x, 1e-30, 3, prec=prec, inner_tol=1e-20, max_cycles=1)
+            ob.pcg_mixed(rr, xr, 1e-30, 3, prec=1, inner_tol=1e-20, max_cycles=1, jacobi=True)
+        assert np.array_equal(x.cpu().numpy(), xr), prec
