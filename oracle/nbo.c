@@ -735,7 +735,7 @@ double nbo_tree_dot(int64_t n, const double* x, const double* y)
 #include <omp.h>
 int nbo_max_threads(void) { return omp_get_max_threads(); }
 
-/* axhelm with matrix-core contractions (library: k_axhelm_mma and
+/* axhelm with matrix-core contractions (library:
  * k_axhelm_mma16, nbx_axhelm_mma.hip), any N, Nf fields: q, D and the G-scaled gradients are
  * rounded to the operand type (bf16 or fp16, nearest even); the 8-term
  * contractions are accumulated in double and rounded to float (the products

@@ -110,3 +110,31 @@ def test_three_field_pcg_per_field_workgroups_match_oracle(nbx, nbo, dev, N, dim
             bp.pcg_mixed(r, x, 1e-30, 3, prec=prec, inner_tol=1e-20, max_cycles=1)
             ob.pcg_mixed(rr, xr, 1e-30, 3, prec=1, inner_tol=1e-20, max_cycles=1, jacobi=True)
         assert np.array_equal(x.cpu().numpy(), xr), prec
+
+
+@pytest.mark.parametrize("N", [7, 9])
+@pytest.mark.parametrize("f16", [False, True], ids=["bf16", "fp16"])
+def test_matrix_core_fields_at_any_alignment(nbx, dev, N, f16):
+    """The matrix-core operator loads node pairs: operands that start at an odd
+    element, with an odd field offset, give the bits of the aligned one-field
+    call."""
+    import torch
+    E, Np = 3, (N + 1) ** 3
+    n = E * Np
+    off = n + 5
+    gen = torch.Generator(device=dev).manual_seed(N)
+    geo = torch.float32 if f16 else torch.bfloat16
+    prec = nbx.NBX_F16 if f16 else nbx.NBX_BF16_MFMA
+    r = lambda m, dt=torch.float32: (torch.rand(m, generator=gen, device=dev) - 0.5).to(dt)
+    bits = lambda a: a if f16 else a.view(torch.int16)
+    at1 = lambda a: torch.cat([a[:1], a])[1:]  # the same values, one element into an allocation
+    g, D, lam, q = r(7 * n, geo), r((N + 1) ** 2), r(2 * off, geo), r(3 * off)
+    lam1 = torch.cat([lam[:n], lam[off:off + n]])
+    for bk in (1, 0):
+        out = torch.full((3 * off + 1,), 7.0, device=dev)[1:]
+        nbx.axhelm(N, 3, bk, E, off, bits(at1(g)), at1(D), bits(at1(lam)), at1(q), out, prec=prec)
+        for f in range(3):
+            one = torch.empty(n, device=dev)
+            nbx.axhelm(N, 1, bk, E, n, bits(g), D, bits(lam1), q[f * off:f * off + n].clone(), one, prec=prec)
+            assert torch.equal(out[f * off:f * off + n], one), (bk, f)
+            assert bool((out[f * off + n:(f + 1) * off] == 7.0).all())
