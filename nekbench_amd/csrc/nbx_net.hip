@@ -35,6 +35,9 @@ constexpr int kFRow = 800;                            // a factor row: node (x, 
 // 128 nodes of 96 channel rows; row stride 4 modulo the banks, so the 8 rows
 // that 8 lanes read 16 bytes of lie in different banks
 constexpr int kTrainRow = 132, kTrainRows = 96;
+// T rows in the same buffer: the rows 4 g + u of a product lie 16 banks apart for g = 0..3
+constexpr int kTRow = 516;
+static_assert(16 * kTRow <= kTrainRows * kTrainRow, "a product's T rows fit the buffer");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -168,25 +171,31 @@ __global__ __launch_bounds__(512) void k_net_apply(const int32_t E, const float*
 // unweighted element output invDiag (r + s y) at local node n of element e;
 // the kernel then back-propagates dL/dy = G invDiag s and reports no loss.
 //
-// Lane n is node n for the forward pass and the data gradients (weights as
-// scalar operands, FP32 vector ALUs).  The parameter gradients are products
-// over the 512 nodes, dW[a][c] = sum_n A[a][n] B[n][c], an fma chain in
-// increasing n: they run on the matrix cores as 16x16x4 FP32 products, which
-// accumulate k in increasing order with one rounding a step -- the chain's
-// bits -- one 16x16 tile of one tensor a wave, 16 tiles over two phases:
+// All products run on the matrix cores as 16x16x4 FP32 products, which
+// accumulate k in increasing order with one rounding a step: the bits of the
+// fma chains they stand for.
+// Forward pass and data gradients: a wave takes the 64 nodes of its plane, the
+// layers' channels as rows and the nodes as columns; channels are held in the
+// order in which one product's result is the next one's operand (NodeChannels).
+// The first layer's taps and the last layer's backward taps are read from the
+// zero-padded 10^3 tiles of r^ and dL/dy.
+// The parameter gradients are products over the 512 nodes, dW[a][c] =
+// sum_n A[a][n] B[n][c] in increasing n, one 16x16 tile of one tensor a wave,
+// 16 tiles over two phases:
 //   phase 1: W3 (taps x channels; dL/dT and h2), W2 (h1 and dL/dpre2)
 //   phase 2: Wr, Wg and b1 as 35 rows (r^ taps, factors, ones; dL/dpre1),
 //            b2 (ones; dL/dpre2), and b3 as a plain chain beside them.
 // The lanes hand their channels to the tiles through LDS 128 nodes at a time,
 // nodes ordered inside 16 so that a lane's four k values are one 16-byte
-// read; the tap operands are the zero-padded 10^3 tiles of r^ and dL/dy at a
-// fixed offset, the factors rows of the same layout.
-// Bound: FP32 vector issue (4864 fma a node, 130 us of 2048 samples on this
-// chip) beside 2048 matrix products of 32 cycles a sample (55 us); 80 KB of
-// LDS and 128 registers keep two workgroups a CU, so that one's products run
-// under the other's vector work.  2048 samples: 3836 -> 290 us against the
-// form that held one parameter a lane (two LDS reads an fma) and gave a
-// workgroup a whole chunk of samples (half the chip idle at 16 a chunk).
+// read; the tap operands are the tiles at a fixed offset, the factors rows of
+// the same layout.
+// Bound: 4608 products of 32 cycles a sample (123 us of 2048 samples on this
+// chip; half of the kernel's time), the rest waits: 80 KB of LDS and 128
+// registers keep two workgroups a CU, and a sample has 22 barriers.
+// 2048 samples: 3836 us for the form that held one parameter a lane (two LDS
+// reads an fma) and gave a workgroup a whole chunk of samples (half the chip
+// idle at 16 a chunk); 290 with the forward pass and the data gradients on the
+// vector ALUs, lane = node, weights as scalar operands; 252 now.
 struct TrainLds {
   float rh[kPadN], dy[kPadN];      // zero-padded tiles
   float g[kG * kFRow];             // factors, node (x, y, z) at 100 z + 10 y + x
@@ -194,72 +203,65 @@ struct TrainLds {
   double red[kP / 64];
 };
 
-// Half a row of 32 weights in scalar registers (constant address space:
-// scalar loads); the pointer is made opaque at every half, or the compiler
-// loads weights long before their use and spills them.  for_rows runs
-// f(r, c, w[c % 16]) over the rows and channels in order; the next half's loads
-// are issued after the first product, which waits for this half's, and are in
-// flight during the others.
-typedef const float __attribute__((address_space(4)))* WeightPtr;
-struct WHalf {
-  float w[kC / 2];
-  __device__ __forceinline__ void load(WeightPtr p, int half)
-  {
-    asm volatile("" : "+s"(p));
-#pragma unroll
-    for (int c = 0; c < kC / 2; ++c) w[c] = p[half * (kC / 2) + c];
-  }
-};
-template <int ROWS, typename F>
-__device__ __forceinline__ void for_rows(const float* base, F&& f)
-{
-  const WeightPtr p = (WeightPtr)base;
-  WHalf R, Rn;
-  R.load(p, 0);
-#pragma unroll
-  for (int h = 0; h < 2 * ROWS; ++h) {
-    const int c0 = (h & 1) * (kC / 2);
-    f(h >> 1, c0, R.w[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    if (h + 1 < 2 * ROWS) Rn.load(p, h + 1);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 1; c < kC / 2; ++c) f(h >> 1, c0 + c, R.w[c]);
-    R = Rn;
-  }
-}
-// the value is formed here: without this the compiler moves whole products,
-// weights and all, into the later branch that stores their results
-__device__ __forceinline__ void keep_here(float& v) { asm volatile("" : "+v"(v)); }
-// acc[c] = fma(w[r][c], x(r), acc[c]) over the rows in order
-template <int ROWS, typename X>
-__device__ __forceinline__ void add_rows(const float* base, X&& x, float (&acc)[kC])
-{
-  float v;
-  for_rows<ROWS>(base, [&](int r, int c, float w) {
-    if (c == 0) v = x(r);
-    acc[c] = __builtin_fmaf(w, v, acc[c]);
-  });
-#pragma unroll
-  for (int c = 0; c < kC; ++c) keep_here(acc[c]);
-}
-// to(r, sum_c w[r][c] x[c]), the chain over c in order
-template <int ROWS, typename S>
-__device__ __forceinline__ void dot_rows(const float* base, const float (&x)[kC], S&& to)
-{
-  float t;
-  for_rows<ROWS>(base, [&](int r, int c, float w) {
-    t = __builtin_fmaf(w, x[c], c == 0 ? 0.f : t);
-    if (c == kC - 1) {
-      keep_here(t);
-      to(r, t);
-    }
-  });
-}
-
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
 {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The 64 nodes of a wave's plane by 32 channels: node tile tt (nodes 16 tt + col),
+// channel tile m; value u is channel 16 m + 4 u + kg.  That is a product's
+// result if its rows are the channels in the order of chan_row, and the next
+// product's operand at step 4 m + u, whose k = 4 (4 m + u) + kg is the channel:
+// the layers chain in registers, each channel's chain in increasing order.
+struct NodeChannels {
+  f32x4 v[4][2];
+};
+__device__ __forceinline__ int chan_row(int r) { return 4 * (r & 3) + (r >> 2); }
+
+// acc += A x over STEPS steps of four terms: a(t, m) is the lane's weight of
+// channel tile m (those of AHEAD steps in registers at once), x(t, tt) its
+// operand of node tile tt
+template <int STEPS, int AHEAD, typename WA, typename X>
+__device__ __forceinline__ void layer(WA&& a, X&& x, NodeChannels& acc)
+{
+#pragma unroll
+  for (int t0 = 0; t0 < STEPS; t0 += AHEAD) {
+    float w[AHEAD][2];
+#pragma unroll
+    for (int t = t0; t < min(t0 + AHEAD, STEPS); ++t)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) w[t - t0][m] = a(t, m);
+#pragma unroll
+    for (int t = t0; t < min(t0 + AHEAD, STEPS); ++t)
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        const float b = x(t, tt);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) acc.v[tt][m] = mfma4(w[t - t0][m], b, acc.v[tt][m]);
+      }
+  }
+}
+
+template <typename F>
+__device__ __forceinline__ void each_channel(F&& f)
+{
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) f(tt, m, u);
+}
+
+// (the values are opaque afterwards: relu' compares them again, or the compiler
+// keeps 64 comparisons in scalar registers and spills them)
+__device__ __forceinline__ void relu(NodeChannels& h)
+{
+  each_channel([&](int tt, int m, int u) {
+    float v = h.v[tt][m][u] > 0.f ? h.v[tt][m][u] : 0.f;
+    asm volatile("" : "+v"(v));
+    h.v[tt][m][u] = v;
+  });
 }
 
 __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ samples, const int64_t pairStride,
@@ -273,8 +275,6 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
   const int n = threadIdx.x, l = n & 63, wv = n >> 6, col = l & 15, kg = l >> 4;
   const int i = n & 7, j = (n >> 3) & 7, k = n >> 6;
   const int place = 100 * k + 10 * j + i;  // in the 10-strided layout; the tiles' interior starts at 111
-  const float* Wr = W + kOffWr;
-  const float* Wg = W + kOffWg;
   const float* W2 = W + kOffW2;
   const float* W3 = W + kOffW3;
   const int2 pe = samples[blockIdx.x];
@@ -284,42 +284,66 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
   const double en = G ? 0.0 : (double)Ev[off];
   const double di = invDiag[e * kP + n];
   for (int q = n; q < kPadN; q += kP) lds.rh[q] = lds.dy[q] = 0.f;
-  float h1[kC], g[kG];
 #pragma unroll
-  for (int q = 0; q < kG; ++q) g[q] = feat[(e * kG + q) * kP + n];
-#pragma unroll
-  for (int c = 0; c < kC; ++c) h1[c] = W[kOffB1 + c];
-#pragma unroll
-  for (int q = 0; q < kG; ++q) lds.g[q * kFRow + place] = g[q];
-  add_rows<kG>(Wg, [&](int q) { return g[q]; }, h1);
+  for (int q = 0; q < kG; ++q) lds.g[q * kFRow + place] = feat[(e * kG + q) * kP + n];
   const double s = element_scale(rn, lds.red);  // its barrier also ends the zero fill
   const double inv = s > 0.0 ? 1.0 / s : 0.0;
   lds.rh[111 + place] = (float)(rn * inv);
   __syncthreads();
-  add_rows<kTaps>(Wr, [&](int tap) { return lds.rh[place + tap_place(tap)]; }, h1);
+  // the lane's nodes in the products are those of its wave's plane, tile tt's
+  // at pl + 20 tt; its weights' rows are channels 16 m + ch
+  const int pl = 100 * wv + 10 * (col >> 3) + (col & 7), ch = chan_row(col);
+  const float* const lds0 = reinterpret_cast<const float*>(&lds);  // rh, dy, g in that order
+  NodeChannels h1, h2;
+  each_channel([&](int tt, int m, int u) { h1.v[tt][m][u] = W[kOffB1 + 16 * m + 4 * u + kg]; });
+  {
+    // terms: the factors, then the taps (zero past the last)
+    constexpr int kTerms = kG + kTaps, kSteps = (kTerms + 3) / 4;
+    int at[kSteps], wt[kSteps];
 #pragma unroll
-  for (int c = 0; c < kC; ++c) h1[c] = h1[c] > 0.f ? h1[c] : 0.f;
-  float h2[kC];
-#pragma unroll
-  for (int c = 0; c < kC; ++c) h2[c] = W[kOffB2 + c];
-  add_rows<kC>(W2, [&](int ci) { return h1[ci]; }, h2);
-#pragma unroll
-  for (int c = 0; c < kC; ++c) h2[c] = h2[c] > 0.f ? h2[c] : 0.f;
-  // y = b3 + sum over the taps of T[tap] at node n + tap, nine taps (one dz)
-  // at a time through two halves of the buffer
+    for (int t = 0; t < kSteps; ++t) {
+      const int term = 4 * t + kg, tap = min(max(term - kG, 0), kTaps - 1);
+      at[t] = pl + (term < kG ? 2 * kPadN + term * kFRow : tap_place(tap));
+      wt[t] = (term < kG ? kOffWg + term * kC : kOffWr + tap * kC) + ch;
+    }
+    layer<kSteps, kSteps>([&](int t, int m) { return 4 * t + kg < kTerms ? W[wt[t] + 16 * m] : 0.f; },
+                  [&](int t, int tt) {
+                    const float v = lds0[at[t] + 20 * tt];
+                    return 4 * t + 3 < kTerms || 4 * t + kg < kTerms ? v : 0.f;
+                  },
+                  h1);
+  }
+  relu(h1);
+  each_channel([&](int tt, int m, int u) { h2.v[tt][m][u] = W[kOffB2 + 16 * m + 4 * u + kg]; });
+  layer<kC / 4, 8>([&](int t, int m) { return W2[(4 * t + kg) * kC + 16 * m + ch]; },
+                [&](int t, int tt) { return h1.v[tt][t >> 2][t & 3]; }, h2);
+  relu(h2);
+  // y = b3 + sum over the taps of T[tap] at node n + tap: a product's 16 taps at
+  // a time through the buffer
   const bool ox[3] = {i > 0, true, i < 7}, oy[3] = {j > 0, true, j < 7}, oz[3] = {k > 0, true, k < 7};
   float y = W[kOffB3];
 #pragma unroll
-  for (int z = 0; z < 3; ++z) {
-    float* const T = lds.buf + (z & 1) * 9 * kP;
-    dot_rows<9>(W3 + 9 * z * kC, h2, [&](int u, float t) { T[u * kP + n] = t; });
+  for (int m = 0; m < 2; ++m) {
+    f32x4 T[4] = {};
+    float w[kC / 4];
+#pragma unroll
+    for (int t = 0; t < kC / 4; ++t) w[t] = W3[min(16 * m + col, kTaps - 1) * kC + 4 * t + kg];
+#pragma unroll
+    for (int t = 0; t < kC / 4; ++t)
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) T[tt] = mfma4(w[t], h2.v[tt][t >> 2][t & 3], T[tt]);
+    if (m) __syncthreads();  // the first taps' readers are done
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) lds.buf[(4 * kg + u) * kTRow + 64 * wv + 16 * tt + col] = T[tt][u];
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 9; ++u) {
-      const int dx = u % 3, dyy = u / 3;
+    for (int tap = 16 * m; tap < min(16 * m + 16, kTaps); ++tap) {
+      const int dx = tap % 3, dyy = (tap / 3) % 3, z = tap / 9;
       const bool in = ox[dx] && oy[dyy] && oz[z];
-      const int m = n + (dx - 1) + 8 * (dyy - 1) + 64 * (z - 1);
-      const float v = T[u * kP + (in ? m : n)];
+      const int nb = n + (dx - 1) + 8 * (dyy - 1) + 64 * (z - 1);
+      const float v = lds.buf[(tap - 16 * m) * kTRow + (in ? nb : n)];
       y = y + (in ? v : 0.f);
     }
   }
@@ -346,16 +370,29 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
     reinterpret_cast<double*>(po + kNetParamsPadded)[0] = t;
   }
   // dL/dpre2 = relu'(h2) sum over the taps of W3[tap] dy(n - tap)
-  float d2[kC];
+  NodeChannels d2 = {};
+  {
+    constexpr int kSteps = (kTaps + 3) / 4;
+    int at[kSteps];
 #pragma unroll
-  for (int c = 0; c < kC; ++c) d2[c] = 0.f;
-  add_rows<kTaps>(W3, [&](int tap) { return lds.dy[place + tap_place(26 - tap)]; }, d2);
-#pragma unroll
-  for (int c = 0; c < kC; ++c) d2[c] = h2[c] > 0.f ? d2[c] : 0.f;
+    for (int t = 0; t < kSteps; ++t) at[t] = kPadN + pl + tap_place(26 - min(4 * t + kg, kTaps - 1));
+    layer<kSteps, 4>([&](int t, int m) { return 4 * t + kg < kTaps ? W3[(4 * t + kg) * kC + 16 * m + ch] : 0.f; },
+                  [&](int t, int tt) {
+                    const float v = lds0[at[t] + 20 * tt];
+                    return 4 * t + 3 < kTaps || 4 * t + kg < kTaps ? v : 0.f;
+                  },
+                  d2);
+  }
+  each_channel([&](int tt, int m, int u) { d2.v[tt][m][u] = h2.v[tt][m][u] > 0.f ? d2.v[tt][m][u] : 0.f; });
 
   // the node's column in a 128-node buffer row: inside 16 nodes, 4 s + g is
   // kept at 4 g + s, so k group g reads the nodes 4 s + g, s = 0..3, at once
-  const int cpos = (n & 0x70) | ((n & 3) << 2) | ((n >> 2) & 3);
+  const int cpos = (wv & 1) * 64 + ((col & 3) << 2) + (col >> 2);
+  auto put = [&](int row0, const NodeChannels& x) {
+    each_channel([&](int tt, int m, int u) {
+      lds.buf[(row0 + 16 * m + 4 * u + kg) * kTrainRow + cpos + 16 * tt] = x.v[tt][m][u];
+    });
+  };
   const int rd = col * kTrainRow + 4 * kg;  // a lane's operand read: row col, group kg
   // phase 1: waves 0..3 W3, waves 4..7 W2; one (row tile, channel tile) each
   {
@@ -366,12 +403,9 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
     for (int h = 0; h < 4; ++h) {
       __syncthreads();  // the buffer's last readers are done
       if ((wv >> 1) == h) {
-#pragma unroll
-        for (int c = 0; c < kC; ++c) {
-          lds.buf[c * kTrainRow + cpos] = h2[c];
-          lds.buf[(kC + c) * kTrainRow + cpos] = h1[c];
-          lds.buf[(2 * kC + c) * kTrainRow + cpos] = d2[c];
-        }
+        put(0, h2);
+        put(kC, h1);
+        put(2 * kC, d2);
       }
       __syncthreads();
       if (wv < 4) {
@@ -401,8 +435,11 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
       else if (row < kTaps) po[kOffW3 + row * kC + 16 * ct + col] = acc[u];
     }
   }
-  // dL/dpre1 = relu'(h1) W2 dL/dpre2, over h2's registers
-  dot_rows<kC>(W2, d2, [&](int ci, float a) { h2[ci] = h1[ci] > 0.f ? a : 0.f; });
+  // dL/dpre1 = relu'(h1) W2 dL/dpre2
+  NodeChannels d1 = {};
+  layer<kC / 4, 8>([&](int t, int m) { return W2[(16 * m + ch) * kC + 4 * t + kg]; },
+                [&](int t, int tt) { return d2.v[tt][t >> 2][t & 3]; }, d1);
+  each_channel([&](int tt, int m, int u) { d1.v[tt][m][u] = h1.v[tt][m][u] > 0.f ? d1.v[tt][m][u] : 0.f; });
   // phase 2: waves 0..5 the 35 rows of Wr, Wg, b1 (three row tiles), waves 6, 7 b2
   {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -415,11 +452,8 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
     for (int h = 0; h < 4; ++h) {
       __syncthreads();
       if ((wv >> 1) == h) {
-#pragma unroll
-        for (int c = 0; c < kC; ++c) {
-          lds.buf[c * kTrainRow + cpos] = h2[c];
-          lds.buf[(kC + c) * kTrainRow + cpos] = d2[c];
-        }
+        put(0, d1);
+        put(kC, d2);
       }
       __syncthreads();
       const float* const b = lds.buf + ((rt == 3 ? kC : 0) + 16 * ct) * kTrainRow + rd;
