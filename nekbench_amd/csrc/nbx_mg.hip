@@ -174,102 +174,118 @@ __global__ __launch_bounds__(256) void k_cheb_sum(const int32_t n, const int32_t
   }
 }
 
-// Restriction of one element: res -= Ad (stored), u = w res, then
+// Elements of a workgroup of the transfers between levels: as many as its 256
+// lanes have fine nodes for (orders known at compile time), one otherwise; LDS
+// for those nodes only.  (N = 3 to 1, 32768 elements, one element a workgroup
+// and 28 KB: restriction 31 us, prolongation 17; now 10.4 and 7.8.)
+template <int NQF>
+struct MgTransfer {
+  static constexpr int epb = NQF == 0 || NQF > 6 ? 1 : 256 / (NQF * NQF * NQF);
+  static constexpr int nodes = NQF == 0 ? 12 * 12 * 12 : epb * NQF * NQF * NQF;
+};
+
+// Restriction of an element: res -= Ad (stored), u = w res, then
 // rc[a,b,c] = sum_k J[k][c] sum_j J[j][b] sum_i J[i][a] u[i,j,k]
 // (node index i + j Nq + k Nq^2; fma chains in ascending fine index).
 // NQF, NQC: the orders at compile time (the loops unroll, the index
 // arithmetic folds); 0 takes them from the arguments.  Either way each
-// output is the same fma chain.  Launched with 256 lanes.
+// output is the same fma chain.  Launched with 256 lanes.  At N = 7 bound by
+// memory, 20 bytes a node (53 us at 32768 elements, 6.3 TB/s); the weight from
+// the one-byte degree instead, 13 bytes: 56 us with a division, 63 with a
+// table.
 template <typename V, typename O, int NQF = 0, int NQC = 0>
-__global__ __launch_bounds__(256) void k_mg_restrict(const int nqf, const int nqc, const int32_t offf,
+__global__ __launch_bounds__(256) void k_mg_restrict(const int32_t E, const int nqf, const int nqc, const int32_t offf,
                                                      const int32_t offc, const V* __restrict__ J,
                                                      const double* __restrict__ w, V* __restrict__ res,
-                                                     const V* __restrict__ Ad, O* __restrict__ rc,
-                                                     const int* __restrict__ skip)
+                                                     const V* __restrict__ Ad, O* __restrict__ rc, const int* __restrict__ skip)
 {
+  using M = MgTransfer<NQF>;
   if (skip && *skip) return;
-  __shared__ V s_u[12 * 12 * 12];
-  __shared__ V s_t[12 * 12 * 12];
+  __shared__ V s_u[M::nodes];
+  __shared__ V s_t[M::nodes];
   __shared__ V s_J[12 * 12];
   constexpr int kLanes = 256;
   const int Nqf = NQF ? NQF : nqf, Nqc = NQC ? NQC : nqc;
-  const int64_t e = blockIdx.x;
+  const int64_t e0 = (int64_t)blockIdx.x * M::epb;
+  const int ne = (int)(E - e0 < M::epb ? E - e0 : M::epb);
   const int Npf = Nqf * Nqf * Nqf, Npc = Nqc * Nqc * Nqc;
   for (int q = threadIdx.x; q < Nqf * Nqc; q += kLanes) s_J[q] = J[q];
   const int64_t fo = (int64_t)blockIdx.y * offf, fc = (int64_t)blockIdx.y * offc;  // blockIdx.y = field
-  for (int q = threadIdx.x; q < Npf; q += kLanes) {
-    const int64_t id = e * Npf + q;
+  for (int q = threadIdx.x; q < ne * Npf; q += kLanes) {
+    const int64_t id = e0 * Npf + q;
     const V rq = res[fo + id] - Ad[fo + id];
     res[fo + id] = rq;
     s_u[q] = (V)w[id] * rq;
   }
   __syncthreads();
-  // x: t1[a + Nqc (j + Nqf k)]
-  for (int q = threadIdx.x; q < Nqc * Nqf * Nqf; q += kLanes) {
+  // x: t1[a + Nqc (j + Nqf (k + Nqf element))]
+  for (int q = threadIdx.x; q < ne * Nqc * Nqf * Nqf; q += kLanes) {
     const int a = q % Nqc, jk = q / Nqc;
     V acc = V(0);
     for (int i = 0; i < Nqf; ++i) acc = fmaV<V>(s_J[i * Nqc + a], s_u[i + Nqf * jk], acc);
     s_t[q] = acc;
   }
   __syncthreads();
-  // y: t2[a + Nqc (b + Nqc k)] into s_u
-  for (int q = threadIdx.x; q < Nqc * Nqc * Nqf; q += kLanes) {
+  // y: t2[a + Nqc (b + Nqc (k + Nqf element))] into s_u
+  for (int q = threadIdx.x; q < ne * Nqc * Nqc * Nqf; q += kLanes) {
     const int a = q % Nqc, b = (q / Nqc) % Nqc, k = q / (Nqc * Nqc);
     V acc = V(0);
     for (int j = 0; j < Nqf; ++j) acc = fmaV<V>(s_J[j * Nqc + b], s_t[a + Nqc * (j + Nqf * k)], acc);
     s_u[q] = acc;
   }
   __syncthreads();
-  // z: rc[a + Nqc (b + Nqc c)]
-  for (int q = threadIdx.x; q < Npc; q += kLanes) {
-    const int ab = q % (Nqc * Nqc), c = q / (Nqc * Nqc);
+  // z: rc[a + Nqc (b + Nqc (c + Nqc element))]
+  for (int q = threadIdx.x; q < ne * Npc; q += kLanes) {
+    const int ab = q % (Nqc * Nqc), c = (q / (Nqc * Nqc)) % Nqc, el = q / Npc;
     V acc = V(0);
-    for (int k = 0; k < Nqf; ++k) acc = fmaV<V>(s_J[k * Nqc + c], s_u[ab + Nqc * Nqc * k], acc);
-    rc[fc + e * Npc + q] = (O)acc;
+    for (int k = 0; k < Nqf; ++k) acc = fmaV<V>(s_J[k * Nqc + c], s_u[ab + Nqc * Nqc * (k + Nqf * el)], acc);
+    rc[fc + e0 * Npc + q] = (O)acc;
   }
 }
 
-// Prolongation of one element: v[i,j,k] = sum_c J[k][c] sum_b J[j][b] sum_a J[i][a] xc[a,b,c];
+// Prolongation of an element: v[i,j,k] = sum_c J[k][c] sum_b J[j][b] sum_a J[i][a] xc[a,b,c];
 // d = v (x takes it up with the held directions).
 template <typename V, typename I, int NQF = 0, int NQC = 0>
-__global__ __launch_bounds__(256) void k_mg_prolong(const int nqf, const int nqc, const int32_t offf,
+__global__ __launch_bounds__(256) void k_mg_prolong(const int32_t E, const int nqf, const int nqc, const int32_t offf,
                                                     const int32_t offc, const V* __restrict__ J,
                                                     const I* __restrict__ xc, V* __restrict__ d,
                                                     const int* __restrict__ skip)
 {
+  using M = MgTransfer<NQF>;
   if (skip && *skip) return;
-  __shared__ V s_u[12 * 12 * 12];
-  __shared__ V s_t[12 * 12 * 12];
+  __shared__ V s_u[M::nodes];
+  __shared__ V s_t[M::nodes];
   __shared__ V s_J[12 * 12];
   constexpr int kLanes = 256;
   const int Nqf = NQF ? NQF : nqf, Nqc = NQC ? NQC : nqc;
-  const int64_t e = blockIdx.x;
+  const int64_t e0 = (int64_t)blockIdx.x * M::epb;
+  const int ne = (int)(E - e0 < M::epb ? E - e0 : M::epb);
   const int Npf = Nqf * Nqf * Nqf, Npc = Nqc * Nqc * Nqc;
   for (int q = threadIdx.x; q < Nqf * Nqc; q += kLanes) s_J[q] = J[q];
   const int64_t fo = (int64_t)blockIdx.y * offf, fc = (int64_t)blockIdx.y * offc;  // blockIdx.y = field
-  for (int q = threadIdx.x; q < Npc; q += kLanes) s_u[q] = (V)xc[fc + e * Npc + q];
+  for (int q = threadIdx.x; q < ne * Npc; q += kLanes) s_u[q] = (V)xc[fc + e0 * Npc + q];
   __syncthreads();
-  // x: t1[i + Nqf (b + Nqc c)]
-  for (int q = threadIdx.x; q < Nqf * Nqc * Nqc; q += kLanes) {
+  // x: t1[i + Nqf (b + Nqc (c + Nqc element))]
+  for (int q = threadIdx.x; q < ne * Nqf * Nqc * Nqc; q += kLanes) {
     const int i = q % Nqf, bc = q / Nqf;
     V acc = V(0);
     for (int a = 0; a < Nqc; ++a) acc = fmaV<V>(s_J[i * Nqc + a], s_u[a + Nqc * bc], acc);
     s_t[q] = acc;
   }
   __syncthreads();
-  // y: t2[i + Nqf (j + Nqf c)] into s_u
-  for (int q = threadIdx.x; q < Nqf * Nqf * Nqc; q += kLanes) {
+  // y: t2[i + Nqf (j + Nqf (c + Nqc element))] into s_u
+  for (int q = threadIdx.x; q < ne * Nqf * Nqf * Nqc; q += kLanes) {
     const int i = q % Nqf, j = (q / Nqf) % Nqf, c = q / (Nqf * Nqf);
     V acc = V(0);
     for (int b = 0; b < Nqc; ++b) acc = fmaV<V>(s_J[j * Nqc + b], s_t[i + Nqf * (b + Nqc * c)], acc);
     s_u[q] = acc;
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < Npf; q += kLanes) {
-    const int ij = q % (Nqf * Nqf), k = q / (Nqf * Nqf);
+  for (int q = threadIdx.x; q < ne * Npf; q += kLanes) {
+    const int ij = q % (Nqf * Nqf), k = (q / (Nqf * Nqf)) % Nqf, el = q / Npf;
     V acc = V(0);
-    for (int c = 0; c < Nqc; ++c) acc = fmaV<V>(s_J[k * Nqc + c], s_u[ij + Nqf * Nqf * c], acc);
-    d[fo + e * Npf + q] = acc;
+    for (int c = 0; c < Nqc; ++c) acc = fmaV<V>(s_J[k * Nqc + c], s_u[ij + Nqf * Nqf * (c + Nqc * el)], acc);
+    d[fo + e0 * Npf + q] = acc;
   }
 }
 
@@ -426,7 +442,7 @@ int power_lmax(nbx_bp* bp, uint64_t seed, uint64_t stream_id, int iters, double*
 // workgroup 0, read by the next pass B and pass A).
 //   Pass A: a quad of lanes per element (lane t = i + 2j of the 2 x 2 face,
 //   columns k = 0, 1), 64 elements per 256-lane workgroup; the element
-//   operator is axhelm_column's arithmetic for Nq = 2 with the other lanes'
+//   operator is the element operator's arithmetic for Nq = 2 with the other lanes'
 //   values brought by DPP quad permutes instead of LDS, so no barrier; the
 //   element share is the fused PCG's lane chain (fields, then k) and lane tree
 //   (a0 + a2) + (a1 + a3); the partial is a halving tree over each wave's 16
@@ -539,7 +555,7 @@ __global__ __launch_bounds__(256) void k_cg_pass_a(const int32_t E, const int32_
       pk[kk] = active ? __builtin_fma(beta, pv[f][kk], zv[f][kk]) : 0.0;
       if (active) p[base + kk * 4] = pk[kk];
     }
-    // axhelm_column for Nq = 2 (same operations in the same order)
+    // the element operator for Nq = 2 (same operations in the same order)
     double rAt[2] = {0.0, 0.0}, rArs[2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -779,7 +795,7 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
   nbx_bp* bp = L.bp;
   const int32_t n = bp->Nlocal, off = bp->fieldOffset;
   const dim3 g((unsigned)((n + 255) / 256), (unsigned)bp->Nf), b(256);
-  const dim3 ge((unsigned)bp->E, (unsigned)bp->Nf);
+  auto transfer_grid = [&](int epb) { return dim3((unsigned)((bp->E + epb - 1) / epb), (unsigned)bp->Nf); };
   const int k = mg->degree;
   V* res = static_cast<V*>(L.res);
   V* Ad = static_cast<V*>(L.Ad);
@@ -843,8 +859,8 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
   {
     const double* wv = nbx_ogs_inv_degree(bp->ogs);
 #define NBX_RESTRICT(F, C_)                                                                                  \
-  hipLaunchKernelGGL((k_mg_restrict<V, CV, F, C_>), ge, b, 0, bp->stream, L.Nq, C.Nq, off, C.bp->fieldOffset, \
-                     level_J<V>(L), wv, res, Ad, rcv, skip)
+  hipLaunchKernelGGL((k_mg_restrict<V, CV, F, C_>), transfer_grid(MgTransfer<F>::epb), b, 0, bp->stream, bp->E,   \
+                     L.Nq, C.Nq, off, C.bp->fieldOffset, level_J<V>(L), wv, res, Ad, rcv, skip)
     if (L.Nq == 8 && C.Nq == 4) NBX_RESTRICT(8, 4);
     else if (L.Nq == 4 && C.Nq == 2) NBX_RESTRICT(4, 2);
     else if (L.Nq == 10 && C.Nq == 5) NBX_RESTRICT(10, 5);
@@ -860,8 +876,8 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
   // coarse correction
   V* v = free_buffer();
 #define NBX_PROLONG(F, C_)                                                                                 \
-  hipLaunchKernelGGL((k_mg_prolong<V, CV, F, C_>), ge, b, 0, bp->stream, L.Nq, C.Nq, off, C.bp->fieldOffset, \
-                     level_J<V>(L), static_cast<const CV*>(C.x), v, skip)
+  hipLaunchKernelGGL((k_mg_prolong<V, CV, F, C_>), transfer_grid(MgTransfer<F>::epb), b, 0, bp->stream, bp->E,  \
+                     L.Nq, C.Nq, off, C.bp->fieldOffset, level_J<V>(L), static_cast<const CV*>(C.x), v, skip)
   if (L.Nq == 8 && C.Nq == 4) NBX_PROLONG(8, 4);
   else if (L.Nq == 4 && C.Nq == 2) NBX_PROLONG(4, 2);
   else if (L.Nq == 10 && C.Nq == 5) NBX_PROLONG(10, 5);
