@@ -944,7 +944,7 @@ def main():
                    "time_to_1e-8": compare, "mesh16": mesh16},
         "roofline": {"bound": "hbm", "achieved": round(ax_gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(ax_gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_axhelm_bk8_split", "bytes_per_launch": ax_bytes,
+                     "kernel": "k_axhelm", "bytes_per_launch": ax_bytes,
                      "us_per_launch": round(ax_s * 1e6, 3), "buffer_sets": ROOF_SETS,
                      "timing": "per-launch HIP events, 2 ms idle before each launch",
                      "us_per_launch_back_to_back": round(ax_b2b_s * 1e6, 3),

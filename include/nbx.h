@@ -376,10 +376,11 @@ int nbx_net_train_energy(nbx_net* net, nbx_bp* bp, int steps, float lr, uint64_t
  * timer tags of nekBone/solve.cpp:71-109).  With profiling on, every PCG
  * solve records events at its phase boundaries and accumulates device time
  * per phase: seconds[0] local Ax (with the fused p = z + beta p and the pAp
- * shares), [1] gs (gather-scatter + mask), [2] updatePCG (x, r update, and
- * with COPY/JACOBI the preconditioner and the dots' tile partials, fused into
- * one pass), [3] dot (the reductions' finishing passes; with MG/LEARNED also
- * the dots), [4] preco (the V-cycle or the network with its assembly).
+ * shares), [1] gs (gather-scatter + mask, in the fused schedule with the finish
+ * of pAp), [2] updatePCG (x, r update, and with COPY/JACOBI the preconditioner
+ * and the dots' tile partials, fused into one pass; with MG/LEARNED those of
+ * <r, r>), [3] dot (the reductions' finishing passes; with MG/LEARNED also
+ * the other dots), [4] preco (the V-cycle or the network with its assembly).
  * The events add a little time to each phase.  reset != 0 zeroes the sums. */
 int nbx_bp_set_profiling(nbx_bp* bp, int on);
 int nbx_bp_profile(nbx_bp* bp, double* seconds, int reset);

@@ -306,6 +306,8 @@ __device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[
 // N = 7 BK (129 registers; 32768 elements 177 against 179 us).  N = 12 non-BK
 // is held to the 168 registers of three waves (204 against 213 us); at higher
 // orders that spills.
+// The one-field FP64 non-BK form at N = 10 is the one that the column form was
+// faster in (8e6 nodes 120 us, 131 here; two slabs in flight: the same).
 template <typename T, int NQ, bool BK>
 struct AxShape {
   static constexpr bool f64 = sizeof(T) == 8;

@@ -1,5 +1,5 @@
-"""Gather-scatter on both sides of the line between one lane per group for all
-fields and a row of lanes per field: pairs, triples, quads and octets in one
+"""Gather-scatter of one to seven fields (a grid row each), from a few groups to
+more than the chip holds at once: pairs, triples, quads and octets in one
 list, singletons and excluded nodes between them."""
 import numpy as np
 import pytest
@@ -7,7 +7,6 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# the line lies at 524288 lanes, one per group
 @pytest.mark.parametrize("groups", [5, 60000, 700000])
 @pytest.mark.parametrize("k", [1, 2, 3, 7])
 @pytest.mark.parametrize("type_,dtype,op", [("double", np.float64, "add"), ("int", np.int32, "min"),
