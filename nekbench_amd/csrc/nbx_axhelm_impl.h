@@ -274,6 +274,12 @@ __device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[
         ar[i] = fmaT(R.d[i], gr, ar[i]);
         as[i] = fmaT(R.d[i], gs, as[i]);
       }
+      // the step's sums are opaque here: otherwise nothing holds the products
+      // to their step, they move behind the last row's loads, and every row of
+      // D spills (126 scalar registers in vector lanes for FP64 Helmholtz at
+      // N = 9, 464 at N = 15; 0 and 16 now; N = 9, 1e6 nodes: 18.2 -> 17.4 us)
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) asm volatile("" : "+v"(ar[i]), "+v"(as[i]));
       R = Rn;
       gr = grn;
       gs = gsn;
