@@ -154,8 +154,9 @@ struct GeoKept {
 // (or k) in increasing order, as the oracle has it.
 // rq: q of the lane's column on entry; after_forward() may replace it (the
 // next field's); q_again(mq) gives q once more for the mass term, before the
-// transposed contractions or, with LATE, after them.
-template <typename T, int NQ, bool BK, bool LATE = false, typename GEO, typename F1, typename F2>
+// transposed contractions or, with LATE, after them.  EARLY: the first slabs of
+// factors are fetched before the forward contractions (AxShape::early).
+template <typename T, int NQ, bool BK, bool LATE = false, bool EARLY = false, typename GEO, typename F1, typename F2>
 __device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[NQ], ConstPtr<T> D, T* s_r, T* s_s,
                                              GEO& geo, F1&& after_forward, F2&& q_again)
 {
@@ -179,6 +180,7 @@ __device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[
       qm[m] = lq[m * RS];
     }
     __syncthreads();
+    if (EARLY) geo.begin();
     DRow<T, NQ> R, Rn;
     R.load(D, 0);
     T qr, qs;
@@ -214,7 +216,7 @@ __device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[
   after_forward();
   __syncthreads();
   {
-    geo.begin();
+    if (!EARLY) geo.begin();
     DRow<T, NQ> R, Rn;
     R.load(D, 0);
     T qr = nr[0], qs = ns[0], qrn, qsn;
@@ -307,19 +309,38 @@ __device__ __forceinline__ void axhelm_lines(const int t, T (&rq)[NQ], T (&out)[
 // Elements per workgroup (threadIdx.y = slot): enough to fill two to four
 // waves with few idle lanes, no more (a workgroup's waves wait for each other
 // at five barriers; N = 1 with 64 instead of 32 elements cost 8 % at 37500).
-// Slabs of factors in flight: four; two where FP64 would drop below three
-// waves per SIMD (N = 11 non-BK, 12e6 nodes: 195 against 219 us); all eight at
-// N = 7 BK (129 registers; 32768 elements 177 against 179 us).  N = 12 non-BK
-// is held to the 168 registers of three waves (204 against 213 us); at higher
-// orders that spills.
-// The one-field FP64 non-BK form at N = 10 is the one that the column form was
-// faster in (8e6 nodes 120 us, 131 here; two slabs in flight: the same).
-template <typename T, int NQ, bool BK>
+// ahead: slabs of factors in flight, four; two where FP64 would drop below
+// three waves per SIMD; all eight at N = 7 FP64 Poisson (177 against 179 us for
+// 32768 elements); six at N = 10 FP64 Helmholtz (one field, 2e6 nodes: 33.0
+// against 35 us with four); eight at N = 11 with bf16 geometry, Helmholtz
+// (1e6 nodes 13.4 -> 11.6 us, 8e6 49.7 -> 47.0; Poisson gains at 1e6 only and
+// loses 6 to 13 % from 8e6 on).
+// early: the first slabs are fetched before the forward contractions, so that
+// memory works during them, and q through the caches (a solver has just
+// written it).  One field, us, fetched after them with nontemporal q / now
+// (the column form that preceded the line form in brackets), 8e6 nodes:
+//   FP64 Poisson    N = 7  81.6 / 77.0 (84.0)    N = 9  91.2 / 83.0 (99.8)
+//                   N = 10 97.1 / 86.1 (94.5)
+//   FP64 Helmholtz  N = 9  127.4 / 116.2 (123.6) N = 10 130.1 / 119.5 (119.3)
+//   FP32 Poisson    N = 7  41.1 / 40.1 (41.8), 17e6 87.3 / 82.3 (84.2)
+//                   N = 10 49.6 / 45.1 (47.9)
+//   FP32 Helmholtz  N = 10 68.1 / 63.7 (65.0)
+// N = 11 and 13 FP64 lose 3 to 6 % by it (their registers leave two waves),
+// and bf16 geometry has fewer bytes to wait for (0 to 17 % slower).
+// Slower than the column form are only FP64 Helmholtz at N = 10 on half of
+// 8e6 nodes by a list (63.7 against 62.0 us), and on 17e6 nodes in buffers that
+// no cache holds (266 against 262), and bf16 Poisson at N = 11 on 1e6 nodes
+// (12.2 against 12.0).
+template <typename T, int NQ, bool BK, typename G = T>
 struct AxShape {
   static constexpr bool f64 = sizeof(T) == 8;
   static constexpr int epb = NQ == 2 ? 32 : NQ == 3 ? 14 : NQ == 4 ? 8 : NQ == 5 ? 5 : NQ == 6 ? 3 : 1;
-  static constexpr int ahead = f64 && (NQ >= 12 || (NQ == 9 && !BK)) ? 2 : f64 && NQ == 8 && BK ? 8 : 4;
-  static constexpr int waves = f64 && NQ == 13 && !BK ? 3 : 1;
+  static constexpr int ahead = f64 && (NQ >= 12 || (NQ == 9 && !BK))       ? 2
+                               : f64 && NQ == 11 && !BK                    ? 6
+                               : (f64 && NQ == 8 && BK)                    ? 8
+                               : (sizeof(G) == 2 && NQ == 12 && !BK)       ? 8
+                                                                           : 4;
+  static constexpr bool early = sizeof(G) != 2 && NQ <= 11;
 };
 // Three fields: the element's factors kept in registers for all of them
 // (k_axhelm_kept) against one workgroup per field (k_axhelm), whose second
@@ -393,12 +414,13 @@ struct ElemPlace {
 // follow each other on one XCD (workgroup b runs on XCD b % 8), so its L2
 // serves the factors to the second and third.
 template <typename T, int NQ, int NF, bool BK, bool PARTIAL, typename G>
-__global__ __launch_bounds__((NQ * NQ * AxShape<T, NQ, BK>::epb), (AxShape<T, NQ, BK>::waves)) void k_axhelm(
+__global__ __launch_bounds__((NQ * NQ * AxShape<T, NQ, BK>::epb)) void k_axhelm(
     const int32_t Nelements, const int32_t offset, const int32_t* __restrict__ elementList,
     const G* __restrict__ ggeo, const T* __restrict__ D, const G* __restrict__ lambda, const T* __restrict__ q,
     T* __restrict__ Aq, const int* __restrict__ skip)
 {
-  using S = AxShape<T, NQ, BK>;
+  using S = AxShape<T, NQ, BK, G>;
+  constexpr bool EARLY = NF == 1 && S::early;
   using LL = LineLayout<T, NQ>;
   constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = S::epb;
   if (skip && *skip) return;
@@ -421,8 +443,8 @@ __global__ __launch_bounds__((NQ * NQ * AxShape<T, NQ, BK>::epb), (AxShape<T, NQ
   T* Af = Aq + E.base * NP + (int64_t)f * offset;
   T rq[NQ], out[NQ];
 #pragma unroll
-  for (int k = 0; k < NQ; ++k) rq[k] = ldnt(&qf[lo + k * NQ2]);
-  axhelm_lines<T, NQ, BK>(
+  for (int k = 0; k < NQ; ++k) rq[k] = EARLY ? qf[lo + k * NQ2] : ldnt(&qf[lo + k * NQ2]);
+  axhelm_lines<T, NQ, BK, false, EARLY>(
       t, rq, out, (ConstPtr<T>)D, s_r[slot], s_s[slot], geo, []() {},
       [&](T(&mq)[NQ]) {
 #pragma unroll
@@ -571,7 +593,7 @@ template <int NQ, int NF, bool BK, typename T, typename G, int FORM>
 struct AxPcg {
   static constexpr bool kept = NF == 3 && FORM == kInTurn && AxKept<T, NQ, BK>::value;
   static constexpr int epb = FORM != kInTurn ? 1 : kept ? AxKept<T, NQ, BK>::epb : AxShape<T, NQ, BK>::epb;
-  static constexpr int waves = kept ? AxKept<T, NQ, BK>::waves : NF == 1 ? AxShape<T, NQ, BK>::waves : 1;
+  static constexpr int waves = kept ? AxKept<T, NQ, BK>::waves : 1;
   // the next field's z and p in flight during the current one, where the registers allow it
   static constexpr bool prefetch = kept && (sizeof(T) == 4 || NQ <= 8);
   static constexpr bool late = NF == 3 && FORM == kInTurn && !prefetch;
@@ -650,7 +672,7 @@ __global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FORM>::epb * (FO
             }
           });
       if (SUMS) acc = 0.0;
-      if (FG && !SUMS) {  // the chain over fields then k: each group continues the previous one's
+      if constexpr (FG && !SUMS) {  // the chain over fields then k: each group continues the previous one's
         for (int c = 0; c < NF; ++c) {
           if (c == y) {
             acc = c == 0 ? 0.0 : s_acc[c - 1][t];
