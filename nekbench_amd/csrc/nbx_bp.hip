@@ -18,8 +18,9 @@
 //   4. Ap = gs(Ap), Ap[mask] = 0               (BPAxOperator: oogs::start/finish; mask)
 //   5. pAp = <p,Ap>_w, one-block finish: alpha = rdotz/pAp (BPWeightedInnerProduct)
 // With the fused operator the shares of pAp come from pass 3 and the finish of
-// 5 runs beside 4.  Multigrid and learned preconditioners: the update, <r,r>_w
-// and the stopping test, then z = M r, then the other dots.
+// 5 runs beside 4.  Multigrid: the update, <r,r>_w and the stopping test, then
+// z = M r, then the other dots.  Learned: the update, z = M r, then every dot's
+// finish and the stopping test.
 // Moving the update into the next iteration's first pass changes no value:
 // every element-wise operation is the same single fma in the same order.
 // The dots use the fixed reduction tree of nbx_reduce.h.  The CPU oracle
@@ -331,10 +332,10 @@ __global__ __launch_bounds__(256) void k_pcg_finish_pap(const unsigned int nb, c
 }
 
 // Multigrid and learned preconditioners: x += alpha p, r -= alpha Ap of the
-// previous iteration (BPUpdatePCG) and the tile partials of <r,r>_w, so that
-// the stopping test comes before the preconditioner: the cycle of the
-// iteration that has converged is not run (one of ten at 32768 elements,
-// 1e-8).  Each lane issues the loads of four nodes and a field together.
+// previous iteration (BPUpdatePCG) and the tile partials of <r,r>_w.  With
+// multigrid the stopping test follows at once: the cycle of the iteration
+// that has converged is not run (one of ten at 32768 elements, 1e-8).  Each
+// lane issues the loads of four nodes and a field together.
 template <bool DEG>
 __global__ __launch_bounds__(256) void k_pcg_update_rr(const int32_t N, const int32_t offset, const int Nf,
                                                        const double* __restrict__ w, const uint8_t* __restrict__ deg,
@@ -442,14 +443,17 @@ __global__ __launch_bounds__(256) void k_pcg_dots_z(const int32_t N, const int32
   store_partials<2>(v, partials);
 }
 
+// RR: <r,r>_w is still to be finished too (its partials behind the others)
+template <bool RR>
 __global__ __launch_bounds__(256) void k_pcg_finish_rz(const unsigned int nb, const double* __restrict__ partials,
-                                                       PcgScalars* S, const double* __restrict__ hist_rdotr)
+                                                       PcgScalars* S, double* __restrict__ hist_rdotr)
 {
   if (S->done) return;
-  __shared__ double s4[2 * 4];
-  double v[2];
-  combine_partials<2>(v, partials, nb, s4);
-  if (threadIdx.x == 0) pcg_after_rz(S, v[0], v[1], hist_rdotr);
+  constexpr int NV = RR ? 3 : 2;
+  __shared__ double s4[NV * 4];
+  double v[NV];
+  combine_partials<NV>(v, partials, nb, s4);
+  if (threadIdx.x == 0 && (!RR || pcg_after_rr(S, v[NV - 1], hist_rdotr))) pcg_after_rz(S, v[0], v[1], hist_rdotr);
 }
 
 // vecInv (nekBone/kernel/utils.okl:605-613)
@@ -729,22 +733,30 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
   const uint8_t* deg = ogs_degree(bp->ogs);
   const double* zsrc = jac ? bp->z : r;
   if (o.precon == NBX_PRECON_LEARNED || o.precon == NBX_PRECON_MG) {
-    // update and stopping test; z = M r (learned: gs(w invDiag (r + s f(r))),
-    // Jacobi after a stall; multigrid: one V-cycle); dots; finish
+    // update and the partials of <r,r>; z = M r (learned: gs(w invDiag (r + s
+    // f(r))), Jacobi after a stall; multigrid: one V-cycle); the other dots.
+    // A cycle is long: its stopping test comes before it.  The network's step is
+    // not: its test waits for the other dots, so that one kernel finishes all
+    // three (a finish of its own before the network: 30 iterations of 8
+    // elements 1193 -> 1366 us, of 512 elements 1548 -> 1620).
+    const bool early = o.precon == NBX_PRECON_MG;
+    double* rr = early ? bp->red.partials : bp->red.partials + 2 * (size_t)nb;
     if (deg)
       hipLaunchKernelGGL(k_pcg_update_rr<true>, dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, bp->fieldOffset,
-                         bp->Nf, w, deg, bp->p, bp->Ap, x, r, bp->red.partials, bp->S);
+                         bp->Nf, w, deg, bp->p, bp->Ap, x, r, rr, bp->S);
     else
       hipLaunchKernelGGL(k_pcg_update_rr<false>, dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, bp->fieldOffset,
-                         bp->Nf, w, deg, bp->p, bp->Ap, x, r, bp->red.partials, bp->S);
+                         bp->Nf, w, deg, bp->p, bp->Ap, x, r, rr, bp->S);
     prof_mark(bp, kProfUpdate);
-    hipLaunchKernelGGL(k_pcg_finish_rr, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
-                       bp->hist_rdotr, &bp->hS->done);
-    NBX_HIP_LAUNCH();
-    prof_mark(bp, kProfDot);
-    NBX_HIP(hipEventRecord(bp->ev_test, bp->stream));
+    if (early) {
+      hipLaunchKernelGGL(k_pcg_finish_rr, dim3(1), dim3(256), 0, bp->stream, nb, rr, bp->S, bp->hist_rdotr,
+                         &bp->hS->done);
+      NBX_HIP_LAUNCH();
+      prof_mark(bp, kProfDot);
+      NBX_HIP(hipEventRecord(bp->ev_test, bp->stream));
+    }
     int rc;
-    if (o.precon == NBX_PRECON_MG) {
+    if (early) {
       if ((rc = mg_apply(bp, r, bp->z, &bp->S->done))) return rc;
     } else {
       if ((rc = net_apply_learned(bp, r, bp->z, &bp->S->fallback, &bp->S->done))) return rc;
@@ -759,8 +771,12 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
     else
       hipLaunchKernelGGL(k_pcg_dots_z<false>, dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, bp->fieldOffset,
                          bp->Nf, w, deg, r, bp->z, bp->Ap, bp->red.partials, bp->S);
-    hipLaunchKernelGGL(k_pcg_finish_rz, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
-                       bp->hist_rdotr);
+    if (early)
+      hipLaunchKernelGGL(k_pcg_finish_rz<false>, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
+                         bp->hist_rdotr);
+    else
+      hipLaunchKernelGGL(k_pcg_finish_rz<true>, dim3(1), dim3(256), 0, bp->stream, nb, bp->red.partials, bp->S,
+                         bp->hist_rdotr);
     NBX_HIP_LAUNCH();
     prof_mark(bp, kProfDot);
     zsrc = bp->z;

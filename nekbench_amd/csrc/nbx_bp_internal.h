@@ -73,7 +73,7 @@ struct nbx_bp {
   int hist_cap = 0;
   int last_iters = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  hipEvent_t ev_test = nullptr;  // an iteration's stopping test (multigrid, learned)
+  hipEvent_t ev_test = nullptr;  // an iteration's stopping test (multigrid)
   // learned preconditioner (attached network, features, per-element output)
   nbx_net* net = nullptr;
   nbx_mg* mg = nullptr;     // p-multigrid preconditioner (levels own their handles)
