@@ -738,7 +738,7 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
     // A cycle is long: its stopping test comes before it.  The network's step is
     // not: its test waits for the other dots, so that one kernel finishes all
     // three (a finish of its own before the network: 30 iterations of 8
-    // elements 1193 -> 1366 us, of 512 elements 1548 -> 1620).
+    // elements 1366 us against 1139, of 512 elements 1620 against 1444).
     const bool early = o.precon == NBX_PRECON_MG;
     double* rr = early ? bp->red.partials : bp->red.partials + 2 * (size_t)nb;
     if (deg)

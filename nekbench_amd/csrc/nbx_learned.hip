@@ -573,6 +573,9 @@ extern "C" int nbx_net_set_pairs(nbx_net* n, nbx_bp* bp, int npairs, const float
   return NBX_SUCCESS;
 }
 
+// chunks of a batch (a chunk may be any positive int, so not nsamples + chunk - 1)
+static int chunk_count(int nsamples, int chunk) { return (nsamples - 1) / chunk + 1; }
+
 static int ensure_work(nbx_net* n, int nsamples, int chunk)
 {
   if (nsamples > n->sample_cap) {
@@ -581,7 +584,7 @@ static int ensure_work(nbx_net* n, int nsamples, int chunk)
     NBX_HIP(hipMalloc(&n->samples, sizeof(int2) * nsamples));
     n->sample_cap = nsamples;
   }
-  const int nblocks = (nsamples + chunk - 1) / chunk;
+  const int nblocks = chunk_count(nsamples, chunk);
   if (nblocks > n->partial_cap) {
     if (n->partials) (void)hipFree(n->partials);
     n->partials = nullptr;
@@ -602,7 +605,7 @@ static int ensure_work(nbx_net* n, int nsamples, int chunk)
 // gradient over the nsamples samples already in n->samples (G: energy mode)
 static int run_gradient(nbx_net* n, nbx_bp* bp, int nsamples, int chunk, const double* G = nullptr)
 {
-  const int nblocks = (nsamples + chunk - 1) / chunk;
+  const int nblocks = chunk_count(nsamples, chunk);
   for (int first = 0; first < nsamples; first += kNetBatch) {
     int rc = net_train_launch(first, std::min(kNetBatch, nsamples - first), chunk, n->samples, n->pairStride, n->R,
                               n->Ev, n->invNorm, n->wbf, bp->feat, bp->invDiagA, G, n->grads, n->partials, bp->stream);
@@ -612,7 +615,8 @@ static int run_gradient(nbx_net* n, nbx_bp* bp, int nsamples, int chunk, const d
 }
 
 // Gradient of the training loss over the given (pair, element) samples, in
-// the library's fixed order (chunk samples per workgroup); host outputs.
+// the library's fixed order (sums of chunk samples, then of the chunks); host
+// outputs.
 extern "C" int nbx_net_gradient(nbx_net* n, nbx_bp* bp, const int32_t* samples, int nsamples, int chunk,
                                 const double* G, float* grad_host, double* loss_host)
 {

@@ -1,0 +1,36 @@
+"""Parameter gradients at the limits of their arguments: chunks up to the
+largest int, and element outputs whose derivative is not finite."""
+import numpy as np
+import pytest
+
+from test_gpu_net import make, net_with, random_net
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def case(nbx, nbo, dev):
+    import torch
+    bp, ob = make(nbx, nbo, dims=(2, 1, 1))
+    rng = np.random.default_rng(11)
+    W = nbo.bf16_round(random_net(rng))
+    net = net_with(nbx, nbo, bp, W)
+    n = bp.fieldOffset
+    R = (rng.standard_normal((2, n)) * 1e-2).astype(np.float32)
+    Ev = (rng.standard_normal((2, n)) * 1e-1).astype(np.float32)
+    net.set_pairs(bp, torch.tensor(R, device=dev), torch.tensor(Ev, device=dev))
+    invNorm = np.array([nbo.sumsq_inv_f(e) for e in Ev])
+    feat = nbo.net_features(ob.E, 512, ob.mesh["ggeo"])
+    samples = np.stack([rng.integers(0, 2, 5), rng.integers(0, 2, 5)], axis=1).astype(np.int32)
+
+    def oracle(s, chunk, G=None):
+        return nbo.net_gradient(s, chunk, n, R.ravel(), Ev.ravel(), invNorm, W, feat, ob.invdiag(), G=G)
+    return bp, net, samples, n, oracle
+
+
+@pytest.mark.parametrize("chunk", [5, 6, 2 ** 31 - 5, 2 ** 31 - 1])
+def test_chunk_past_the_batch(case, chunk):
+    bp, net, samples, _, oracle = case
+    g, loss = net.gradient(bp, samples, chunk)
+    og, oloss = oracle(samples, 5)
+    assert np.array_equal(g, og) and loss == oloss
