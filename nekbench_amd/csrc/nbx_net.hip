@@ -201,6 +201,7 @@ struct TrainLds {
   float g[kG * kFRow];             // factors, node (x, y, z) at 100 z + 10 y + x
   float buf[kTrainRows * kTrainRow];  // T exchange, then 128 nodes of the channels
   double red[kP / 64];
+  int nonfinite;                   // dL/dpre1 of some node and channel
 };
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
@@ -264,6 +265,33 @@ __device__ __forceinline__ void relu(NodeChannels& h)
   });
 }
 
+// Rows row .. row + 3 of the first layer's gradient (taps, then factors), one
+// channel, over the 128 nodes of the planes k0 and k0 + 1, where some dL/dpre1
+// is not finite: a tap whose neighbour lies outside of the element takes no
+// part, while the products would multiply its padding, and 0 inf is not 0.
+__device__ __noinline__ void taps_in_range(const TrainLds& lds, const int row, const int channel, const int k0,
+                                           f32x4& acc)
+{
+#pragma unroll 1
+  for (int u = 0; u < 4; ++u) {
+    const int r = row + u, tap = min(r, kTaps - 1);
+    const int dx = r < kTaps ? tap % 3 - 1 : 0, dy = r < kTaps ? (tap / 3) % 3 - 1 : 0, dz = r < kTaps ? tap / 9 - 1 : 0;
+    const float* const a = r < kTaps ? lds.rh + tap_place(tap) : lds.g + (r - kTaps) * kFRow;
+    float v = u == 0 ? acc[0] : u == 1 ? acc[1] : u == 2 ? acc[2] : acc[3];
+#pragma unroll 1
+    for (int m = 0; m < 128; ++m) {
+      const int i = m & 7, j = (m >> 3) & 7, k = k0 + (m >> 6);
+      const bool in = (unsigned)(i + dx) < 8u && (unsigned)(j + dy) < 8u && (unsigned)(k + dz) < 8u;
+      const float b = lds.buf[channel * kTrainRow + (m & ~15) + 4 * (m & 3) + ((m & 15) >> 2)];
+      if (in) v = __builtin_fmaf(a[100 * k + 10 * j + i], b, v);
+    }
+    if (u == 0) acc[0] = v;
+    else if (u == 1) acc[1] = v;
+    else if (u == 2) acc[2] = v;
+    else acc[3] = v;
+  }
+}
+
 __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ samples, const int64_t pairStride,
                                                       const float* __restrict__ R, const float* __restrict__ Ev,
                                                       const double* __restrict__ invNorm, const float* __restrict__ W,
@@ -284,6 +312,7 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
   const double en = G ? 0.0 : (double)Ev[off];
   const double di = invDiag[e * kP + n];
   for (int q = n; q < kPadN; q += kP) lds.rh[q] = lds.dy[q] = 0.f;
+  if (n == 0) lds.nonfinite = 0;
 #pragma unroll
   for (int q = 0; q < kG; ++q) lds.g[q * kFRow + place] = feat[(e * kG + q) * kP + n];
   const double s = element_scale(rn, lds.red);  // its barrier also ends the zero fill
@@ -440,6 +469,11 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
   layer<kC / 4, 8>([&](int t, int m) { return W2[(16 * m + ch) * kC + 4 * t + kg]; },
                 [&](int t, int tt) { return d2.v[tt][t >> 2][t & 3]; }, d1);
   each_channel([&](int tt, int m, int u) { d1.v[tt][m][u] = h1.v[tt][m][u] > 0.f ? d1.v[tt][m][u] : 0.f; });
+  {
+    float zero = 0.f;  // not zero where a value is not finite
+    each_channel([&](int tt, int m, int u) { zero = __builtin_fmaf(d1.v[tt][m][u], 0.f, zero); });
+    if (!(zero == 0.f)) lds.nonfinite = 1;
+  }
   // phase 2: waves 0..5 the 35 rows of Wr, Wg, b1 (three row tiles), waves 6, 7 b2
   {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -456,6 +490,10 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
         put(kC, d2);
       }
       __syncthreads();
+      if (rt < 2 && lds.nonfinite) {
+        taps_in_range(lds, 16 * rt + 4 * kg, 16 * ct + col, 2 * h, acc);
+        continue;
+      }
       const float* const b = lds.buf + ((rt == 3 ? kC : 0) + 16 * ct) * kTrainRow + rd;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {

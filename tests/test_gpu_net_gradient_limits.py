@@ -34,3 +34,19 @@ def test_chunk_past_the_batch(case, chunk):
     g, loss = net.gradient(bp, samples, chunk)
     og, oloss = oracle(samples, 5)
     assert np.array_equal(g, og) and loss == oloss
+
+
+# a derivative that is not finite reaches the parameters of the taps whose
+# neighbour lies in the element, and no others
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, 1e43])
+@pytest.mark.parametrize("node", [0, 7, 56 + 448, 511, 8 * 3, 64 * 3 + 8 * 4 + 4])
+def test_derivative_that_is_not_finite(case, dev, value, node):
+    import torch
+    bp, net, _, n, oracle = case
+    G = np.random.default_rng(node).standard_normal(n)
+    G[512 + node] = value
+    samples = np.array([[0, 1], [1, 0]], dtype=np.int32)
+    g, _ = net.gradient(bp, samples, 16, G=torch.tensor(G, device=dev))
+    og, _ = oracle(samples, 16, G=G)
+    assert np.isfinite(og).sum() < og.size
+    assert np.array_equal(g, og, equal_nan=True)
