@@ -292,6 +292,10 @@ int nbx_bp_pcg_mixed(nbx_bp* bp, const double* lambda, double* r, double* x, dou
  * cycle reads the FP64 residual and returns an FP64 correction; the coarse
  * PCG is FP64).  One or three fields (one Jacobi diagonal and lambda_max for
  * all fields; bf16 geometry: one field), N <= 11.  Uses the handle's lambda.
+ * Memory per fine node and field beside the coarse handles (about a seventh of
+ * the fine one's): vectors of the cycle's precision, three and up to 2 degree -
+ * 2 (at most 7) more if they fit into an eighth of the free memory; with FP32
+ * or bf16 cycles 9 values of geometry and lambda in that type and the diagonal.
  * Not for the singular all-Neumann problem (nbx_bp_all_neumann). */
 int nbx_bp_mg_setup(nbx_bp* bp, int nlevels, const int* orders, int degree, int coarse_iters, double lo, double hi,
                     nbx_prec prec);
@@ -356,7 +360,8 @@ int nbx_net_generate_mg_pairs(nbx_net* net, nbx_bp* bp, int nseeds, uint64_t see
  * local-vector length each */
 int nbx_net_copy_pairs(const nbx_net* net, int first, int count, float* R, float* E);
 /* loss sum_samples sum_n (z - e)^2 / sum_pair e^2 and its parameter gradient
- * over (pair, element) samples (host int pairs), chunk samples per workgroup.
+ * over (pair, element) samples (host int pairs), summed in chunks of chunk
+ * samples; the network keeps up to 4096 samples' gradients (50 MB).
  * G (device, local vector, may be NULL): when given, the loss is external and
  * G[e*Np+n] is its derivative with respect to the unweighted element output
  * invDiag (r + s f(r)); the returned loss is then 0 */

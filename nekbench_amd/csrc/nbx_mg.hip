@@ -59,7 +59,10 @@ struct nbx_mg_level {
   // vectors of the cycle's precision (double or float); the last level's r
   // and x are double (its PCG); level 0 reads r and writes x of the solver
   void *r = nullptr, *x = nullptr, *res = nullptr, *Ad = nullptr;
-  void* d[nbx::kMgHeld + 1] = {};  // directions (those held and the one being formed)
+  // directions (those held and the one being formed): nd of them, two at least;
+  // the second is the handle's Ax, which nothing uses during a cycle
+  void* d[nbx::kMgHeld + 1] = {};
+  int nd = 0;
   double* J = nullptr;  // [Nq][Nq of level l+1]: interpolation from the next coarser level
   float* J32 = nullptr;
   float* invD32 = nullptr;  // FP32 Jacobi diagonal (FP32 / bf16 cycles)
@@ -107,8 +110,8 @@ __device__ __forceinline__ float fmaV<float>(float a, float b, float c) { return
 
 // Directions of a cycle that its solution has not taken up yet, in order.
 // x is not read and written at every smoothing step: each step leaves its
-// direction in a buffer of its own, and the last one (or one that would exceed
-// kHeld buffers) adds them all, x = ((x + d_1) + d_2) + ... as the steps would
+// direction in a buffer of its own, and the last one (or one that finds no
+// free buffer) adds them all, x = ((x + d_1) + d_2) + ... as the steps would
 // have.  Per node and FP32 cycle of degree 3 with an FP64 x: 104 bytes of x and
 // 8 of the last residual and direction become 32.
 constexpr int kHeld = kMgHeld;
@@ -815,7 +818,8 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
   auto smooth = [&](int s, bool post, bool last) {
     const bool first_post = post && s == 0;
     const V c1 = first_post ? V(0) : (V)L.c1[s], c2 = (V)L.c2[s];
-    if (last || H.n >= (post ? kHeld : kHeld - 1)) {  // before the coarse correction one stays free for it
+    // before the coarse correction one buffer stays free for it
+    if (last || H.n >= (post ? kHeld : kHeld - 1) || used >= (post ? L.nd : L.nd - 1)) {
 #define NBX_SUM(MODE, KEEP)                                                                                         \
   hipLaunchKernelGGL((k_cheb_sum<MODE, V, X, KEEP>), g, b, 0, bp->stream, n, off, c1, c2, invD, res, Ad, d, d, H, x, \
                      skip)
@@ -831,7 +835,7 @@ int vcycle_level(nbx_mg* mg, int l, const R* r, X* x, const int* skip)
       H.n = 0;
       H.started = 1;
       // the held buffers are free again, all but the one d sits in
-      std::swap(L.d[0], *std::find(L.d, L.d + kHeld + 1, static_cast<void*>(d)));
+      std::swap(L.d[0], *std::find(L.d, L.d + L.nd, static_cast<void*>(d)));
       used = 1;
       return;
     }
@@ -1007,6 +1011,29 @@ static int mg_capture(nbx_mg* mg, nbx_bp* bp, const double* r, double* z, const 
   return NBX_SUCCESS;
 }
 
+// A level's direction buffers.  Two are enough for any degree; a cycle's 2
+// degree - 1 directions before the last (or kMgHeld and the one being formed)
+// save it the passes over x between them, for a vector each: they are taken
+// from an eighth of the free memory at most, so that a mesh that fills the
+// card still fits with its solution and right-hand side.
+static int mg_directions(nbx_mg* mg, nbx_mg_level& L, size_t es)
+{
+  nbx_bp* b = L.bp;
+  int rc;
+  if ((rc = mg_alloc(mg, &L.d[0], b->Nall, es))) return rc;
+  L.d[1] = b->Ax;
+  L.nd = 2;
+  const size_t bytes = es * (size_t)std::max<int64_t>(b->Nall, 1);
+  size_t avail = 0, total = 0;
+  NBX_HIP(hipMemGetInfo(&avail, &total));
+  const size_t more = std::min<size_t>(avail / 8 / bytes, std::min(2 * mg->degree, kMgHeld + 1) - L.nd);
+  for (size_t q = 0; q < more; ++q) {
+    if ((rc = mg_alloc(mg, &L.d[L.nd], b->Nall, es))) return rc;
+    ++L.nd;
+  }
+  return NBX_SUCCESS;
+}
+
 int mg_apply_direct(nbx_bp* bp, const double* r, double* z)
 {
   if (!bp->mg) return fail(NBX_ERR_INVALID, "multigrid preconditioner: not set up (nbx_bp_mg_setup)");
@@ -1083,10 +1110,7 @@ extern "C" int nbx_bp_mg_setup(nbx_bp* bp, int nlevels, const int* orders, int d
     if ((rc = bp_update_jacobi(b, b->lambda))) break;
     const bool last = l + 1 == nlevels;
     if (!last && ((rc = mg_alloc(mg, &L.res, b->Nall, es)) || (rc = mg_alloc(mg, &L.Ad, b->Nall, es)))) break;
-    // a cycle's directions before the last: 2 degree, or kMgHeld and the one being formed
-    for (int q = 0; !last && q < std::min(2 * degree, kMgHeld + 1) && rc == NBX_SUCCESS; ++q)
-      rc = mg_alloc(mg, &L.d[q], b->Nall, es);
-    if (rc) break;
+    if (!last && (rc = mg_directions(mg, L, es))) break;
     if (l > 0 && ((rc = mg_alloc(mg, &L.r, b->Nall, last ? sizeof(double) : es)) ||
                   (rc = mg_alloc(mg, &L.x, b->Nall, last ? sizeof(double) : es))))
       break;
