@@ -457,7 +457,12 @@ __global__ __launch_bounds__((NQ * NQ * AxShape<T, NQ, BK>::epb)) void k_axhelm(
 }
 
 // Three fields in turn, the element's factors read once (GeoKept); the next
-// field's q is loaded while the factors are applied to the current one.
+// field's q is loaded while the factors are applied to the current one.  Up to
+// NQ = 6 the load is left out after the last field (12e6 nodes, with it / now:
+// N = 2 FP64 Poisson 250 / 241 us, N = 5 FP64 Helmholtz 282 / 274, FP32 Poisson
+// 108 / 104); above, the branch costs more than the load, whose lines the
+// caches hold (1e6 nodes, FP64 Poisson: N = 8 31.9 us without the branch, 35.4
+// with it, N = 9 22.8 / 24.5, N = 7 18.1 / 18.4).
 template <typename T, int NQ, bool BK, bool PARTIAL, typename G>
 __global__ __launch_bounds__((NQ * NQ * AxKept<T, NQ, BK>::epb), (AxKept<T, NQ, BK>::waves)) void k_axhelm_kept(
     const int32_t Nelements, const int32_t offset, const int32_t* __restrict__ elementList,
@@ -489,8 +494,10 @@ __global__ __launch_bounds__((NQ * NQ * AxKept<T, NQ, BK>::epb), (AxKept<T, NQ, 
     axhelm_lines<T, NQ, BK>(
         t, rq, out, (ConstPtr<T>)D, s_r[slot], s_s[slot], geo,
         [&]() {
+          if (NQ > 6 || f + 1 < NF) {  // (at the end of NQ > 6 the last field's again, unused)
 #pragma unroll
-          for (int k = 0; k < NQ; ++k) rq[k] = qf[lo + k * NQ2];
+            for (int k = 0; k < NQ; ++k) rq[k] = qf[lo + k * NQ2];
+          }
         },
         [&](T(&mq)[NQ]) {
           if (!BK) {
@@ -594,7 +601,10 @@ struct AxPcg {
   static constexpr bool kept = NF == 3 && FORM == kInTurn && AxKept<T, NQ, BK>::value;
   static constexpr int epb = FORM != kInTurn ? 1 : kept ? AxKept<T, NQ, BK>::epb : AxShape<T, NQ, BK>::epb;
   static constexpr int waves = kept ? AxKept<T, NQ, BK>::waves : 1;
-  // the next field's z and p in flight during the current one, where the registers allow it
+  // the next field's z and p in flight during the current one, where the
+  // registers allow it (after the last field nothing is loaded: 13824 elements,
+  // 12 iterations FP64, with / without that load, N = 7 6.49 / 6.36 ms, N = 5
+  // 3.04 / 2.99)
   static constexpr bool prefetch = kept && (sizeof(T) == 4 || NQ <= 8);
   static constexpr bool late = NF == 3 && FORM == kInTurn && !prefetch;
 };
@@ -662,7 +672,7 @@ __global__ __launch_bounds__((NQ * NQ * AxPcg<NQ, NF, BK, T, G, FORM>::epb * (FO
       axhelm_lines<T, NQ, BK, P::late>(
           t, rq, out, (ConstPtr<T>)D, s_r[y], s_s[y], geo,
           [&]() {
-            if (P::prefetch) load_zp();  // the next field's (at the end the last field's again, unused)
+            if (P::prefetch && f + 1 < LOOP) load_zp();  // the next field's
           },
           [&](T(&mq)[NQ]) {
 #pragma unroll
