@@ -344,42 +344,72 @@ struct AxShape {
 };
 // Three fields: the element's factors kept in registers for all of them
 // (k_axhelm_kept) against one workgroup per field (k_axhelm), whose second
-// and third read of the factors come from L2 at about 9 TB/s at most.  12e6
-// nodes, kept against per field: FP64 N = 7 207 / 242 us (BK) and 266 / 315
-// (non-BK), N = 9 BK 287 / 300, FP32 N = 7 113 / 123 and N = 5 124 / 155; the
-// FP64 non-BK form at N = 9 would spill and is per field (377 / 442).  Three
-// times the workgroups are better while the chip is not full: 1e6 nodes, FP32
-// N = 7 14.3 / 11.2 us and FP64 N = 8 non-BK 45.8 / 40.4; FP64 gains from the
-// kept factors up to N = 7 at every size (21.8 / 25.2).
+// and third read of the factors come from L2 at about 9 TB/s at most.  Three
+// times the workgroups are better while the chip is not full.  us, kept / per
+// field:
+//                       3e5 nodes     1e6           3e6           12e6
+//   FP64 Poisson  N = 1 7.2 / 7.1     24.8 / 21.0   69.2 / 60.2   264 / 283
+//                 N = 3 8.0 / 6.6     16.9 / 18.6   46.7 / 48.0   165 / 219
+//                 N = 5 10.1 / 8.0    22.5 / 22.1   55.6 / 58.6   183 / 259
+//                 N = 7 9.9 / 7.6     19.1 / 20.5   56.1 / 51.3   178 / 219
+//                 N = 9 16.3 / 9.9    24.8 / 25.1   65.9 / 64.3   216 / 271
+//        Helmholtz N = 5 11.3 / 9.6   32.1 / 26.2   76.6 / 72.8   275 / 337
+//                 N = 7 11.3 / 9.1    23.1 / 24.5   63.9 / 65.0   231 / 298
+//                 N = 8 16.3 / 12.5   38.7 / 33.1   89.5 / 91.7   318 / 419
+//   FP32 Poisson  N = 2 6.8 / 7.2     16.3 / 19.1   45.2 / 51.1   166 / 211
+//                 N = 7 7.9 / 5.0     11.7 / 9.4    30.2 / 26.0   93 / 101
+//        Helmholtz N = 4 8.1 / 6.2    17.1 / 16.1   46.4 / 43.8   162 / 203
+// The lines are in waves of elements' lanes (Nq^2 an element, eight waves a
+// SIMD are 8192).  The FP64 non-BK form at N = 9 would spill and is per field,
+// the FP32 form at N = 1 is slower throughout (198 / 156 at 12e6).
 template <typename T, int NQ, bool BK>
 struct AxKept {
   static constexpr bool f64 = sizeof(T) == 8;
-  static constexpr bool value = f64 ? NQ <= 9 || (NQ == 10 && BK) : NQ <= 8;
+  static constexpr bool value = f64 ? NQ <= 9 || (NQ == 10 && BK) : NQ <= 8;  // (the PCG form too)
   static constexpr int epb = NQ == 2 ? 32 : NQ == 3 ? 14 : NQ == 4 ? 8 : NQ == 5 ? 5 : NQ == 6 ? 3 : 1;
   static constexpr int waves = f64 && NQ >= 7 ? 2 : 1;
-  static bool when(int64_t Nelements)
-  {
-    const bool full = Nelements * (NQ * NQ) >= 64 * 8192;  // eight waves per SIMD
-    return f64 ? NQ <= 8 || BK || full : NQ >= 3 && full;
-  }
+  static constexpr int64_t from =
+      f64 ? (NQ == 2 ? 32768 : NQ == 3 ? 16384 : NQ == 5 || NQ == 6 ? 8192 : NQ == 9 ? 6144 : 1536)
+          : (NQ == 2 ? INT64_MAX / 64 : NQ == 3 ? 1024 : 8192);
+  static bool when(int64_t Nelements) { return Nelements * (NQ * NQ) >= 64 * from; }
 };
 
 // Three-field PCG form: one thread group per field of an element against the
 // fields in turn.  Groups are faster while the chip is not full, and where the
-// fields in turn leave one wave per SIMD (FP64 non-BK, us, groups / in turn:
-// N = 7 at 1e5 nodes 7.8 / 11.0, at 8e6 288 / 236; N = 11 at 8e6 399 / 752).
-// The line in lanes (Nq^2 per element) lies between the measured sizes on each
-// side.
+// fields in turn leave one wave per SIMD.  us, groups / in turn:
+//                            1e5 nodes     1e6           3e6           8e6
+//   FP64 Poisson   N = 5     6.7 / 9.8     30.0 / 33.2   82.6 / 81.4   236 / 198
+//                  N = 7     7.2 / 10.3    29.3 / 27.4   72.7 / 74.4   210 / 179
+//                  N = 8     8.8 / 13.0    32.0 / 44.2   80.1 / 102    240 / 245
+//                  N = 9     10.6 / 14.3   44.1 / 34.6   120 / 94.3    341 / 225
+//                  N = 10    12.2 / 16.6   42.5 / 43.5   114 / 118     330 / 299
+//                  N = 11    13.5 / 19.0   47.0 / 57.2   106 / 125     320 / 325
+//                  N = 13    21.5 / 26.9   50.9 / 67.5   125 / 167     345 / 414
+//        Helmholtz N = 7     7.2 / 10.5    32.2 / 31.3   97.5 / 84.6   262 / 204
+//                  N = 8     9.2 / 13.9    35.2 / 48.7   109 / 115     293 / 275
+//   FP32 Poisson   N = 7     5.9 / 8.7     22.7 / 22.4   58.1 / 58.7   157 / 143
+//                  N = 9     8.7 / 13.0    26.2 / 31.1   69.1 / 90.3   186 / 223
+//   bf16 geometry  N = 4     6.7 / 8.7     32.1 / 29.2   86.4 / 78.1   240 / 195  (Helmholtz)
+//                  N = 5     5.9 / 9.2     24.0 / 26.2   60.1 / 68.1   151 / 165  (Poisson)
+//                  N = 9     9.5 / 15.6    38.5 / 32.6   94.6 / 85.3   271 / 214  (Helmholtz)
+//                  N = 9     9.1 / 14.7    27.1 / 30.7   72.5 / 80.8   197 / 193  (Poisson)
+//                  N = 13    16.9 / 25.3   42.8 / 43.3   111 / 94.4    279 / 228  (Poisson)
+// Each line (in waves of Nq^2 lanes an element) lies between the measured sizes
+// on its two sides; kAll: groups at every size, the fields in turn are not built.
 template <typename T, int NQ, bool BK, typename G>
 struct AxFieldGroups {
   static constexpr bool fits = NQ >= 4 && 3 * (LineLayout<T, NQ>::SZ + LineLayout<T, NQ>::SS) * sizeof(T) < 150000;
-  static bool when(int64_t Nelements)
-  {
-    const int64_t lanes = Nelements * (NQ * NQ);
-    if (sizeof(T) == 8) return NQ == 9 || NQ >= 12 || lanes < 64 * (NQ == 11 ? 4096 : 1024);
-    if (sizeof(G) == 2 && (NQ == 10 || NQ == 11)) return lanes < 64 * 2048;
-    return NQ >= 9 || lanes < 64 * 16384;
-  }
+  static constexpr int64_t kAll = INT64_MAX / 64;
+  static constexpr int64_t below = sizeof(T) == 8   ? (NQ >= 12 ? kAll : NQ == 9 || NQ == 11 ? 8192 : NQ == 6 ? 4096 : 768)
+                                   : sizeof(G) == 4 ? (NQ >= 9 ? kAll : 12288)
+                                   : NQ == 5 || NQ == 7 || NQ == 8 ? 1024
+                                   : NQ == 10                      ? (BK ? 8192 : 1024)
+                                   : NQ == 11                      ? 2048
+                                   : NQ == 14 && BK                ? 2048
+                                   : NQ == 15                      ? 8192
+                                                                   : kAll;
+  static constexpr bool always = fits && below == kAll;
+  static bool when(int64_t Nelements) { return always || Nelements * (NQ * NQ) < 64 * below; }
 };
 
 // The elements of a workgroup: a uniform base and a lane offset, so that the
@@ -527,20 +557,21 @@ struct AxFieldSums {
 // take the place of one that holds three fields' lines in LDS or one field's
 // registers on one wave per SIMD, and G and lambda of the fields after the
 // first come from the XCD's L2.  us, the better other form / this one:
-//            3e5 nodes      1e6            8e6
-//   N = 9    24.6 / 17.4    52.2 / 40.0    395 / 333   FP64 (1e5: 12.6 / 12.4)
-//   N = 10   17.8 / 17.9    51.0 / 40.7    415 / 320   FP64 (1e5: 15.2 / 11.9)
-//   N = 11   20.1 / 22.4    58.0 / 46.7    400 / 363   FP64 (6e5: 38.6 / 33.9)
-//   N = 9    13.1 / 12.4    35.7 / 30.9    251 / 231   FP32 (1e5: 9.1 / 10.0)
-//   N = 10   12.2 / 13.0    37.6 / 30.9    297 / 231   FP32 (6e5: 24.5 / 19.0)
-//   N = 11   13.7 / 16.1    40.2 / 33.2    265 / 239   FP32 (6e5: 26.3 / 26.2)
-// N = 7 and 8 lose (FP64 at 8e6 237 / 289 and 314 / 377).  Below one element a
-// CU only FP64 N = 9 and 10 gain.
+//            1e5 nodes      3e5            1e6            8e6
+//   N = 9    11.3 / 11.0    22.3 / 16.3    46.5 / 38.3    365 / 307   FP64
+//   N = 10   13.7 / 10.5    16.3 / 16.2    46.8 / 39.3    380 / 295   FP64
+//   N = 11   14.7 / 11.5    17.7 / 20.1    50.6 / 42.5    355 / 314   FP64
+//   N = 9    8.8 / 9.5      12.4 / 11.9    34.8 / 30.1    230 / 220   FP32
+//   N = 10   10.5 / 9.5     11.7 / 12.2    36.0 / 29.9    266 / 218   FP32
+//   N = 11   11.1 / 10.3    12.3 / 14.9    37.9 / 31.3    246 / 207   FP32
+// N = 7 and 8 lose but for the smallest meshes, the small kernel not counted
+// (FP64 at 8e6 nodes 202 / 261 and 274 / 348).  Where three workgroups an element no longer have a
+// CU each, and up to one element a CU, only FP64 N = 9 and 10 gain.
 template <int NQ, int NF, bool BK, typename T, typename G>
 struct AxFieldBlocks {
   static constexpr bool value = AxFieldSums<NQ, NF, BK, G>::value && NQ >= 10;
   static constexpr bool always = value && sizeof(T) == 8 && NQ <= 11;
-  static bool when(int64_t Nelements) { return always || Nelements >= 256; }
+  static bool when(int64_t Nelements) { return always || Nelements >= 256 || 3 * Nelements <= 256; }
 };
 
 template <int NQ2>
@@ -915,7 +946,7 @@ static void axhelm_pcg_launch_k(int32_t Nelements, int32_t offset, const void* g
       return;
     }
   }
-  if constexpr (!AxFieldBlocks<NQ, NF, BK, T, G>::always) {
+  if constexpr (!AxFieldBlocks<NQ, NF, BK, T, G>::always && !(NF == 3 && AxFieldGroups<T, NQ, BK, G>::always)) {
     constexpr int EPB = AxPcg<NQ, NF, BK, T, G, kInTurn>::epb;
     hipLaunchKernelGGL((k_axhelm_pcg<NQ, NF, BK, T, G, kInTurn>), dim3((Nelements + EPB - 1) / EPB),
                        dim3(NQ * NQ, EPB), 0, s, Nelements, offset, (const G*)ggeo, (const T*)D, (const G*)lambda, z,
