@@ -236,14 +236,13 @@ __global__ __launch_bounds__(Mma16<NQ>::TH, 8) void k_axhelm_mma16(
   }
 }
 
-int axhelm_mma_launch(int N, int Nf, int bk, bool bf16_geometry, bool f16_operands, int32_t Nelements,
-                      int32_t offset, const void* ggeo, const void* D, const void* lambda, const void* q, void* Aq,
+int axhelm_mma_launch(int N, int Nf, int bk, bool f16_operands, int32_t Nelements, int32_t offset,
+                      const void* ggeo, const void* D, const void* lambda, const void* q, void* Aq,
                       const int* skip, hipStream_t s)
 {
   const char* name = f16_operands ? "axhelm fp16-MFMA" : "axhelm bf16-MFMA";
   if (!((N == 7 || N == 9) && (Nf == 1 || Nf == 3)))
     return fail(NBX_ERR_UNSUPPORTED, "%s: N = 7 or 9, one or three fields", name);
-  if (f16_operands && bf16_geometry) return fail(NBX_ERR_UNSUPPORTED, "%s: FP32 geometry only", name);
   if (Nelements <= 0) return Nelements == 0 ? NBX_SUCCESS : fail(NBX_ERR_INVALID, "axhelm: Nelements < 0");
   if (Nf == 3 && offset < Nelements * (N + 1) * (N + 1) * (N + 1))
     return fail(NBX_ERR_INVALID, "axhelm: offset < Nelements * Np");
@@ -255,8 +254,7 @@ int axhelm_mma_launch(int N, int Nf, int bk, bool bf16_geometry, bool f16_operan
   if (bk) NBX_MMA16(NQV, NFV, true, GT, OPT); else NBX_MMA16(NQV, NFV, false, GT, OPT);
 #define NBX_MMA16_T(NQV, NFV)                                   \
   if (f16_operands) { NBX_MMA16_BK(NQV, NFV, float, OpF16) }     \
-  else if (bf16_geometry) { NBX_MMA16_BK(NQV, NFV, uint16_t, OpBf16) } \
-  else { NBX_MMA16_BK(NQV, NFV, float, OpBf16) }
+  else { NBX_MMA16_BK(NQV, NFV, uint16_t, OpBf16) }
   if (N == 7 && Nf == 1) { NBX_MMA16_T(8, 1) }
   else if (N == 7) { NBX_MMA16_T(8, 3) }
   else if (Nf == 1) { NBX_MMA16_T(10, 1) }

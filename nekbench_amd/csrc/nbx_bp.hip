@@ -102,12 +102,11 @@ __device__ __forceinline__ void pcg_after_dots(PcgScalars* S, double rdotz, doub
 constexpr int kUpdateBatch = 8;
 
 // 1. [x += alpha p, r -= alpha Ap of the previous iteration]; z = M r
-//    (Jacobi: invDiag r; copy: z is r itself); tile partials of the dots
+//    (Jacobi: invDiag r; copy: z is r itself); tile partials of the dots; one field
 template <bool JAC, bool FLEX, bool DEG>
 __global__ __launch_bounds__(256) void k_pcg_update_precon_dots(
-    const int32_t N, const int32_t offset, const int Nf, const double* __restrict__ w, const uint8_t* __restrict__ deg,
-    const double* __restrict__ invDiag, const double* __restrict__ p, const double* __restrict__ Ap,
-    double* __restrict__ x, double* __restrict__ r, double* __restrict__ z, double* __restrict__ partials,
+    const int32_t N, const double* __restrict__ w, const uint8_t* __restrict__ deg, const double* __restrict__ invDiag,
+    const double* __restrict__ p, const double* __restrict__ Ap, double* __restrict__ x, double* __restrict__ r, double* __restrict__ z, double* __restrict__ partials,
     const PcgScalars* S)
 {
   if (S->done) return;
@@ -119,8 +118,8 @@ __global__ __launch_bounds__(256) void k_pcg_update_precon_dots(
 #pragma unroll
   for (int c = 0; c < NV; ++c) v[c] = 0.0;
   const int64_t b0 = (int64_t)blockIdx.x * kRedTile + threadIdx.x;
-  if (update && Nf == 1 && (int64_t)(blockIdx.x + 1) * kRedTile <= N) {
-    // a full tile of one field after the first iteration (every block but the
+  if (update && (int64_t)(blockIdx.x + 1) * kRedTile <= N) {
+    // a full tile after the first iteration (every block but the
     // last): each lane issues the loads of all its nodes before the first
     // store, instead of one node's loads per round trip to memory; the
     // arithmetic and the order of the sums are those of the general loop
@@ -165,25 +164,22 @@ __global__ __launch_bounds__(256) void k_pcg_update_precon_dots(
     const int64_t id = b0 + u * kRedLanes;
     if (id < N) {
       const double wid = weight<DEG>(w, deg, id);
-      for (int f = 0; f < Nf; ++f) {
-        const int64_t iid = id + (int64_t)f * offset;
-        double rf = ldnt(&r[iid]);
-        double apf = 0.0;
-        if (update || FLEX) apf = ldnt(&Ap[iid]);
-        if (update) {
-          stnt(__builtin_fma(alpha, ldnt(&p[iid]), ldnt(&x[iid])), &x[iid]);  // BPUpdatePCG, utils.okl:795-807
-          rf = __builtin_fma(-alpha, apf, rf);
-          stnt(rf, &r[iid]);
-        }
-        double zf = rf;
-        if (JAC) {
-          zf = ldnt(&invDiag[id]) * rf;
-          stnt(zf, &z[iid]);
-        }
-        v[0] = __builtin_fma(wid * rf, zf, v[0]);
-        v[1] = __builtin_fma(wid * rf, rf, v[1]);
-        if (FLEX) v[NV - 1] = __builtin_fma(wid * zf, apf, v[NV - 1]);
+      double rf = ldnt(&r[id]);
+      double apf = 0.0;
+      if (update || FLEX) apf = ldnt(&Ap[id]);
+      if (update) {
+        stnt(__builtin_fma(alpha, ldnt(&p[id]), ldnt(&x[id])), &x[id]);  // BPUpdatePCG, utils.okl:795-807
+        rf = __builtin_fma(-alpha, apf, rf);
+        stnt(rf, &r[id]);
       }
+      double zf = rf;
+      if (JAC) {
+        zf = ldnt(&invDiag[id]) * rf;
+        stnt(zf, &z[id]);
+      }
+      v[0] = __builtin_fma(wid * rf, zf, v[0]);
+      v[1] = __builtin_fma(wid * rf, rf, v[1]);
+      if (FLEX) v[NV - 1] = __builtin_fma(wid * zf, apf, v[NV - 1]);
     }
   }
   block_sum256<NV>(v, s4);
@@ -786,9 +782,8 @@ int bp_enqueue_iteration(nbx_bp* bp, const double* lambda, double* r, double* x)
     hipLaunchKernelGGL((k_pcg_update_precon_dots3<J, F, DG>), dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal,     \
                        bp->fieldOffset, w, deg, bp->invDiagA, bp->p, bp->Ap, x, r, bp->z, bp->red.partials, bp->S); \
   else                                                                                                           \
-    hipLaunchKernelGGL((k_pcg_update_precon_dots<J, F, DG>), dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal,        \
-                     bp->fieldOffset, bp->Nf, w, deg, bp->invDiagA, bp->p, bp->Ap, x, r, bp->z, bp->red.partials,  \
-                     bp->S)
+    hipLaunchKernelGGL((k_pcg_update_precon_dots<J, F, DG>), dim3(nb), dim3(256), 0, bp->stream, bp->Nlocal, w,     \
+                       deg, bp->invDiagA, bp->p, bp->Ap, x, r, bp->z, bp->red.partials, bp->S)
 #define NBX_PD2(J, F) \
   if (deg) NBX_PD(J, F, true); else NBX_PD(J, F, false);
   if (jac && flex) { NBX_PD2(true, true) }

@@ -8,7 +8,7 @@
 // kernel skips singletons, gatherScatterMany.okl:68), which for a hex box
 // removes ~40-60% of the work without changing any result.
 //
-// Kernel: one lane per shared group, all k fields per lane (ids read once).
+// Kernel: one lane per shared group and field (a row of the grid per field).
 // Add/mul start from 0/1 and combine members in ascending order, min/max
 // start from the first member (gatherScatterMany.okl:58-86, 148-176, 300-330,
 // 455-485), so every result is bit-identical to the reference kernel's.
@@ -238,7 +238,7 @@ static int64_t gs_classes(const nbx_ogs* o, int32_t Nmasked, const int32_t* mask
 // A row of the grid per field: a row's lines stay in the L2s as one field's do,
 // and small meshes fill the chip.  The fields in turn by the same lanes read
 // the members once, but their slices take several fields' lines of L2 and a
-// lane's chain grows: never faster in the sizes measured, us in turn / rows
+// lane's chain grows: slower but for one size by 1 %, us in turn / rows
 // (8e6 nodes, FP64): N = 7 two fields 72.6 / 65.5, three 112 / 95.5, four
 // 197 / 139; N = 3 four 288 / 178; N = 2 four 531 / 319; 2e6 nodes, N = 7 three
 // 23.6 / 23.9; 512 elements of N = 7, three fields, 22 / 5.7.

@@ -63,3 +63,16 @@ def test_operator_rows_of_D_do_not_spill(built):
             assert k[".sgpr_spill_count"] <= allowed, (name, k[".sgpr_spill_count"])
             assert k[".vgpr_spill_count"] == 0, (name, k[".vgpr_spill_count"])
     assert seen == 15 * 2 * (2 + 2 + 1)  # orders, forms; whole and list in FP64 and FP32, whole with bf16 geometry
+
+
+def test_forms_that_no_call_reaches_are_not_built(built):
+    """FP32 geometry with bf16 operands has no precision of its own, and the
+    three-field PCG form takes a thread group per field at every mesh size for
+    these orders."""
+    mma = [n for n in built if "14k_axhelm_mma16I" in n]
+    assert mma and not [n for n in mma if "EfNS_6OpBf16E" in n]
+    turn = {m.groups() for m in (re.match(r"_ZN3nbx12k_axhelm_pcgILi(\d+)ELi3ELb([01])E([df])(\w)Li0E", n) for n in built)
+            if m}
+    assert ("8", "1", "d", "d") in turn and ("15", "1", "d", "d") in turn
+    assert not [t for t in turn if t[2] == "d" and t[0] in ("12", "13", "14")]
+    assert not [t for t in turn if t[3] == "f" and int(t[0]) >= 9]
