@@ -33,10 +33,19 @@ sys.path.insert(0, str(ROOT))
 METRIC = "PCG time-to-1e-8 residual, learned/mixed vs FP64 Jacobi; axhelm GDOF/s"
 HBM_PEAK_GBS = 8000.0
 ROOF_SETS = 4  # rotating buffer sets of the roofline measurement
+ROOF_KERNEL = "k_axhelm<double, 8, 1, true, false, double>"  # the FP64 BK operator at N = 7, one field
 
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
+
+
+def counter_traffic(entry, kernel, path=ROOT / "profiles" / "traffic.json"):
+    """HBM bytes per launch of the recorded counter runs, or None where they are of another kernel."""
+    if not path.exists():
+        return None
+    rec = json.loads(path.read_text()).get(entry, {})
+    return rec.get("traffic_bytes_per_launch") if rec.get("kernel") == kernel else None
 
 
 def run_cpu_baseline(pcg_nx, axhelm_nx, log):
@@ -910,10 +919,7 @@ def main():
         compare = solver_comparison(nbx, bp, b, r, x, log, bp_mg=bp_mg, mg_cfg=mg_cfg, net=net)
         bp_mg.free()
 
-    traffic = None
-    tfile = ROOT / "profiles" / "traffic.json"
-    if tfile.exists() and NX == 32:
-        traffic = json.loads(tfile.read_text()).get("axhelm_bk_f64_n7_32cube", {}).get("traffic_bytes_per_launch")
+    traffic = counter_traffic("axhelm_bk_f64_n7_32cube", ROOF_KERNEL) if NX == 32 else None
     cpu = None if args.no_cpu else run_cpu_baseline(NX, 0 if args.no_compare else 16, log)
     if mesh16 is not None and cpu and "axhelm" in cpu:
         mesh16["cpu_reference_axhelm"] = dict(cpu["axhelm"], cores=cpu["cores"]["threads"], cpu=cpu["cores"]["cpu"])
@@ -944,7 +950,7 @@ def main():
                    "time_to_1e-8": compare, "mesh16": mesh16},
         "roofline": {"bound": "hbm", "achieved": round(ax_gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(ax_gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_axhelm", "bytes_per_launch": ax_bytes,
+                     "kernel": ROOF_KERNEL, "bytes_per_launch": ax_bytes,
                      "us_per_launch": round(ax_s * 1e6, 3), "buffer_sets": ROOF_SETS,
                      "timing": "per-launch HIP events, 2 ms idle before each launch",
                      "us_per_launch_back_to_back": round(ax_b2b_s * 1e6, 3),
