@@ -269,7 +269,7 @@ __device__ __forceinline__ void relu(NodeChannels& h)
 // channel, over the 128 nodes of the planes k0 and k0 + 1, where some dL/dpre1
 // is not finite: a tap whose neighbour lies outside of the element takes no
 // part, while the products would multiply its padding, and 0 inf is not 0.
-__device__ __noinline__ void taps_in_range(const TrainLds& lds, const int row, const int channel, const int k0,
+__device__ __forceinline__ void taps_in_range(const TrainLds& lds, const int row, const int channel, const int k0,
                                            f32x4& acc)
 {
 #pragma unroll 1
@@ -470,8 +470,9 @@ __global__ __launch_bounds__(512, 4) void k_net_train(const int2* __restrict__ s
                 [&](int t, int tt) { return d2.v[tt][t >> 2][t & 3]; }, d1);
   each_channel([&](int tt, int m, int u) { d1.v[tt][m][u] = h1.v[tt][m][u] > 0.f ? d1.v[tt][m][u] : 0.f; });
   {
-    float zero = 0.f;  // not zero where a value is not finite
-    each_channel([&](int tt, int m, int u) { zero = __builtin_fmaf(d1.v[tt][m][u], 0.f, zero); });
+    float z[4] = {};  // not zero where a value is not finite
+    each_channel([&](int tt, int m, int u) { z[tt] = __builtin_fmaf(d1.v[tt][m][u], 0.f, z[tt]); });
+    const float zero = (z[0] + z[1]) + (z[2] + z[3]);
     if (!(zero == 0.f)) lds.nonfinite = 1;
   }
   // phase 2: waves 0..5 the 35 rows of Wr, Wg, b1 (three row tiles), waves 6, 7 b2
