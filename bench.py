@@ -848,10 +848,10 @@ def main():
     # buffer sets (4 x 1.2 GB, far beyond the 256 MB Infinity Cache, so no
     # launch finds its inputs in cache), HIP events on the launch stream.
     # Each launch is timed by its own event pair with 2 ms of idle time before
-    # it: back to back, after about a dozen launches (2-3 ms) this FP64 kernel
-    # slows from ~178 to 200-240 us while a triad of the same bytes does not,
-    # i.e. the board's power management lowers the clocks; the back-to-back
-    # average is reported beside it.
+    # it: earlier forms of this kernel slowed from ~178 to 200-240 us after a
+    # dozen launches back to back, as the board lowered its clocks.  This form
+    # does not (176-183 us over 40 launches); the back-to-back average is
+    # reported beside it.
     ggeo = bp.device_array("ggeo", E * 7 * bp.Np)
     D = bp.device_array("D", (N + 1) ** 2)
     Ap = torch.empty_like(x)

@@ -195,7 +195,7 @@ __global__ __launch_bounds__(512) void k_net_apply(const int32_t E, const float*
 // 2048 samples: 3836 us for the form that held one parameter a lane (two LDS
 // reads an fma) and gave a workgroup a whole chunk of samples (half the chip
 // idle at 16 a chunk); 290 with the forward pass and the data gradients on the
-// vector ALUs, lane = node, weights as scalar operands; 252 now.
+// vector ALUs, lane = node, weights as scalar operands; 248 now.
 struct TrainLds {
   float rh[kPadN], dy[kPadN];      // zero-padded tiles
   float g[kG * kFRow];             // factors, node (x, y, z) at 100 z + 10 y + x
